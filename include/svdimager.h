@@ -256,12 +256,13 @@ int svdi_image_snapshots_planned(svdi_context* ctx, const svdi_snapshot* snapsho
 
 /* Work shape of the MFMA window gridder (no counterpart in the reference, whose gridder has no
  * shape to tune; the batching form picks it per image size with svdi_autotune).  The gridder
- * contracts 16 x 16 windows of the grid; a window's records are contracted by one wavefront
- * when there are at most coop_min of them, else in pieces of at most coop_cap records each
- * taken by a whole workgroup.  Records are binned by row classes of 2^class_log2 rows.  Zero
- * fields select the library's defaults (coop_min 1024, coop_cap 24576, class_log2 2 when its
- * histogram fits in LDS, else 3).  The shape changes how the FP32 sums are ordered, not what
- * is summed: images agree to rounding. */
+ * contracts 16 x 16 windows of the grid; half a window's records (those whose footprints start
+ * in it) are contracted by one wavefront when there are at most coop_min of them, else in pieces
+ * of at most coop_cap records each taken by a whole workgroup.  Records are binned by row classes
+ * of 2^class_log2 rows.  Zero fields select the library's defaults (coop_min 256 .. 1024 and
+ * coop_cap 2048 .. 16384 by the number of samples, class_log2 2 when its histogram fits in LDS,
+ * else 3).  The shape changes how the FP32 sums are ordered, not what is summed: images agree to
+ * rounding. */
 typedef struct svdi_tuning {
     uint32_t coop_min;          /* 0, or 32 .. 65536 */
     uint32_t coop_cap;          /* 0, or 4096 .. 16777216 */
@@ -278,7 +279,7 @@ int svdi_set_tuning(svdi_context* ctx, size_t grid_size, const svdi_tuning* tuni
 int svdi_get_tuning(svdi_context* ctx, size_t grid_size, svdi_tuning* tuning);
 
 /* Autotuner (no counterpart in the reference): images `snapshot` at image_size / cell_size with
- * the MFMA gridder under each candidate shape (coop_min 256 .. 2048, coop_cap 12288 .. 49152, both
+ * the MFMA gridder under each candidate shape (coop_min 256 .. 2048, coop_cap 4096 .. 16384, both
  * class heights), `repeats` times each (>= 1), times the grid stage with HIP events, and keeps the
  * fastest for this grid size on the context (svdi_set_tuning); *best receives it with its time
  * and the defaults' time.  K, the slabs and ES support stay the reference's: the search changes

@@ -1509,7 +1509,7 @@ int svdi_autotune(svdi_context* ctx, const svdi_snapshot* snap, size_t image_siz
             svdi_tuning pick = defaults;
             pick.grid_ms = default_ms;
             for (uint32_t cmin : {256u, 512u, 1024u, 2048u})
-                for (uint32_t ccap : {12288u, 24576u, 49152u})
+                for (uint32_t ccap : {4096u, 8192u, 16384u})
                     for (int cls : {2, 3}) {
                         svdi_tuning t = {};
                         t.coop_min = cmin;

@@ -143,6 +143,8 @@ class Workspace {
     size_t bytes_held() const;
     void begin_arena(void* base, size_t capacity);
     void end_arena();
+    // Bytes of the arena not carved yet (SIZE_MAX outside arena mode).
+    size_t arena_left() const { return arena_ != nullptr ? arena_cap_ - arena_used_ : SIZE_MAX; }
     // Frozen: a slot that would have to grow throws ArgError instead of allocating.
     void set_frozen(bool on) { frozen_ = on; }
     ~Workspace() { release(); }
@@ -272,9 +274,7 @@ struct WindowJob {
     float2* planes = nullptr;
     float2* partial = nullptr;
     float2* trash = nullptr;
-    const uint32_t* boff = nullptr;
-    const uint32_t* ioff = nullptr;
-    const uint32_t* multi = nullptr;
+    const void* reduce = nullptr;          // the windows that reduce_windows completes
     uint32_t max_slots = 0;
     int K = 0, G = 0, prec = 0;
     int geom[16] = {};                     // the window geometry (windows.hip)

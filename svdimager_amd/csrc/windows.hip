@@ -8,9 +8,9 @@
 // with (a, b) the window's cells and p_r the sample's position relative to the window.  For each
 // window row a, D_a = C * B_a runs on v_mfma_f32_16x16x32_f16, with C = c (16 x 32 samples) and
 // B_a[r][b] = ku_r[a] kv_r[b] (32 samples x 16 columns), the 16 row blocks (64 FP32 accumulators
-// per lane) staying in registers across the window's samples.  A window is written once: by the
-// wavefront or workgroup that contracted it, or, when it was split over several workgroup
-// pieces, as partial windows that k_win_reduce adds in piece order; no atomics touch the planes.
+// per lane) staying in registers across the window's samples.  Half windows that hold many samples
+// are contracted by workgroups instead, sorted by footprint column (k_win_dense); their partial
+// sums are added in piece order by k_win_reduce, and no atomics touch the planes.
 // Precision: c and the ES factors are split into f16 hi + lo and each product taken as
 // hi*hi + lo*hi + hi*lo with FP32 accumulation (~22 significant bits per product); c is scaled by
 // a power of two fixed from the largest |v| of the call and the ES factors by 2^7 each, so
@@ -36,6 +36,7 @@
 #include "records.hpp"
 
 #include <cstring>
+#include <type_traits>
 
 namespace svdi {
 namespace {
@@ -51,6 +52,7 @@ constexpr int kBinChanGroups = kBinThreads / kBinRowsPerSet;
 constexpr int kBinPerThread = 16;        // samples per thread, preprocessed input
 constexpr int kLdsBins = 36864;          // largest block-local histogram (144 KB of LDS)
 constexpr size_t kMaxBlockHistBytes = size_t(1) << 31;   // per-block histograms of all bands
+constexpr size_t kMaxPartialBytes = size_t(1) << 29;     // partial slots of the dense halves
 constexpr int kChunk = 32;               // samples per MFMA reduction step
 constexpr int kStride = 36;              // floats per c staging row (32 samples + pad)
 constexpr int kStrideH = 40;             // halves per ES staging row (32 samples + pad, 16-byte rows)
@@ -85,10 +87,6 @@ struct WinTraits {
     // kernel keeps its ~150 registers without spills; 16 (four per SIMD) would need 128 and a
     // staging area without row padding, which measured slower (542 against 500 us for split3).
     static constexpr int kWaves = (kEsLo || kBf16) ? 12 : 16;
-    // Accumulator slots of the workgroup reduction (within the staging area).
-    static constexpr int kSlots = (kEsLo || kBf16) ? 6 : 4;
-    static_assert(kWaves % kSlots == 0, "reduction rounds");
-    static_assert(kSlots * kWin * 64 * 4 <= kStageFloats * kWaves, "reduction slots exceed the staging area");
 };
 // ES(1) 2^7, the ninth footprint cell of an integer position, as f16 hi + lo.
 constexpr _Float16 kEsPolyEdgeHi = static_cast<_Float16>(kEsPolyEdge);
@@ -116,14 +114,20 @@ struct WinGeom {
     uint32_t coop_cap;   // records per workgroup piece
 };
 
-// A work item: records [start, start + count) of window `win`; bnd[j] (j = 1 .. ncls - 1) is the
-// first record of the window's class j (d = j - 8 / c), records before bnd[1] are of class 0,
-// and bnd[j] for j >= ncls is the window's end.
-// slot >= 0: the item is one piece of a window split over several workgroup items and writes its
-// partial window to partial slot `slot`; slot < 0: it writes the window to the planes.
+// A work item of window `win`.  slot < 0: a wavefront item, the `count` records from `start` on
+// that are not among [hole, hole + hole_len); bnd[j] (j = 1 .. ncls - 1) is the first record of the
+// window's class j (d = j - 8 / c), records before bnd[1] are of class 0, and bnd[j] for j >= ncls
+// is the window's end; skip (bits 0, 1, 2: the half above, the lower half, the upper half): records
+// with a negative first column are skipped.  slot >= 0: the piece [start, start + count) of half
+// `half`, whose share goes to partial slot `slot`; skip (0 or 1) as above.
 struct WItem {
     int win, start, count, slot;
     int bnd[kMaxClasses];
+    int hole, hole_len, half, skip;
+    __device__ __forceinline__ int record(int j) const {      // absolute index of the item's record j
+        const int i = start + j;
+        return i + (i >= hole ? hole_len : 0);
+    }
 };
 
 // Records: 16 bytes each (records.hpp), one aligned 16-byte access to write or read.
@@ -419,7 +423,13 @@ k_win_scatter(SampleInput in, GridParams gp, WinGeom wg, const uint32_t* __restr
         const int home = ((h << wg.cls_log2) + 8) >> 4;
         const int base1 = kSnap ? f.a0 - home * kWin : off - home * kWin;
         const int base2 = kSnap ? f.b0 - wb * kWin : off - wb * kWin;
-        rec.put(slot, rec_encode(base1, f.q1, base2, f.q2, f.s, f.vw.x, f.vw.y));
+        RecordWords w = rec_encode(base1, f.q1, base2, f.q2, f.s, f.vw.x, f.vw.y);
+        // A negative first column marks the copy of a record whose home is the window to the left.  A
+        // position just above an integer that the encoding rounds to it (first cell one lower, F = 0)
+        // keeps its home's first cell 0, with the largest fraction instead.
+        if (wb > 0 && f.b0 >= wb * kWin && static_cast<int32_t>(w.w[3]) < 0)
+            w.w[3] = (((1u << kRecFracBits) - 1u) << 8) | (w.w[3] & 0xffu);
+        rec.put(slot, w);
     };
     const size_t blk = blockIdx.x;
     if (!wg.use_lds) {
@@ -468,25 +478,27 @@ __device__ __forceinline__ WinRange window_range(const uint32_t* __restrict__ bo
     return x;
 }
 
-// Work items.  A window with at most coop_min records is one wavefront item.  A larger one is
-// taken by whole workgroups: pieces of at most coop_cap records whose chunks the workgroup's
-// wavefronts share, their accumulators summed in LDS.  A window with several pieces writes one
-// partial window per piece, and k_win_reduce adds them in piece order (so the result does not
-// depend on timing).  Both queues run largest first, by octave classes: class c holds items
-// with count * 2^c <= cap < count * 2^(c+1) (cap = coop_min for wavefront items, coop_cap for
-// workgroup items; the last class also the smaller and empty ones), so that the wavefronts and
-// workgroups finish together.  The default limits were measured (SKA-Low snapshot at 1024^2,
-// whose 9216 windows hold 1 to 1.8 M records each): below ~1000 records a workgroup item spends
-// a large part of its time summing the wavefronts' accumulators, and pieces much above ~25000
-// records leave the last ones running alone at the end of the launch; a context's tuning
-// (svdi_autotune) may replace them per grid size.
-// icount: [kItemClasses][nwin_total] wavefront items, [kItemClasses][nwin_total] workgroup items,
-// [nwin_total] partial slots; one exclusive scan gives the queue positions and slot numbers.
-// totals[0] = records, [1] = wavefront items, [2] = (unused), [3] = workgroup items,
-// [4] = max |v| bits, [5] = workgroup queue head, [6] = windows with several pieces.
+// Work items.  A window's home records are those of the 16 / c classes whose first footprint row
+// lies in the window; its halves are the two runs of classes of first rows 0 .. 7 and 8 .. 15.  A
+// half with more than coop_min home records is dense: k_win_dense takes them, in pieces of at
+// most coop_cap records, a workgroup each, and writes each piece's share of the 16 rows and 24
+// columns that its footprints reach (the lower eight rows of the upper half and the last eight
+// columns lie in the windows below and to the right) to a partial slot.  Every other record is read
+// by the wavefront items of k_win_grid, one per window: the halves that are not dense and the
+// upper half of the window above unless that is.  Either way the copies of records whose home is
+// a dense half of the window to the left (negative first column) are skipped.  k_win_reduce then
+// adds the partial slots, in piece order, to the windows that dense pieces reach (a window with
+// no other records gets no wavefront item).  Both queues run largest first, by octave classes: class c
+// holds items with count * 2^c <= cap < count * 2^(c+1) (cap = 3 coop_min for wavefront items,
+// coop_cap for pieces; the last class also the smaller and empty ones), so that the wavefronts
+// and workgroups finish together.
+// icount: [kItemClasses][nwin_total] wavefront items, [kItemClasses][2 nwin_total] pieces of the
+// halves, [2 nwin_total] partial slots; one exclusive scan gives the queue positions and slot
+// numbers.  totals[0] = records, [1] = wavefront items, [2] = (unused), [3] = pieces,
+// [4] = max |v| bits, [5] = piece queue head, [6] = windows that k_win_reduce completes.
 constexpr int kItemClasses = 8;
 constexpr uint32_t kCoopMinDefault = 1024;
-constexpr uint32_t kCoopCapDefault = 24576;
+constexpr uint32_t kCoopCapDefault = 16384;
 
 __device__ __forceinline__ int item_class(uint32_t count, uint32_t cap) {
     if (count == 0) return kItemClasses - 1;
@@ -495,8 +507,60 @@ __device__ __forceinline__ int item_class(uint32_t count, uint32_t cap) {
     return c;
 }
 
-__device__ __forceinline__ uint32_t coop_pieces(const WinGeom& wg, uint32_t c) {
-    return (c + wg.coop_cap - 1) / wg.coop_cap;
+// A dense window's pieces: equal runs of `per` records (a multiple of 32), the last one shorter.
+struct Pieces {
+    uint32_t count, per;
+};
+__device__ __forceinline__ Pieces dense_pieces(const WinGeom& wg, uint32_t records) {
+    const uint32_t n = (records + wg.coop_cap - 1) / wg.coop_cap;
+    const uint32_t per = ((records + n - 1) / n + 31u) & ~31u;
+    return {(records + per - 1) / per, per};
+}
+
+// Home records of half `half` of window (wa, wb) of slab ls (0 outside the grid of windows).
+__device__ __forceinline__ uint32_t half_records(const uint32_t* __restrict__ boff, const WinGeom& wg, int ls, int wa, int wb,
+                                                 int half) {
+    if (wa < 0 || wb < 0) return 0u;
+    const int per = 8 >> wg.cls_log2;                      // classes per half
+    const int base = (ls * wg.nw + wb) * wg.nh, h = (2 * wa + half) * per;
+    return boff[base + min(h + per, wg.nh)] - boff[base + min(h, wg.nh)];
+}
+
+// How window w's records are shared out: [h[0], h[1]) and [h[1], h[2]) the home records of its two
+// halves; [s0, s1) less [hole, hole + hole_len) the records of its wavefront item, s_count of them.
+// up, left[2], up_left: the records of the dense halves that reach it from the windows above and
+// to the left (0 where a half is not dense).
+struct WinSplit {
+    uint32_t h[3], s0, s1, hole, hole_len, s_count;
+    uint32_t up, left[2], up_left;
+    bool dense[2];
+    __device__ bool reduced() const { return dense[0] || dense[1] || (up | left[0] | left[1] | up_left) != 0; }
+    // Bit 0, 1, 2: skip the copies in the half above, the lower half and the upper half.
+    __device__ int skip() const { return (up_left != 0 ? 1 : 0) | (left[0] != 0 ? 2 : 0) | (left[1] != 0 ? 4 : 0); }
+};
+__device__ __forceinline__ WinSplit window_split(const uint32_t* __restrict__ boff, const WinGeom& wg, int w,
+                                                 const WinRange& x, uint32_t end) {
+    const int ls = w / wg.nwin, r = w - ls * wg.nwin;
+    const int wa = r / wg.nw, wb = r - wa * wg.nw;
+    auto if_dense = [&](uint32_t n) { return n > wg.coop_min ? n : 0u; };
+    WinSplit s;
+    s.h[0] = wg.cls_log2 == 2 ? x.bnd[2] : x.bnd[1];
+    s.h[1] = wg.cls_log2 == 2 ? x.bnd[4] : x.bnd[2];
+    s.h[2] = end;
+    s.dense[0] = s.h[1] - s.h[0] > wg.coop_min;
+    s.dense[1] = s.h[2] - s.h[1] > wg.coop_min;
+    // (The classes below the home ones are the upper half of the window above; none at the top.)
+    s.up = if_dense(s.h[0] - x.start());
+    s.left[0] = if_dense(half_records(boff, wg, ls, wa, wb - 1, 0));
+    s.left[1] = if_dense(half_records(boff, wg, ls, wa, wb - 1, 1));
+    s.up_left = if_dense(half_records(boff, wg, ls, wa - 1, wb - 1, 1));
+    s.s0 = s.up != 0 ? (s.dense[0] ? s.h[1] : s.h[0]) : x.start();
+    s.s1 = s.dense[1] ? (s.dense[0] ? s.h[0] : s.h[1]) : s.h[2];
+    if (s.s1 < s.s0) s.s1 = s.s0;                          // both halves and the one above are dense
+    s.hole = s.h[0];
+    s.hole_len = s.dense[0] && s.s0 <= s.h[0] && s.s1 >= s.h[1] ? s.h[1] - s.h[0] : 0u;
+    s.s_count = s.s1 - s.s0 - s.hole_len;
+    return s;
 }
 
 __global__ void __launch_bounds__(256)
@@ -508,32 +572,59 @@ k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __res
     if (w >= nwt) return;
     uint32_t end;
     const WinRange x = window_range(boff, wg, w, end);
-    const uint32_t c = end - x.start();
-    for (int k = 0; k <= 2 * kItemClasses; ++k) icount[k * nwt + w] = 0u;
-    if (c <= wg.coop_min) {
-        icount[item_class(c, wg.coop_min) * nwt + w] = 1u;
-        return;
+    const WinSplit s = window_split(boff, wg, w, x, end);
+    const int wcls = s.s_count > 0 || !s.reduced() ? item_class(s.s_count, 3 * wg.coop_min) : -1;
+    for (int k = 0; k < kItemClasses; ++k) icount[k * nwt + w] = k == wcls ? 1u : 0u;
+    uint32_t* half = icount + kItemClasses * nwt;
+    for (int j = 0; j < 2; ++j) {
+        int pcls = -1;
+        Pieces p = {0u, 0u};
+        if (s.dense[j]) {
+            p = dense_pieces(wg, s.h[j + 1] - s.h[j]);
+            pcls = item_class(p.per, wg.coop_cap);
+        }
+        for (int k = 0; k <= kItemClasses; ++k)
+            half[(2 * k + j) * nwt + w] = k == pcls || k == kItemClasses ? p.count : 0u;
     }
-    const uint32_t full = c / wg.coop_cap, rem = c - full * wg.coop_cap;
-    uint32_t* gcount = icount + kItemClasses * nwt;
-    gcount[w] += full;
-    if (rem > 0) gcount[item_class(rem, wg.coop_cap) * nwt + w] += 1u;
-    const uint32_t pieces = coop_pieces(wg, c);
-    if (pieces > 1) {
-        icount[2 * kItemClasses * nwt + w] = pieces;
-        multi[atomicAdd(&totals[6], 1u)] = static_cast<uint32_t>(w);
-    }
+    if (s.reduced()) multi[atomicAdd(&totals[6], 1u)] = static_cast<uint32_t>(w);
 }
 
+// A window that k_win_reduce completes: the partial slots of the halves that reach it (its lower
+// and upper half, the upper half of the window above, the two halves of the window to the left, the
+// upper half of the window above that), and whether the planes hold its wavefront item's sums.
+struct WReduce {
+    int win, add;
+    uint32_t first[6], count[6];
+};
+
 // One thread per item: its (queue, class, window) entry of the counts is found by binary search
-// over the offsets.  Workgroup piece q of class 0 below the window's full count is full piece q;
-// any other is the remainder (piece `full`).
+// over the offsets; and one thread per window that k_win_reduce completes.
 __global__ void __launch_bounds__(256)
 k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__ ioff,
-                 WinGeom wg, WItem* __restrict__ items, uint32_t max_items, uint32_t* __restrict__ totals) {
+                 const uint32_t* __restrict__ multi, WinGeom wg, WItem* __restrict__ items, uint32_t max_items,
+                 WReduce* __restrict__ red, uint32_t* __restrict__ totals) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     const int nwt = wg.nwin_total;
-    const int n = 2 * kItemClasses * nwt;
+    const int n = 3 * kItemClasses * nwt;
+    if (i < totals[6]) {                        // (a window is listed at most once: i < nwt)
+        const int w = static_cast<int>(multi[i]);
+        uint32_t end;
+        const WinRange x = window_range(boff, wg, w, end);
+        const WinSplit s = window_split(boff, wg, w, x, end);
+        WReduce r;
+        r.win = w;
+        r.add = s.s_count > 0 ? 1 : 0;
+        // (n + j nwt + w: the slots of half j of window w.)
+        const uint32_t records[6] = {s.dense[0] ? s.h[1] - s.h[0] : 0u, s.dense[1] ? s.h[2] - s.h[1] : 0u,
+                                     s.up, s.left[0], s.left[1], s.up_left};
+        const int at[6] = {n + w, n + nwt + w, n + nwt + w - wg.nw, n + w - 1, n + nwt + w - 1, n + nwt + w - wg.nw - 1};
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            r.count[k] = records[k] != 0 ? dense_pieces(wg, records[k]).count : 0u;
+            r.first[k] = records[k] != 0 ? ioff[at[k]] - ioff[n] : 0u;
+        }
+        red[i] = r;
+    }
     const uint32_t nwave = ioff[kItemClasses * nwt];
     const uint32_t nitems = min(ioff[n], max_items);
     if (i == 0) {
@@ -547,95 +638,101 @@ k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__
         if (ioff[mid] <= i) lo = mid;
         else hi = mid;
     }
-    const bool coop = lo >= kItemClasses * nwt;
-    const int j = coop ? lo - kItemClasses * nwt : lo;
-    const int cls = j / nwt;
-    const int w = j - cls * nwt;
+    const int row = lo / nwt;                   // wavefront class, then kItemClasses + 2 class + half
+    const int w = lo - row * nwt;
     uint32_t end;
     const WinRange x = window_range(boff, wg, w, end);
-    const uint32_t c = end - x.start();
+    const WinSplit s = window_split(boff, wg, w, x, end);
     WItem t;
     t.win = w;
 #pragma unroll
     for (int j = 0; j < kMaxClasses; ++j) t.bnd[j] = static_cast<int>(x.bnd[j]);
-    t.start = static_cast<int>(x.start());
-    t.count = static_cast<int>(c);
+    t.start = static_cast<int>(s.s0);
+    t.count = static_cast<int>(s.s_count);
+    t.hole = static_cast<int>(s.hole);
+    t.hole_len = static_cast<int>(s.hole_len);
     t.slot = -1;
-    if (coop) {
-        const uint32_t full = c / wg.coop_cap;
+    t.half = 0;
+    t.skip = s.skip();
+    if (row >= kItemClasses) {
+        const int j = (row - kItemClasses) & 1;
+        const uint32_t first = j ? s.h[1] : s.h[0], records = (j ? s.h[2] : s.h[1]) - first;
+        const Pieces p = dense_pieces(wg, records);
         const uint32_t q = i - ioff[lo];
-        const uint32_t piece = (cls == 0 && q < full) ? q : full;
-        t.start = static_cast<int>(x.start() + piece * wg.coop_cap);
-        t.count = static_cast<int>(piece < full ? wg.coop_cap : c - full * wg.coop_cap);
-        if (coop_pieces(wg, c) > 1) t.slot = static_cast<int>(ioff[n + w] - ioff[n] + piece);
+        t.start = static_cast<int>(first + q * p.per);
+        t.count = static_cast<int>(min(p.per, records - q * p.per));
+        t.slot = static_cast<int>(ioff[n + j * nwt + w] - ioff[n] + q);
+        t.half = j;
+        t.skip = (s.skip() >> (j + 1)) & 1;
     }
     items[i] = t;
 }
 
-// Windows with several pieces: the sum of their partial windows, in piece order, into the
-// planes.  One unit = (listed window, term) per workgroup of kReduceGroups x 256 threads: group g
-// sums the pieces g, g + kReduceGroups, ... of every cell (the densest windows have over a
-// hundred pieces, which one thread per cell would request one after another), and the groups'
-// sums are added in group order, so the result does not depend on timing.
-constexpr int kReduceGroups = 4;
-__global__ void __launch_bounds__(kReduceGroups * 256)
-k_win_reduce(const uint32_t* __restrict__ boff, const uint32_t* __restrict__ ioff,
-             const uint32_t* __restrict__ multi, const uint32_t* __restrict__ totals, WinGeom wg,
+// Partial slots: [term][kDenseRows rows][kDenseCols columns] from the half's first row and the
+// window's first column: a first cell in the half's 8 x 16, and eight cells more at most.
+constexpr int kDenseRows = kWin / 2 + 8;
+constexpr int kDenseCols = kWin + 8;
+constexpr int kDenseCells = kDenseRows * kDenseCols;
+
+// The windows that dense pieces reach: the sum of the pieces' shares, in piece order (of the window's
+// own halves, then of those above and to the left), added to what the window's wavefront item
+// wrote to the planes, if it has one; so the result does not depend on timing.  One unit =
+// (listed window, term) per workgroup, a thread per cell.  Bound by latency (a unit's chain of
+// descriptor, slots and planes), so many small workgroups are resident, and the densest windows,
+// with over a hundred pieces, are read sixteen pieces at a time.
+__global__ void __launch_bounds__(256)
+k_win_reduce(const WReduce* __restrict__ red, const uint32_t* __restrict__ totals, WinGeom wg,
              int G, int K, uint32_t max_slots, const float2* __restrict__ partial, float2* __restrict__ planes) {
-    __shared__ float2 s_sum[kReduceGroups - 1][256];
-    const int n = 2 * kItemClasses * wg.nwin_total;
     const uint32_t units = totals[6] * static_cast<uint32_t>(K);
     const size_t plane_size = static_cast<size_t>(G) * G;
-    const size_t piece_size = static_cast<size_t>(K) * kWin * kWin;
-    const int cell = threadIdx.x & 255, grp = threadIdx.x >> 8;
+    const size_t piece_size = static_cast<size_t>(K) * kDenseCells;
+    const int cell = threadIdx.x, row = cell / kWin, col = cell % kWin;
     for (uint32_t u = blockIdx.x; u < units; u += gridDim.x) {
-        const int w = static_cast<int>(multi[u / K]);
-        const int k = static_cast<int>(u % K);
-        uint32_t end;
-        const WinRange x = window_range(boff, wg, w, end);
-        const uint32_t pieces = coop_pieces(wg, end - x.start());
-        const uint32_t first = ioff[n + w] - ioff[n];
-        if (first + pieces > max_slots) continue;          // never: the slot count bounds the pieces
-        const float2* src = partial + (first + grp) * piece_size + static_cast<size_t>(k) * kWin * kWin + cell;
-        const size_t step = kReduceGroups * piece_size;
-        // This group's pieces, eight requested at a time, summed into four accumulators in a
-        // fixed order.
-        const uint32_t mine = pieces > static_cast<uint32_t>(grp) ? (pieces - grp + kReduceGroups - 1) / kReduceGroups : 0;
-        float2 acc[4] = {};
-        uint32_t p = 0;
-        for (; p + 8 <= mine; p += 8) {
-            float2 v[8];
+        const WReduce& r = red[u / K];
+        const int k = static_cast<int>(u % K), w = r.win;
+        const int ls = w / wg.nwin, rem = w - ls * wg.nwin;
+        const int wa = rem / wg.nw, wb = rem - wa * wg.nw;
+        const int a = wa * kWin + row, b = wb * kWin + col;
+        const bool in_grid = a < G && b < G;
+        float2* dst = planes + (static_cast<size_t>(ls) * K + k) * plane_size + static_cast<size_t>(a) * G + b;
+        // The sum is FP64: over a hundred FP32 additions one after another would cost half a digit
+        // (6.3e-7 against 3.1e-7 of the signed SKA-Low image).
+        double sx = 0.0, sy = 0.0;
+        if (r.add != 0 && in_grid) {
+            const float2 v = *dst;
+            sx = v.x;
+            sy = v.y;
+        }
+        auto add_pieces = [&](int j, bool reached, int at) {
+            const uint32_t first = r.first[j], pieces = r.count[j];
+            if (pieces == 0 || !reached || first + pieces > max_slots) return;   // (the slot count bounds the pieces)
+            const float2* src = partial + first * piece_size + static_cast<size_t>(k) * kDenseCells + at;
+            uint32_t p = 0;
+            for (; p + 16 <= pieces; p += 16) {
+                float2 v[16];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = src[(p + j) * step];
+                for (int q = 0; q < 16; ++q) v[q] = src[(p + q) * piece_size];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                acc[j & 3].x += v[j].x;
-                acc[j & 3].y += v[j].y;
+                for (int q = 0; q < 16; ++q) {
+                    sx += v[q].x;
+                    sy += v[q].y;
+                }
             }
-        }
-        for (; p < mine; ++p) {
-            const float2 v = src[p * step];
-            acc[p & 3].x += v.x;
-            acc[p & 3].y += v.y;
-        }
-        const float2 sum = make_float2((acc[0].x + acc[1].x) + (acc[2].x + acc[3].x),
-                                       (acc[0].y + acc[1].y) + (acc[2].y + acc[3].y));
-        if (grp > 0) s_sum[grp - 1][cell] = sum;
-        __syncthreads();
-        if (grp == 0) {
-            float2 t = sum;
-#pragma unroll
-            for (int g = 0; g < kReduceGroups - 1; ++g) {
-                t.x += s_sum[g][cell].x;
-                t.y += s_sum[g][cell].y;
+            for (; p < pieces; ++p) {
+                const float2 v = src[p * piece_size];
+                sx += v.x;
+                sy += v.y;
             }
-            const int ls = w / wg.nwin, r = w - ls * wg.nwin;
-            const int wa = r / wg.nw, wb = r - wa * wg.nw;
-            const int a = wa * kWin + cell / kWin, b = wb * kWin + cell % kWin;
-            if (a < G && b < G)
-                planes[(static_cast<size_t>(ls) * K + k) * plane_size + static_cast<size_t>(a) * G + b] = t;
-        }
-        __syncthreads();
+        };
+        const int at = row * kDenseCols + col;
+        constexpr int kDown = (kWin / 2) * kDenseCols;     // eight rows
+        add_pieces(0, true, at);
+        add_pieces(1, row >= 8, at - kDown);
+        add_pieces(2, row < 8, at + kDown);
+        add_pieces(3, col < 8, at + kWin);
+        add_pieces(4, col < 8 && row >= 8, at + kWin - kDown);
+        add_pieces(5, col < 8 && row < 8, at + kWin + kDown);
+        if (in_grid) *dst = make_float2(static_cast<float>(sx), static_cast<float>(sy));
     }
 }
 
@@ -708,20 +805,42 @@ __device__ __forceinline__ void wave_lds_sync() {
 // hi*lo.  Otherwise B_a = f16(uh vh) (relative error <= 3 x 2^-11 against ku kv, from the three
 // roundings) and D_a += C_hi B_a [+ C_lo B_a].
 template <int P>
-__device__ __forceinline__ void window_row_regs(floatx4& d, const half8& uh, const half8& ul, const half8& vh,
-                                                const half8& vl, const half8& a_hi, const half8& a_lo) {
+__device__ __forceinline__ void es_product(const half8& uh, const half8& ul, const half8& vh, const half8& vl, half8& b_hi,
+                                           half8& b_lo) {
+    b_hi = uh * vh;
+    b_lo = b_hi;
     if constexpr (P == kPrecSplit3) {
-        const half8 p = uh * vh;
-        const half8 e = __builtin_elementwise_fma(uh, vh, -p);
-        const half8 b_lo = __builtin_elementwise_fma(ul, vh, __builtin_elementwise_fma(uh, vl, e));
-        const half8 b_hi = p;
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_hi, b_hi, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_lo, b_hi, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_hi, b_lo, d, 0, 0, 0);
-    } else {
-        const half8 b = uh * vh;
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_hi, b, d, 0, 0, 0);
-        if constexpr (P == kPrecSplitC) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_lo, b, d, 0, 0, 0);
+        const half8 e = __builtin_elementwise_fma(uh, vh, -b_hi);
+        b_lo = __builtin_elementwise_fma(ul, vh, __builtin_elementwise_fma(uh, vl, e));
+    }
+}
+template <int P>
+__device__ __forceinline__ void contract(floatx4& d, const half8& a_hi, const half8& a_lo, const half8& b_hi, const half8& b_lo) {
+    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_hi, b_hi, d, 0, 0, 0);
+    if constexpr (P != kPrecSingle) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_lo, b_hi, d, 0, 0, 0);
+    if constexpr (P == kPrecSplit3) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_hi, b_lo, d, 0, 0, 0);
+}
+
+// The eight ES values (times 2^7, and times dith with kDith) of a footprint with fraction F = t +
+// 1/2: cell j is at x = (F + j) / 4 - 1, for j < 8 the quarter-support polynomial pair (j, 7 - j)
+// in t.
+template <bool kDith>
+__device__ __forceinline__ void es_cells(float t, float dith, float (&v)[8]) {
+    const float t2 = t * t;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float e = kEsPolyEven[j][kEsPolyDegree / 2];
+#pragma unroll
+        for (int i = kEsPolyDegree / 2 - 1; i >= 0; --i) e = fmaf(e, t2, kEsPolyEven[j][i]);
+        float o = kEsPolyOdd[j][kEsPolyDegree / 2 - 1];
+#pragma unroll
+        for (int i = kEsPolyDegree / 2 - 2; i >= 0; --i) o = fmaf(o, t2, kEsPolyOdd[j][i]);
+        if constexpr (kDith) {
+            e *= dith;
+            o *= dith;
+        }
+        v[j] = fmaf(t, o, e);
+        v[7 - j] = fmaf(-t, o, e);
     }
 }
 
@@ -748,10 +867,10 @@ template <int P>
 __device__ __forceinline__ void window_chunk(const WinLane& L, const WItem& it, int c0, int kg, int K,
                                              int cls_log2, const uint4& q, floatx4 (&d)[kWin]) {
     using T = WinTraits<P>;
-    const bool valid = c0 + L.rl < it.count;
+    bool valid = c0 + L.rl < it.count;
     // Classes of the chunk's first and last records (wave-uniform), and the 4-row quarters of
     // the window that they touch: class j covers rows [c d, c d + c + 7], d = j - 8 / c.
-    const int i0 = it.start + c0, i1 = min(it.start + it.count, i0 + kChunk);
+    const int i0 = it.record(c0), i1 = it.record(min(it.count, c0 + kChunk) - 1) + 1;
     // (i >= bnd as the sign of bnd - 1 - i, so that the sums stay in scalar registers; bnd[j] for
     // j >= ncls is the window's end, which no record reaches.)
     int j_first = 0, j_last = 0;
@@ -798,8 +917,12 @@ __device__ __forceinline__ void window_chunk(const WinLane& L, const WItem& it, 
     // that reads the class); this window reads the classes j >= 16 / c as the row above their
     // home, 16 rows up.
     const int foreign = cls_log2 == 2 ? it.bnd[4] : it.bnd[2];
+    const int i = it.record(c0 + L.rl);
+    if (it.skip != 0 && rec_cell(q.w) < 0) {
+        const int part = i >= foreign ? 4 : i >= (cls_log2 == 2 ? it.bnd[2] : it.bnd[1]) ? 2 : 1;
+        valid = valid && (it.skip & part) == 0;
+    }
     if (valid) {
-        const int i = i0 + L.rl;
         const uint32_t pw = L.axis ? q.w : q.z;
         const int fl = rec_cell(pw) + (L.axis == 0 && i >= foreign ? kWin : 0);
         const uint32_t fb = rec_frac_bits(pw);
@@ -807,24 +930,10 @@ __device__ __forceinline__ void window_chunk(const WinLane& L, const WItem& it, 
         // Cell j is at x = (F + j) / 4 - 1 (F the record's fraction in [0, 1)): for j < 8 the
         // quarter-support polynomial pair (j, 7 - j) in t = F - 1/2, for j = 8 ES(1) when F = 0
         // and zero otherwise.
-        const float t = fmaf(static_cast<float>(fb), kRecFracInv, -0.5f), t2 = t * t;
+        const float t = fmaf(static_cast<float>(fb), kRecFracInv, -0.5f);
         const float dith = L.axis ? dith_v : dith_u;
         float v[8];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float e = kEsPolyEven[j][kEsPolyDegree / 2];
-#pragma unroll
-            for (int i = kEsPolyDegree / 2 - 1; i >= 0; --i) e = fmaf(e, t2, kEsPolyEven[j][i]);
-            float o = kEsPolyOdd[j][kEsPolyDegree / 2 - 1];
-#pragma unroll
-            for (int i = kEsPolyDegree / 2 - 2; i >= 0; --i) o = fmaf(o, t2, kEsPolyOdd[j][i]);
-            if constexpr (T::kDither) {
-                e *= dith;
-                o *= dith;
-            }
-            v[j] = fmaf(t, o, e);
-            v[7 - j] = fmaf(-t, o, e);
-        }
+        es_cells<T::kDither>(t, dith, v);
         if constexpr (T::kBf16) {
             float* df = L.s_kf + (first + kPad) * kStrideF;
 #pragma unroll
@@ -936,43 +1045,40 @@ __device__ __forceinline__ void window_chunk(const WinLane& L, const WItem& it, 
                     uh_n = *reinterpret_cast<const half8*>(uhb + (a + 1) * kStrideH);
                     if constexpr (T::kEsLo) ul_n = *reinterpret_cast<const half8*>(ulb + (a + 1) * kStrideH);
                 }
-                window_row_regs<P>(d[a], uh, ul, vh, vl, a_hi, a_lo);
+                half8 b_hi, b_lo;
+                es_product<P>(uh, ul, vh, vl, b_hi, b_lo);
+                contract<P>(d[a], a_hi, a_lo, b_hi, b_lo);
             }
         }
     }
     wave_lds_sync();
 }
 
-// Destination of the window values of (row a, term k, column n16): the planes for a whole
-// window, the partial slot ([k][16][16]) for a piece; out-of-grid cells and k >= K go to the
-// scratch line `trash` so that every lane issues the same stores.
+// Destination of the window values of (row a, term k, column n16) in the planes; out-of-grid cells
+// and k >= K go to the scratch line `trash` so that every lane issues the same stores.
 struct WinOut {
     float2* base;
-    int kstride, astride;
-    bool piece;
+    int kstride, wa16, wb16;
 };
-__device__ __forceinline__ WinOut window_out(const WItem& it, const WinGeom& wg, int K, int G, float2* planes,
-                                             float2* partial, int n16) {
+__device__ __forceinline__ WinOut window_out(const WItem& it, const WinGeom& wg, int K, int G, float2* planes, int n16) {
     const int ls = it.win / wg.nwin, w = it.win - ls * wg.nwin;
     const int wa = w / wg.nw, wb = w - wa * wg.nw;
     const size_t plane_size = static_cast<size_t>(G) * G;
     WinOut o;
-    o.piece = it.slot >= 0;
-    o.base = o.piece ? partial + static_cast<size_t>(it.slot) * K * kWin * kWin + n16
-                     : planes + static_cast<size_t>(ls) * K * plane_size + static_cast<size_t>(wa) * kWin * G + wb * kWin + n16;
+    o.base = planes + static_cast<size_t>(ls) * K * plane_size + static_cast<size_t>(wa) * kWin * G + wb * kWin + n16;
     // Offsets from base fit in 32 bits: k * G^2 + 15 G < 2^31 for K <= 32, G <= 8192.
-    o.kstride = o.piece ? kWin * kWin : static_cast<int>(plane_size);
-    o.astride = o.piece ? kWin : G;
+    o.kstride = static_cast<int>(plane_size);
+    o.wa16 = wa * kWin;
+    o.wb16 = wb * kWin;
     return o;
 }
 
-__device__ __forceinline__ void window_store(const WinOut& o, const WItem& it, const WinGeom& wg, int G, int K,
-                                             int a, int k, int n16, float inv, float2 v, float2* trash, int lane) {
-    const int w = it.win % wg.nwin;
-    const int ag = (w / wg.nw) * kWin + a, bg = (w % wg.nw) * kWin + n16;
+__device__ __forceinline__ void window_store(const WinOut& o, int G, int K, int a, int k, int n16, float inv, float2 v,
+                                             float2* trash, int lane) {
+    const int ag = o.wa16 + a, bg = o.wb16 + n16;
     const float sg = ((ag + bg) & 1) ? -inv : inv;
-    const bool ok = k < K && (o.piece || (ag < G && bg < G));
-    float2* dst = ok ? o.base + (k * o.kstride + a * o.astride) : trash + lane;
+    const bool ok = k < K && ag < G && bg < G;
+    float2* dst = ok ? o.base + (k * o.kstride + a * G) : trash + lane;
     *dst = make_float2(v.x * sg, v.y * sg);
 }
 
@@ -994,14 +1100,18 @@ struct WinJobs {
     int count;
 };
 
-// The c scale of a job from the largest |v| of its call: |c| <= 2^14 after scaling.
-__device__ __forceinline__ void job_scale(const WinJob& J, WinLane& L) {
+// The c scale of a job from the largest |v| of its call: |c| <= 2^14 after scaling by 2^vexp;
+// inv undoes it and the ES factors' scale.
+struct JobScale {
+    int vexp;
+    float inv;
+};
+__device__ __forceinline__ JobScale job_scale(const WinJob& J) {
     const float vmax = __uint_as_float(J.totals[4]);
     int e = 0;
     if (vmax > 0.0f && vmax <= 3.0e38f) (void)frexpf(vmax, &e);
     e = min(max(e, -100), 100);
-    L.vexp = 14 - e;
-    L.inv = ldexpf(1.0f, e - 14 - kEsScaleLog2Sq);
+    return {14 - e, ldexpf(1.0f, e - 14 - kEsScaleLog2Sq)};
 }
 
 // The job of global item index g of a queue whose per-job starts are off[0 .. count] (LDS):
@@ -1012,22 +1122,558 @@ __device__ __forceinline__ int job_of(const int* off, int count, int g) {
     return j;
 }
 
-// Persistent workgroups, one per CU, over the items of all the launch's jobs.  First the
-// workgroup items of every job, from one queue: all wavefronts of the workgroup claim the item's
-// chunks from a shared counter, then sum their accumulators in LDS (over the staging area) and
-// the workgroup writes the window once.  Then the wavefront items of every job, each wavefront
-// on its own: the next item is claimed while the current one is contracted and its first records
-// are requested before the current window is written, so the write-out overlaps the next item's
+// ---- Dense halves -----------------------------------------------------------------------------
+//
+// k_win_dense contracts the home records of the dense half windows sorted by footprint column.  In
+// the 16 x 16 window contraction a record's 8 x 8 footprint meets on average half of the window's
+// rows and all 16 columns are computed for its eight; records that share their footprint's first
+// column b0 fit exactly: the 16 columns of an MFMA block are two grid rows times the eight columns
+// b0 .. b0 + 7, and records sorted by their first row a0 within b0 need four to six of the eight
+// blocks that cover the half's rows.
+//
+// A workgroup takes one piece (records of one half window): it sorts their indices in LDS by (b0,
+// a0), kBatch at a time, and its wavefronts claim runs of 32-record chunks of the sorted list.  A
+// wavefront keeps the eight blocks of its current column b0 in registers and adds them to the
+// piece's tile in LDS (16 rows x 24 columns x 2K) when the column changes or the run ends; a chunk
+// that meets several columns is contracted once per column with c masked.  The tile is FP64
+// because its LDS atomics are: ds_add_f32 handles one lane in three cycles on this chip (193 cycles
+// per wavefront, measured), ds_add_f64 a wavefront in 9.
+//
+// Measured (SKA-Low snapshot, 8.4 M samples at 1024^2, 62% of the records in dense halves): 250 us, and
+// 143 us for the wavefront items that remain, against 476 us for window contraction of everything;
+// eight such snapshots in a batch 5.43 against 6.11 ms.  It issues a quarter of the MFMAs and 0.4 of
+// the VALU instructions of the window form (3.5 M and 71 M).  About 110 us of it are the sort, the
+// tile's clearing and write-out and the barriers around them, the rest the chunks, which wait for
+// their LDS operands as long as they compute (a chunk's chain is about 5000 cycles with three
+// wavefronts per SIMD).  Tried and slower: four wavefronts per SIMD at 128 registers (spills; 265 us),
+// two workgroups of six wavefronts per CU (490 us, smaller batches), one wavefront sorting a batch
+// ahead of the others (260 us), touching the next piece's lines early (255 us), private FP32
+// slots with global atomics (27 us per thousand tile updates).
+constexpr int kDenseHalf = kWin / 2;
+constexpr int kDenseColumns = kWin + 8;                         // first columns -8 .. 15 (copies: -8 .. -1)
+constexpr int kDenseGroups = 2 * kDenseColumns;                 // (first rows -8 .. -1 at the grid's top edge, 0 .. 7)
+constexpr int kDenseKeys = kDenseHalf * kDenseGroups;
+constexpr int kDenseTileStride = kDenseCells + 2;               // doubles per m
+constexpr int kDenseURows = 16, kDenseVRows = 9;                // staged rows; columns + the ninth cell
+constexpr int kDenseBlocks = kDenseURows / 2;
+constexpr int kDStride = 32;                                    // halves or floats per staged ES row (a block's B operand
+                                                                // reads two adjacent rows: no padding needed)
+
+template <int P, int MB>
+struct DenseTraits {
+    using T = WinTraits<P>;
+    static constexpr int kWaves = MB == 1 ? 12 : 8;
+    static constexpr int kBatch = MB == 1 ? 8192 : 4096;        // records sorted at a time
+    static constexpr int kPer = (kBatch + kWaves * 64 - 1) / (kWaves * 64);
+    static constexpr int kRows = kDenseURows + kDenseVRows;
+    // Per wavefront: the ES rows (ku hi [lo], kv hi [lo] in f16, or ku, kv in FP32), then c[16].
+    static constexpr int kEsFloats = T::kBf16 ? kRows * kDStride : kRows * kDStride * (T::kEsLo ? 2 : 1) / 2;
+    static constexpr int kStageFloats = kEsFloats + 16 * kStride;
+    static constexpr int kTileFloats = 2 * 16 * MB * kDenseTileStride;
+    static constexpr size_t kLds = sizeof(float) * (kTileFloats + kWaves * kStageFloats) + sizeof(uint16_t) * kBatch +
+                                   sizeof(uint32_t) * (kDenseKeys + 2 * 64 + 2);
+    static_assert(kEsFloats % 4 == 0 && kTileFloats % 4 == 0, "16-byte aligned staging rows");
+};
+
+// Barrier for data exchanged through LDS: global loads and stores stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// A wavefront's staging area and place in the chunk.
+template <int P>
+struct DenseLane {
+    _Float16 *s_kuh, *s_kvh;        // ku rows (hi, then lo), kv rows
+    float *s_kuf, *s_kvf;           // FP32 rows (kPrecBf16)
+    float* s_c;
+    double* tile;
+    int lane, rl, axis, g8, n16;
+};
+
+// The C operands of a chunk: A (16 x 32): lane holds A[n16][g8 + i], hi and lo, per 16-row block.
+template <int P, int MB>
+struct DenseC {
+    typedef typename std::conditional<WinTraits<P>::kBf16, bf16x8, half8>::type op8;
+    op8 hi[MB], lo[MB];
+};
+
+template <int P, int MB>
+__device__ __forceinline__ void load_c(const DenseLane<P>& L, int mb, DenseC<P, MB>& A) {
+    const float* row = L.s_c + L.n16 * kStride + L.g8;
+    const float4 x0 = *reinterpret_cast<const float4*>(row), x1 = *reinterpret_cast<const float4*>(row + 4);
+    if constexpr (WinTraits<P>::kBf16) {
+        const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        split_bf16(x, A.hi[mb], A.lo[mb]);
+    } else if constexpr (WinTraits<P>::kCLo) {
+        split_hilo(x0, x1, A.hi[mb], A.lo[mb]);
+    } else {
+        A.hi[mb] = __builtin_convertvector((floatx8){x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w}, half8);
+        A.lo[mb] = A.hi[mb];
+    }
+}
+
+// The operands of one chunk of a dense piece, staged: `cnt` records (this lane's in q; lanes past
+// them hold the last one and contribute c = 0) for the terms kg .. kg + 8 MB - 1.  Returns the
+// blocks that the chunk's rows meet, q_lo .. q_hi; row_adj: row of the stored cell 0 in the half.
+template <int P, int MB>
+__device__ __forceinline__ void dense_stage(const DenseLane<P>& L, int cnt, int kg, int vexp, int row_adj, const uint4& q,
+                                            int& q_lo, int& q_hi, DenseC<P, MB>& A) {
+    using T = WinTraits<P>;
+    const int lane = L.lane, rl = L.rl, axis = L.axis;
+    const bool valid = rl < cnt;
+    const uint32_t pw = axis ? q.w : q.z;
+    const uint32_t fb = rec_frac_bits(pw);
+    const bool edge = fb == 0u;
+    // First row within the half's eight (row_adj is a multiple of eight).
+    const int r0 = rec_cell(pw) & (kDenseHalf - 1);
+    {
+        const int lo = axis ? kDenseHalf : r0, hi = axis ? 0 : r0 + (edge ? 1 : 0);
+        q_lo = __ballot(lo < 2) != 0 ? 0 : __ballot(lo < 4) != 0 ? 1 : __ballot(lo < 6) != 0 ? 2 : 3;
+        q_hi = __ballot(hi >= 7) != 0 ? 7 : __ballot(hi >= 5) != 0 ? 6 : __ballot(hi >= 3) != 0 ? 5 : __ballot(hi >= 1) != 0 ? 4 : 3;
+    }
+    const uint64_t edges = __ballot(axis && valid && edge) >> 32;
+    float dith_u = 1.0f, dith_v = 1.0f;
+    if constexpr (T::kDither) {                     // (as window_chunk)
+        const uint32_t h = (q.x ^ q.y ^ q.z) * 0x9E3779B1u;
+        dith_u = 1.0f + static_cast<float>(h >> 24) * (1.0f / 256.0f);
+        dith_v = 1.0f + static_cast<float>((h >> 16) & 0xffu) * (1.0f / 256.0f);
+    }
+    // The rows of ku are cleared, then every lane writes its sample's cells: ku at rows r0 .. r0 + 8 of
+    // sixteen, kv at rows 0 .. 7 (and its ninth cell at a row that is not read).
+    {
+        const uint4 z = make_uint4(0u, 0u, 0u, 0u);
+        if constexpr (T::kBf16) {
+#pragma unroll
+            for (int i = 0; i < kDenseURows * 8; i += 64)
+                reinterpret_cast<uint4*>(L.s_kuf + ((lane + i) >> 3) * kDStride)[lane & 7] = z;
+        } else {
+            constexpr int kRows = kDenseURows * (T::kEsLo ? 2 : 1);
+#pragma unroll
+            for (int i = 0; i < kRows * 4; i += 64)
+                reinterpret_cast<uint4*>(L.s_kuh + ((lane + i) >> 2) * kDStride)[lane & 3] = z;
+        }
+    }
+    wave_lds_sync();
+    const int row0 = axis ? 0 : r0;
+    {
+        const float dith = axis ? dith_v : dith_u;
+        float v[8];
+        es_cells<T::kDither>(fmaf(static_cast<float>(fb), kRecFracInv, -0.5f), dith, v);
+        if constexpr (T::kBf16) {
+            float* df = (axis ? L.s_kvf : L.s_kuf) + rl + row0 * kDStride;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) df[j * kDStride] = v[j];
+            df[8 * kDStride] = edge ? kEsPolyEdge : 0.0f;
+        } else {
+            _Float16* dh = (axis ? L.s_kvh : L.s_kuh) + rl + row0 * kDStride;
+            _Float16* dl = dh + (axis ? kDenseVRows : kDenseURows) * kDStride;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const half2v h = __builtin_convertvector((float2v){v[j], v[7 - j]}, half2v);
+                dh[j * kDStride] = h[0];
+                dh[(7 - j) * kDStride] = h[1];
+                if constexpr (T::kEsLo) {
+                    const half2v l = residual_f16x2(h, v[j], v[7 - j]);
+                    dl[j * kDStride] = l[0];
+                    dl[(7 - j) * kDStride] = l[1];
+                }
+            }
+            if constexpr (T::kEsLo) {
+                dh[8 * kDStride] = edge ? kEsPolyEdgeHi : static_cast<_Float16>(0.0f);
+                dl[8 * kDStride] = edge ? kEsPolyEdgeLo : static_cast<_Float16>(0.0f);
+            } else {
+                dh[8 * kDStride] = static_cast<_Float16>(edge ? kEsPolyEdge * dith : 0.0f);
+            }
+        }
+    }
+    // c rows 2k + axis for the terms kg .. kg + 8 MB - 1 (terms k >= K are dropped at write-out).
+    {
+        float vs = valid ? rec_v(axis ? q.y : q.x, q.w, vexp) : 0.0f;
+        if constexpr (T::kDither) vs *= __builtin_amdgcn_rcpf(dith_u * dith_v);
+        const float s = rec_s(q.x, q.y, q.z), s2 = 2.0f * s;
+        float t0 = 1.0f, t1 = s;
+        for (int k = 0; k < kg; ++k) {
+            const float t2 = s2 * t1 - t0;
+            t0 = t1;
+            t1 = t2;
+        }
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            if (mb > 0) wave_lds_sync();
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                L.s_c[(2 * j + axis) * kStride + rl] = t0 * vs;
+                const float t2 = s2 * t1 - t0;
+                t0 = t1;
+                t1 = t2;
+            }
+            wave_lds_sync();
+            if constexpr (MB > 1) load_c<P, MB>(L, mb, A);
+            // Footprints of an exactly integer column position have a ninth column, of value ES(1):
+            // their contribution to it goes straight to the tile, one record at a time.
+            for (uint64_t left = edges; left != 0; left &= left - 1) {
+                const int r = __builtin_ctzll(left);
+                const int rb = ((__shfl(rec_cell(q.z) + row_adj, r, 64) + kPad) & ~(kDenseHalf - 1)) - kPad;
+                const int col = __shfl(rec_cell(q.w), r, 64) + 8;
+                const float ev = kEsPolyEdge * __shfl(dith_v, r, 64);
+                if (col < 0 || col >= kDenseCols) continue;
+                for (int t = lane; t < 16 * kDenseURows; t += 64) {
+                    const int m = t / kDenseURows, a = t - m * kDenseURows, ar = rb + a;
+                    float ku;
+                    if constexpr (T::kBf16) {
+                        ku = L.s_kuf[a * kDStride + r];
+                    } else {
+                        ku = static_cast<float>(L.s_kuh[a * kDStride + r]);
+                        if constexpr (T::kEsLo) ku += static_cast<float>(L.s_kuh[(kDenseURows + a) * kDStride + r]);
+                    }
+                    if (ar >= 0 && ar < kDenseRows)
+                        atomicAdd(L.tile + (16 * mb + m) * kDenseTileStride + ar * kDenseCols + col,
+                                  static_cast<double>(L.s_c[m * kStride + r]) * (ku * ev));
+                }
+            }
+        }
+    }
+}
+
+// The staged chunk's records of bits `sel` (bit i = record i) contracted into the blocks d.
+// B (32 x 16): lane holds B[g8 + i][n16] = ku of row 2b + n16 / 8 times kv of column n16 % 8;
+// D (16 x 16): lane holds D[4 (lane / 16) + i][n16].
+template <int P, int MB>
+__device__ __forceinline__ void dense_contract(const DenseLane<P>& L, const DenseC<P, MB>& A, uint32_t sel, int q_lo, int q_hi,
+                                               floatx4 (&d)[MB][kDenseBlocks]) {
+    using T = WinTraits<P>;
+    const int g8 = L.g8, n16 = L.n16, par = n16 >> 3, j8 = n16 & 7;
+    using op8 = typename DenseC<P, MB>::op8;
+    typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+    // (With one block c is still staged: splitting it again costs less than holding it.)
+    DenseC<P, MB> C = A;
+    if constexpr (MB == 1) load_c<P, MB>(L, 0, C);
+    auto& a_hi = C.hi;
+    auto& a_lo = C.lo;
+    if (sel != 0xffffffffu) {
+        const int m8 = static_cast<int>(sel >> g8);
+        uint4v mask;
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+            mask[p] = (static_cast<uint32_t>((m8 << (31 - 2 * p)) >> 31) & 0xffffu) | (static_cast<uint32_t>((m8 << (30 - 2 * p)) >> 31) & 0xffff0000u);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            a_hi[mb] = __builtin_bit_cast(op8, __builtin_bit_cast(uint4v, a_hi[mb]) & mask);
+            a_lo[mb] = __builtin_bit_cast(op8, __builtin_bit_cast(uint4v, a_lo[mb]) & mask);
+        }
+    }
+    if constexpr (T::kBf16) {
+        const float* vrow = L.s_kvf + j8 * kDStride + g8;
+        const float4 v0 = *reinterpret_cast<const float4*>(vrow), v1 = *reinterpret_cast<const float4*>(vrow + 4);
+#pragma unroll
+        for (int b = 0; b < kDenseBlocks; ++b) {
+            if (b < q_lo || b > q_hi) continue;
+            const float* ur = L.s_kuf + (2 * b + par) * kDStride + g8;
+            const float4 u0 = *reinterpret_cast<const float4*>(ur), u1 = *reinterpret_cast<const float4*>(ur + 4);
+            const float p[8] = {u0.x * v0.x, u0.y * v0.y, u0.z * v0.z, u0.w * v0.w,
+                                u1.x * v1.x, u1.y * v1.y, u1.z * v1.z, u1.w * v1.w};
+            bf16x8 b_hi, b_lo;
+            split_bf16(p, b_hi, b_lo);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                d[mb][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi[mb], b_hi, d[mb][b], 0, 0, 0);
+                d[mb][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo[mb], b_hi, d[mb][b], 0, 0, 0);
+                d[mb][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi[mb], b_lo, d[mb][b], 0, 0, 0);
+            }
+        }
+    } else {
+        // Each block's ku values are requested one block ahead, so that their LDS latency overlaps the
+        // previous block's products and MFMAs.
+        const _Float16* urow = L.s_kuh + (2 * q_lo + par) * kDStride + g8;
+        half8 uh_n = *reinterpret_cast<const half8*>(urow);
+        half8 ul_n = uh_n;
+        if constexpr (T::kEsLo) ul_n = *reinterpret_cast<const half8*>(urow + kDenseURows * kDStride);
+        const _Float16* vrow = L.s_kvh + j8 * kDStride + g8;
+        const half8 vh = *reinterpret_cast<const half8*>(vrow);
+        half8 vl = vh;
+        if constexpr (T::kEsLo) vl = *reinterpret_cast<const half8*>(vrow + kDenseVRows * kDStride);
+#pragma unroll
+        for (int b = 0; b < kDenseBlocks; ++b) {
+            if (b < q_lo || b > q_hi) continue;
+            const half8 uh = uh_n, ul = ul_n;
+            if (b + 1 < kDenseBlocks) {                    // (unused past q_hi)
+                const _Float16* ur = L.s_kuh + (2 * b + 2 + par) * kDStride + g8;
+                uh_n = *reinterpret_cast<const half8*>(ur);
+                if constexpr (T::kEsLo) ul_n = *reinterpret_cast<const half8*>(ur + kDenseURows * kDStride);
+            }
+            half8 b_hi, b_lo;
+            es_product<P>(uh, ul, vh, vl, b_hi, b_lo);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) contract<P>(d[mb][b], a_hi[mb], a_lo[mb], b_hi, b_lo);
+        }
+    }
+}
+
+template <int P, int MB>
+__global__ void __launch_bounds__((DenseTraits<P, MB>::kWaves * 64))
+k_win_dense(WinJobs jobs) {
+    using T = WinTraits<P>;
+    using D = DenseTraits<P, MB>;
+    constexpr int kThreads = D::kWaves * 64;
+    extern __shared__ __align__(16) float dense_lds[];
+    __shared__ int s_item, s_chunk;
+    __shared__ int s_off[kMaxJobs + 1], s_wave_n[kMaxJobs];
+    DenseLane<P> L;
+    const int lane = L.lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    L.rl = lane & 31;
+    L.axis = lane >> 5;
+    L.g8 = 8 * (lane >> 4);
+    L.n16 = lane & 15;
+    double* const tile = L.tile = reinterpret_cast<double*>(dense_lds);
+    float* const stage = dense_lds + D::kTileFloats + wave * D::kStageFloats;
+    L.s_c = stage + D::kEsFloats;
+    L.s_kuh = reinterpret_cast<_Float16*>(stage);
+    L.s_kvh = L.s_kuh + kDenseURows * kDStride * (T::kEsLo ? 2 : 1);
+    L.s_kuf = stage;
+    L.s_kvf = stage + kDenseURows * kDStride;
+    uint16_t* const s_idx = reinterpret_cast<uint16_t*>(dense_lds + D::kTileFloats + D::kWaves * D::kStageFloats);
+    uint32_t* const s_hist = reinterpret_cast<uint32_t*>(s_idx + D::kBatch);
+    uint32_t* const s_gend = s_hist + kDenseKeys;          // the non-empty columns: end in the sorted list,
+    uint32_t* const s_gid = s_gend + 64;                   // and group; [128] their number
+    const int njobs = jobs.count;
+
+    // The jobs' pieces as offsets of one queue, whose head is job 0's totals[5].  The claimed index
+    // is read back into a scalar register, so the loop exit is wave-uniform by construction and
+    // every wavefront runs the same barriers.
+    if (threadIdx.x == 0) {
+        int c = 0;
+        for (int j = 0; j < njobs; ++j) {
+            s_off[j] = c;
+            s_wave_n[j] = static_cast<int>(jobs.job[j].totals[1]);
+            c += static_cast<int>(jobs.job[j].totals[3]);
+        }
+        s_off[njobs] = c;
+        s_item = static_cast<int>(atomicAdd(&jobs.job[0].totals[5], 1u));
+    }
+    // A piece's job and record range, requested while the piece before it is contracted.
+    struct Piece {
+        int job, start, count, half_skip, slot;
+        const uint4* rec;
+    };
+    auto fetch = [&](int gi, Piece& p) {
+        p.job = job_of(s_off, njobs, gi);
+        const WinJob& J = jobs.job[p.job];
+        const WItem* it = J.items + (__builtin_amdgcn_readfirstlane(s_wave_n[p.job]) +
+                                     (gi - __builtin_amdgcn_readfirstlane(s_off[p.job])));
+        p.start = __builtin_amdgcn_readfirstlane(it->start);
+        p.count = __builtin_amdgcn_readfirstlane(it->count);
+        p.half_skip = __builtin_amdgcn_readfirstlane(it->half | it->skip << 1);
+        p.slot = __builtin_amdgcn_readfirstlane(it->slot);
+        p.rec = J.rec.r + p.start;
+    };
+    lds_barrier();
+    const int nitems = __builtin_amdgcn_readfirstlane(s_off[njobs]);
+    int gi = __builtin_amdgcn_readfirstlane(s_item);
+    if (gi >= nitems) return;
+    Piece it;
+    fetch(gi, it);
+    for (;;) {
+        lds_barrier();                                   // s_item read; the tile is free
+        // The next piece is claimed now and published with this one's sorted indices.
+        uint32_t gnext = 0;
+        if (threadIdx.x == 0) gnext = atomicAdd(&jobs.job[0].totals[5], 1u);
+        int gi_next = nitems;
+        Piece itn;
+        const WinJob& J = jobs.job[it.job];
+        const JobScale scale = job_scale(J);
+        const int K = J.K;
+        // (The upper half's records store their row relative to the window below.)
+        const int row_adj = (it.half_skip & 1) ? kDenseHalf : 0;
+        const bool skip = (it.half_skip & 2) != 0;
+        for (int kg = 0; kg < K; kg += 8 * MB) {
+            for (int i = threadIdx.x; i < D::kTileFloats / 4; i += kThreads)
+                reinterpret_cast<float4*>(dense_lds)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            for (int b0 = 0; b0 < it.count; b0 += D::kBatch) {
+                const uint4* rec = it.rec + b0;
+                if (kg == 0 || it.count > D::kBatch) {
+                    // Sort the batch's records by key = (column, first row): counts with each record's
+                    // rank, the counts' prefix, then the sorted indices.
+                    const int nb = min(D::kBatch, it.count - b0);
+                    for (int i = threadIdx.x; i < kDenseKeys; i += kThreads) s_hist[i] = 0;
+                    uint2 w[D::kPer];                      // the records' last two words
+#pragma unroll
+                    for (int u = 0; u < D::kPer; ++u)
+                        w[u] = reinterpret_cast<const uint2*>(rec + min(static_cast<int>(threadIdx.x) + u * kThreads, nb - 1))[1];
+                    lds_barrier();
+                    uint32_t kr[D::kPer];
+#pragma unroll
+                    for (int u = 0; u < D::kPer; ++u) {
+                        const int i = threadIdx.x + u * kThreads;
+                        const int row = rec_cell(w[u].x) + row_adj, col = rec_cell(w[u].y);
+                        const uint32_t r = static_cast<uint32_t>(min(max(row, -kPad), kDenseHalf - 1) + kPad);
+                        const uint32_t c = static_cast<uint32_t>(min(max(col, -kPad), kWin - 1) + kPad);
+                        const uint32_t key = ((r >> 3) * kDenseColumns + c) * kDenseHalf + (r & 7u);
+                        kr[u] = ~0u;
+                        if (i < nb && !(skip && col < 0)) kr[u] = key << 16 | atomicAdd(&s_hist[key], 1u);
+                    }
+                    lds_barrier();
+                    if (wave == 0) {
+                        // One group (8 keys) per lane for 48 lanes.
+                        uint32_t h[kDenseHalf], tot = 0;
+                        const bool on = lane < kDenseGroups;
+#pragma unroll
+                        for (int i = 0; i < kDenseHalf; ++i) {
+                            h[i] = on ? s_hist[lane * kDenseHalf + i] : 0u;
+                            tot += h[i];
+                        }
+                        uint32_t pt = tot;
+                        for (int d = 1; d < 64; d <<= 1) {
+                            const uint32_t a = __shfl_up(pt, d, 64);
+                            if (lane >= d) pt += a;
+                        }
+                        const uint64_t some = __ballot(tot != 0);
+                        if (on) {
+                            uint32_t run = pt - tot;
+#pragma unroll
+                            for (int i = 0; i < kDenseHalf; ++i) {
+                                s_hist[lane * kDenseHalf + i] = run;
+                                run += h[i];
+                            }
+                        }
+                        if (tot != 0) {
+                            const int at = __popcll(some & ((1ull << lane) - 1));
+                            s_gend[at] = pt;
+                            s_gid[at] = lane;
+                        }
+                        if (lane == 0) s_gid[64] = static_cast<uint32_t>(__popcll(some));
+                    }
+                    lds_barrier();
+#pragma unroll
+                    for (int u = 0; u < D::kPer; ++u)
+                        if (kr[u] != ~0u) s_idx[s_hist[kr[u] >> 16] + (kr[u] & 0xffffu)] = static_cast<uint16_t>(threadIdx.x + u * kThreads);
+                }
+                if (threadIdx.x == 0) {
+                    s_chunk = 0;
+                    if (b0 == 0 && kg == 0) s_item = static_cast<int>(gnext);
+                }
+                lds_barrier();
+                if (b0 == 0 && kg == 0) {
+                    gi_next = __builtin_amdgcn_readfirstlane(s_item);
+                    if (gi_next < nitems) fetch(gi_next, itn);
+                }
+
+                // Runs of chunks, claimed from an LDS counter (the SIMDs issue their oldest wavefront
+                // first, so an even split would leave the piece waiting for the youngest): one run of
+                // r chunks per wavefront, then one of r / 2, then single chunks, r = half an even
+                // share.  Lane l holds column l of the list.
+                const int ngroups = __builtin_amdgcn_readfirstlane(static_cast<int>(s_gid[64]));
+                const uint32_t gend = lane < ngroups ? s_gend[lane] : 0xffffffffu;
+                const uint32_t gid = lane < ngroups ? s_gid[lane] : 0u;
+                const int n = ngroups > 0 ? __builtin_amdgcn_readlane(static_cast<int>(gend), ngroups - 1) : 0;
+                const int nch = (n + kChunk - 1) / kChunk;
+                const int run1 = max(1, nch / (2 * D::kWaves)), run2 = max(1, run1 / 2);
+                int left = 0;
+                auto claim = [&]() -> int {
+                    int v = 0;
+                    if (lane == 0) v = atomicAdd(&s_chunk, 1);
+                    v = __builtin_amdgcn_readfirstlane(v);
+                    const int v2 = v - D::kWaves, v3 = v2 - D::kWaves;
+                    left = v2 < 0 ? run1 : v3 < 0 ? run2 : 1;
+                    return v2 < 0 ? run1 * v : v3 < 0 ? run1 * D::kWaves + run2 * v2 : (run1 + run2) * D::kWaves + v3;
+                };
+                auto load = [&](int c) { return rec[s_idx[min(c * kChunk + L.rl, n - 1)]]; };
+                floatx4 d[MB][kDenseBlocks];
+                auto clear = [&]() {
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                        for (int q = 0; q < kDenseBlocks; ++q) d[mb][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+                };
+                auto flush = [&](int group) {
+                    const int rb = group < kDenseColumns ? -kPad : 0;
+                    const int col = (group < kDenseColumns ? group : group - kDenseColumns) - kPad + (L.n16 & 7);
+                    if (col >= 0) {
+                        double* at = tile + (4 * (lane >> 4)) * kDenseTileStride + (rb + (L.n16 >> 3)) * kDenseCols + col;
+#pragma unroll
+                        for (int q = 0; q < kDenseBlocks; ++q) {
+                            const int row = rb + 2 * q + (L.n16 >> 3);
+                            if (row >= 0 && row < kDenseRows) {
+#pragma unroll
+                                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                                    for (int i = 0; i < 4; ++i)
+                                        atomicAdd(at + (16 * mb + i) * kDenseTileStride + 2 * q * kDenseCols, static_cast<double>(d[mb][q][i]));
+                            }
+                        }
+                    }
+                    clear();
+                };
+                int c = claim();
+                uint4 q_next = make_uint4(0u, 0u, 0u, 0u);
+                if (c < nch) q_next = load(c);
+                clear();
+                int g = __popcll(__ballot(gend <= static_cast<uint32_t>(c * kChunk)));
+                bool held = false;                         // d holds sums of column g
+                while (c < nch) {
+                    const uint4 q = q_next;
+                    const int first = c * kChunk, last = min(first + kChunk, n);
+                    int next = c + 1;
+                    if (--left == 0) next = claim();
+                    if (next < nch) q_next = load(next);
+                    int q_lo, q_hi;
+                    DenseC<P, MB> A;
+                    dense_stage<P, MB>(L, last - first, kg, scale.vexp, row_adj, q, q_lo, q_hi, A);
+                    for (int at = first;;) {
+                        const int ge = __builtin_amdgcn_readlane(static_cast<int>(gend), g), to = min(ge, last);
+                        const uint32_t upto = to - first >= 32 ? 0xffffffffu : (1u << (to - first)) - 1u;
+                        const uint32_t sel = at == first && to == last ? 0xffffffffu : upto & ~((1u << (at - first)) - 1u);
+                        dense_contract<P, MB>(L, A, sel, q_lo, q_hi, d);
+                        held = true;
+                        if (ge <= last) {                  // the column ends in this chunk
+                            flush(__builtin_amdgcn_readlane(static_cast<int>(gid), g));
+                            held = false;
+                            ++g;
+                        }
+                        at = to;
+                        if (at >= last) break;
+                    }
+                    wave_lds_sync();
+                    if (next != c + 1) {                   // another run: its column
+                        if (held) flush(__builtin_amdgcn_readlane(static_cast<int>(gid), g));
+                        held = false;
+                        g = __popcll(__ballot(gend <= static_cast<uint32_t>(next * kChunk)));
+                    }
+                    c = next;
+                }
+                if (held) flush(__builtin_amdgcn_readlane(static_cast<int>(gid), g));
+                lds_barrier();
+            }
+            // The piece's share: [term][row][column] with the checkerboard sign.
+            float2* out = J.partial + (static_cast<size_t>(it.slot) * K + kg) * kDenseCells;
+            const int nk = min(8 * MB, K - kg);
+            for (int v = threadIdx.x; v < nk * kDenseCells; v += kThreads) {
+                const int k = v / kDenseCells, cell = v - k * kDenseCells;
+                const float sg = ((cell / kDenseCols + cell) & 1) ? -scale.inv : scale.inv;     // (kDenseCols even)
+                out[v] = make_float2(static_cast<float>(tile[2 * k * kDenseTileStride + cell]) * sg,
+                                     static_cast<float>(tile[(2 * k + 1) * kDenseTileStride + cell]) * sg);
+            }
+            if (kg + 8 * MB < K) lds_barrier();
+        }
+        if (gi_next >= nitems) break;
+        it = itn;
+    }
+}
+
+// Persistent workgroups, one per CU, over the wavefront items of all the launch's jobs: each
+// wavefront claims its next item while the current one is contracted and requests its first
+// records before the current window is written, so the write-out overlaps the next item's
 // loads (vector memory operations complete in order).  The terms are done eight at a time (one
 // 16-row block of m = 2k + ri).
 template <int P>
 __global__ void __launch_bounds__(WinTraits<P>::kWaves * 64)
 k_win_grid(WinJobs jobs) {
     using T = WinTraits<P>;
-    constexpr int kWaves = T::kWaves;
     extern __shared__ __align__(16) float stage_all[];
-    __shared__ int s_item, s_chunk, s_witem;
-    __shared__ int s_coop_off[kMaxJobs + 1], s_wave_off[kMaxJobs + 1];
+    __shared__ int s_witem;
+    __shared__ int s_wave_off[kMaxJobs + 1];
     WinLane L;
     const int wave = threadIdx.x >> 6;
     L.lane = threadIdx.x & 63;
@@ -1059,109 +1705,18 @@ k_win_grid(WinJobs jobs) {
     const int lane = L.lane;
     const int njobs = jobs.count;
 
-    // The jobs' item counts as queue offsets (workgroup items first, then wavefront items, each
-    // job's list in its largest-first order), and the first workgroup item claimed from the one
-    // queue head (job 0's totals[5]).  The claimed index is read back into a scalar register, so
-    // the loop exit is wave-uniform by construction and every wavefront runs the same barriers:
-    // were it left in a vector register, the compiler could treat the exit as divergent and let
-    // lanes other than thread 0 iterate without the claim.  Within an item the wavefronts claim
-    // chunks from an LDS counter (the SIMDs issue their oldest wavefront first, so an even split
-    // would leave the item waiting for the youngest); each claims its next chunk before
-    // contracting the current one, and requests that chunk's records at once.
-    const int wave_id = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    // The jobs' item counts as offsets into the one list (each job's items in its largest-first
+    // order).
     if (threadIdx.x == 0) {
-        int c = 0, w = 0;
+        int w = 0;
         for (int j = 0; j < njobs; ++j) {
-            s_coop_off[j] = c;
             s_wave_off[j] = w;
-            c += static_cast<int>(jobs.job[j].totals[3]);
             w += static_cast<int>(jobs.job[j].totals[1]);
         }
-        s_coop_off[njobs] = c;
         s_wave_off[njobs] = w;
-        s_chunk = 0;
         s_witem = 0;
-        s_item = static_cast<int>(atomicAdd(&jobs.job[0].totals[5], 1u));
     }
-    auto claim_chunk = [&]() -> int {
-        int v = 0;
-        if (lane == 0) v = atomicAdd(&s_chunk, kChunk);
-        return __builtin_amdgcn_readfirstlane(v);
-    };
-    for (;;) {
-        __syncthreads();
-        const int gi = __builtin_amdgcn_readfirstlane(s_item);
-        const int ncoop = __builtin_amdgcn_readfirstlane(s_coop_off[njobs]);
-        __syncthreads();
-        if (gi >= ncoop) break;
-        // The next item is claimed now; wavefront 0 publishes it after the last barrier of this one.
-        uint32_t gnext = 0;
-        if (wave_id == 0 && lane == 0) gnext = atomicAdd(&jobs.job[0].totals[5], 1u);
-        const int jj = job_of(s_coop_off, njobs, gi);
-        const WinJob& J = jobs.job[jj];
-        job_scale(J, L);
-        const int K = J.K, G = J.G;
-        const int nwave_j = __builtin_amdgcn_readfirstlane(s_wave_off[jj + 1] - s_wave_off[jj]);
-        const WItem it = J.items[nwave_j + (gi - __builtin_amdgcn_readfirstlane(s_coop_off[jj]))];
-        for (int kg = 0; kg < K; kg += 8) {
-            floatx4 d[kWin];
-#pragma unroll
-            for (int a = 0; a < kWin; ++a) d[a] = floatx4{0.f, 0.f, 0.f, 0.f};
-            int c0 = claim_chunk();
-            uint4 q_next = make_uint4(0u, 0u, 0u, 0u);
-            if (c0 < it.count) q_next = J.rec.get(it.start + min(c0 + L.rl, it.count - 1));
-            while (c0 < it.count) {
-                const uint4 q = q_next;
-                const int c1 = claim_chunk();
-                if (c1 < it.count) q_next = J.rec.get(it.start + min(c1 + L.rl, it.count - 1));
-                window_chunk<P>(L, it, c0, kg, K, J.wg.cls_log2, q, d);
-                c0 = c1;
-            }
-            // Sum the wavefronts' accumulators in LDS (over the staging area), in a fixed order:
-            // wavefronts 0 .. S-1 store theirs in slots 0 .. S-1, then each following group of S
-            // wavefronts adds theirs to slot w mod S, one group per round, and the write sums the
-            // S slots.  Slot layout red4[slot][a][lane] (float4 = the lane's
-            // D[4 (lane / 16) + i][n16], i = 0..3).  The chunk counter is reset for the next term
-            // block or item once every wavefront is done with it.
-            constexpr int kSlots = T::kSlots;
-            float4* red4 = reinterpret_cast<float4*>(stage_all);
-            __syncthreads();
-            if (wave_id < kSlots) {
-#pragma unroll
-                for (int a = 0; a < kWin; ++a)
-                    red4[(wave_id * kWin + a) * 64 + lane] = make_float4(d[a][0], d[a][1], d[a][2], d[a][3]);
-            }
-            if (threadIdx.x == 0) s_chunk = 0;
-            __syncthreads();
-#pragma unroll
-            for (int round = 1; round < kWaves / kSlots; ++round) {
-                if (wave_id >= round * kSlots && wave_id < (round + 1) * kSlots) {
-#pragma unroll
-                    for (int a = 0; a < kWin; ++a) {
-                        float4& r = red4[((wave_id - round * kSlots) * kWin + a) * 64 + lane];
-                        const float4 v = r;
-                        r = make_float4(v.x + d[a][0], v.y + d[a][1], v.z + d[a][2], v.w + d[a][3]);
-                    }
-                }
-                __syncthreads();
-            }
-            // Write: (row a, source lane sl) -> terms kg + 2 (sl / 16) + h, h = 0, 1, column sl % 16.
-            for (int v = threadIdx.x; v < kWin * 64; v += kWaves * 64) {
-                const int a = v >> 6, sl = v & 63;
-                float4 acc = red4[a * 64 + sl];
-#pragma unroll
-                for (int j = 1; j < kSlots; ++j) {
-                    const float4 x = red4[(j * kWin + a) * 64 + sl];
-                    acc = make_float4(acc.x + x.x, acc.y + x.y, acc.z + x.z, acc.w + x.w);
-                }
-                const WinOut os = window_out(it, J.wg, K, G, J.planes, J.partial, sl & 15);
-                window_store(os, it, J.wg, G, K, a, kg + 2 * (sl >> 4), sl & 15, L.inv, make_float2(acc.x, acc.y), J.trash, sl);
-                window_store(os, it, J.wg, G, K, a, kg + 2 * (sl >> 4) + 1, sl & 15, L.inv, make_float2(acc.z, acc.w), J.trash, sl);
-            }
-            __syncthreads();
-        }
-        if (wave_id == 0 && lane == 0) s_item = static_cast<int>(gnext);
-    }
+    __syncthreads();
 
     // Wavefront items of all jobs, one list.  Workgroup g takes items g, g + G, g + 2G, ... of it,
     // G = the number of workgroups, so the CUs get equal shares without a global queue; its
@@ -1184,28 +1739,30 @@ k_win_grid(WinJobs jobs) {
     WItem it = jobs.job[jj].items[item - __builtin_amdgcn_readfirstlane(s_wave_off[jj])];
     // Records of the next chunk, loaded while the current one is contracted.  Every lane loads
     // (lanes past the end re-read the last record and ignore it), so the loads land in place.
-    uint4 q_next = jobs.job[jj].rec.get(it.count > 0 ? it.start + min(L.rl, it.count - 1) : 0);
+    uint4 q_next = jobs.job[jj].rec.get(it.count > 0 ? it.record(min(L.rl, it.count - 1)) : 0);
     for (;;) {
         ticket = claim_item();
         const WinJob& J = jobs.job[jj];
-        job_scale(J, L);
+        const JobScale scale = job_scale(J);
+        L.vexp = scale.vexp;
+        L.inv = scale.inv;
         const int K = J.K, G = J.G;
         int next = nwave, jn = jj;
         WItem it_next = it;
-        const WinOut o = window_out(it, J.wg, K, G, J.planes, J.partial, L.n16);
+        const WinOut o = window_out(it, J.wg, K, G, J.planes, L.n16);
         for (int kg = 0; kg < K; kg += 8) {
             floatx4 d[kWin];
 #pragma unroll
             for (int a = 0; a < kWin; ++a) d[a] = floatx4{0.f, 0.f, 0.f, 0.f};
             for (int c0 = 0; c0 < it.count; c0 += kChunk) {
                 const uint4 q = q_next;
-                if (c0 + kChunk < it.count) q_next = J.rec.get(it.start + min(c0 + kChunk + L.rl, it.count - 1));
+                if (c0 + kChunk < it.count) q_next = J.rec.get(it.record(min(c0 + kChunk + L.rl, it.count - 1)));
                 window_chunk<P>(L, it, c0, kg, K, J.wg.cls_log2, q, d);
             }
             // What comes next: this item's next term block, or the next item (possibly of
             // another job).  Its first records are requested now, ahead of the stores below.
             {
-                int pstart = it.start, pcount = it.count;
+                int pcount = it.count, pfirst = it.record(min(L.rl, max(it.count - 1, 0)));
                 const WRecords* prec = &J.rec;
                 if (kg + 8 >= K) {
                     const int tn = __builtin_amdgcn_readfirstlane(ticket);
@@ -1213,14 +1770,14 @@ k_win_grid(WinJobs jobs) {
                     if (next < nwave) {
                         jn = job_of(s_wave_off, njobs, next);
                         it_next = jobs.job[jn].items[next - __builtin_amdgcn_readfirstlane(s_wave_off[jn])];
-                        pstart = it_next.start;
                         pcount = it_next.count;
+                        pfirst = it_next.record(min(L.rl, max(it_next.count - 1, 0)));
                         prec = &jobs.job[jn].rec;
                     } else {
                         pcount = 0;
                     }
                 }
-                q_next = prec->get(pcount > 0 ? pstart + min(L.rl, pcount - 1) : 0);
+                q_next = prec->get(pcount > 0 ? pfirst : 0);
             }
             // Rows m = 4 (lane / 16) + i are (re, im) of terms kg + 2 (lane / 16) and
             // kg + 2 (lane / 16) + 1; column n16.
@@ -1228,7 +1785,7 @@ k_win_grid(WinJobs jobs) {
             for (int a = 0; a < kWin; ++a)
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
-                    window_store(o, it, J.wg, G, K, a, kg + 2 * (lane >> 4) + h, L.n16, L.inv,
+                    window_store(o, G, K, a, kg + 2 * (lane >> 4) + h, L.n16, L.inv,
                                  make_float2(d[a][2 * h], d[a][2 * h + 1]), J.trash, lane);
         }
         if (next >= nwave) break;
@@ -1271,8 +1828,6 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     WinGeom wg;
     wg.nw = (gp.G + kWin - 1) / kWin;
     wg.cls_log2 = effective_class_log2(gp, wg.nw);
-    wg.coop_min = gp.coop_min != 0 ? gp.coop_min : kCoopMinDefault;
-    wg.coop_cap = gp.coop_cap != 0 ? gp.coop_cap : kCoopCapDefault;
     wg.ncls = 24 >> wg.cls_log2;
     wg.nh = (gp.G + (1 << wg.cls_log2) - 1) >> wg.cls_log2;
     wg.nwin = wg.nw * wg.nw;
@@ -1283,12 +1838,6 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     const size_t max_records = 2 * S;                      // one row class, at most two window columns
     const size_t nbins = nbins_sz;
     const size_t nwt = static_cast<size_t>(wg.nwin_total);
-    // Wavefront items: one per window at most.  Workgroup pieces: at most one per window plus
-    // reads / coop_cap (a window reads each record at most twice).  Partial slots: only windows
-    // with two or more pieces have them, at most 2 reads / coop_cap.
-    const size_t max_reads = 2 * max_records;
-    const size_t max_items = 2 * nwt + max_reads / wg.coop_cap + 1;
-    const size_t max_slots = 2 * max_reads / wg.coop_cap + 1;
     unsigned blocks;
     if (in.from_snapshot) blocks = static_cast<unsigned>((in.num_rows + kBinRows - 1) / kBinRows);
     else blocks = static_cast<unsigned>((S + kBinThreads * kBinPerThread - 1) / (kBinThreads * kBinPerThread));
@@ -1320,19 +1869,47 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
         ctx->ws.get(Workspace::kBinCursor, (nbins + 8 + nwt + (wg.use_lds ? kBinSegs * nbins : 0)) * sizeof(uint32_t)));
     uint32_t* multi = cursor + nbins + 8;                  // windows with several pieces
     uint32_t* segsum = multi + nwt;                        // [kBinSegs][nbins]
-    const size_t ncounts = (2 * kItemClasses + 1) * nwt;
+    const size_t ncounts = (3 * kItemClasses + 2) * nwt;
     uint32_t* sums = static_cast<uint32_t*>(
         ctx->ws.get(Workspace::kScanSums, scan_blocks(std::max(nbins, ncounts)) * sizeof(uint32_t)));
     uint32_t* icount = static_cast<uint32_t*>(ctx->ws.get(Workspace::kItemCounts, (ncounts + 8) * sizeof(uint32_t)));
     uint32_t* ioff = static_cast<uint32_t*>(ctx->ws.get(Workspace::kItemOffsets, (ncounts + 8) * sizeof(uint32_t)));
-    const size_t piece_floats2 = static_cast<size_t>(gp.K) * kWin * kWin;
+    uint32_t* totals = counts + nbins + 2;
+    WRecords rec;
+    rec.r = static_cast<uint4*>(ctx->ws.get(Workspace::kRecPos, max_records * sizeof(uint4)));
+
+    // Work shape: a half is dense above coop_min records, in pieces of at most coop_cap.  Fewer samples
+    // take smaller pieces, so that they still spread over the chip (a workgroup contracts a piece of
+    // 16384 records in about 100 us), and a lower threshold, so that no wavefront's item is a long
+    // chain.  Measured per call (coop_min / coop_cap): 8.4 M samples at 1024^2 869 us with
+    // 1024 / 16384, 882 with 1024 / 8192, 986 with 512 / 4096; 5.2 M at 512^2 700 with 1024 / 8192,
+    // 745 with 512 / 4096; 2.1 M at 1024^2 642 with 512 / 4096, 677 with 1024 / 8192; 1.4 M at 1000^2 635 with
+    // 512 / 4096, 661 with 256 / 2048, 672 with 1024 / 8192; 32 k at 128^2 210 with 256 / 2048, 232 with
+    // 1024 / 8192.
+    auto clamped = [](size_t v, size_t lo, size_t hi) { return static_cast<uint32_t>(std::min(std::max(v, lo), hi)); };
+    wg.coop_min = gp.coop_min != 0 ? gp.coop_min : clamped(S / 4096, 256, kCoopMinDefault);
+    wg.coop_cap = gp.coop_cap != 0 ? gp.coop_cap : clamped(S / 512, 2048, kCoopCapDefault);
+    // Wavefront items: one per window at most.  Pieces (and partial slots): at most one per dense
+    // half, of which there are at most records / (coop_min + 1), plus records / coop_cap.  The slots
+    // of the worst case are bounded to kMaxPartialBytes (in the fixed scratch range to what is left but
+    // for the items and the FFT's twiddles) by a coarser shape.
+    const size_t slot_bytes = static_cast<size_t>(gp.K) * kDenseCells * sizeof(float2) + sizeof(WItem);
+    const size_t reserve = nwt * (sizeof(WItem) + sizeof(WReduce)) + static_cast<size_t>(gp.G) * sizeof(float2) + (64u << 10);
+    const size_t left = ctx->ws.arena_left();
+    const size_t partial_bytes = std::min(kMaxPartialBytes, left > reserve ? left - reserve : 0);
+    auto slots = [&]() { return max_records / wg.coop_cap + std::min(2 * nwt, max_records / (wg.coop_min + 1)) + 1; };
+    while (slots() * slot_bytes > partial_bytes && (wg.coop_cap < max_records || wg.coop_min < max_records)) {
+        if (max_records / wg.coop_cap >= slots() / 2) wg.coop_cap *= 2;
+        else wg.coop_min *= 2;
+    }
+    const size_t max_slots = slots();
+    const size_t max_items = nwt + max_slots;
+    WItem* items = static_cast<WItem*>(ctx->ws.get(Workspace::kItems, max_items * sizeof(WItem) + nwt * sizeof(WReduce)));
+    WReduce* red = reinterpret_cast<WReduce*>(items + max_items);
+    const size_t piece_floats2 = static_cast<size_t>(gp.K) * kDenseCells;
     float2* partial = static_cast<float2*>(
         ctx->ws.get(Workspace::kWinPartial, (max_slots * piece_floats2 + 64) * sizeof(float2)));
     float2* trash = partial + max_slots * piece_floats2;
-    uint32_t* totals = counts + nbins + 2;
-    WItem* items = static_cast<WItem*>(ctx->ws.get(Workspace::kItems, max_items * sizeof(WItem)));
-    WRecords rec;
-    rec.r = static_cast<uint4*>(ctx->ws.get(Workspace::kRecPos, max_records * sizeof(uint4)));
 
     launch_fill(ctx, reinterpret_cast<float*>(counts), nbins + 12, 0.0f);
     // 16-bit LDS histograms (two bins per word) when there are also more blocks than CUs, so that
@@ -1379,7 +1956,7 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     SVDI_LAUNCH_CHECK();
     launch_exclusive_scan(ctx, icount, ioff, nullptr, sums, ncounts);
     k_win_item_write<<<static_cast<unsigned>((max_items + 255) / 256), 256, 0, ctx->stream>>>(
-        boff, ioff, wg, items, static_cast<uint32_t>(max_items), totals);
+        boff, ioff, multi, wg, items, static_cast<uint32_t>(max_items), red, totals);
     SVDI_LAUNCH_CHECK();
     const uint32_t limit = static_cast<uint32_t>(max_records);
     if (in.from_snapshot) {
@@ -1402,9 +1979,7 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     job.planes = planes;
     job.partial = partial;
     job.trash = trash;
-    job.boff = boff;
-    job.ioff = ioff;
-    job.multi = multi;
+    job.reduce = red;
     job.max_slots = static_cast<uint32_t>(max_slots);
     job.K = gp.K;
     job.G = gp.G;
@@ -1416,6 +1991,7 @@ void contract_windows(svdi_context* ctx, const WindowJob* jobs, int count) {
     if (count < 1 || count > kMaxJobs) throw std::logic_error("window job count out of range");
     WinJobs wj = {};
     wj.count = count;
+    int most_terms = 0;
     for (int j = 0; j < count; ++j) {
         if (jobs[j].prec != jobs[0].prec) throw std::logic_error("window jobs of one launch differ in precision");
         WinJob& d = wj.job[j];
@@ -1428,12 +2004,22 @@ void contract_windows(svdi_context* ctx, const WindowJob* jobs, int count) {
         std::memcpy(&d.wg, jobs[j].geom, sizeof d.wg);
         d.K = jobs[j].K;
         d.G = jobs[j].G;
+        most_terms = std::max(most_terms, d.K);
     }
     const size_t tok = stage_begin(ctx, 5);
     const unsigned grid = static_cast<unsigned>(std::max(1, ctx->cu_count - ctx->grid_reserve));
     auto launch = [&](auto prec) {
         constexpr int P = decltype(prec)::value;
         using T = WinTraits<P>;
+        auto dense = [&](auto mb) {
+            constexpr int MB = decltype(mb)::value;
+            using D = DenseTraits<P, MB>;
+            allow_dynamic_lds(reinterpret_cast<const void*>(&k_win_dense<P, MB>), D::kLds);
+            k_win_dense<P, MB><<<grid, D::kWaves * 64, D::kLds, ctx->stream>>>(wj);
+            SVDI_LAUNCH_CHECK();
+        };
+        if (most_terms <= 8) dense(std::integral_constant<int, 1>());
+        else dense(std::integral_constant<int, 2>());
         constexpr size_t lds = sizeof(float) * T::kStageFloats * T::kWaves;
         allow_dynamic_lds(reinterpret_cast<const void*>(&k_win_grid<P>), lds);
         k_win_grid<P><<<grid, T::kWaves * 64, lds, ctx->stream>>>(wj);
@@ -1450,8 +2036,8 @@ void contract_windows(svdi_context* ctx, const WindowJob* jobs, int count) {
 void reduce_windows(svdi_context* ctx, const WindowJob& job) {
     WinGeom wg;
     std::memcpy(&wg, job.geom, sizeof wg);
-    k_win_reduce<<<2048, kReduceGroups * 256, 0, ctx->stream>>>(job.boff, job.ioff, job.multi, job.totals, wg, job.G,
-                                                                job.K, job.max_slots, job.partial, job.planes);
+    k_win_reduce<<<4096, 256, 0, ctx->stream>>>(static_cast<const WReduce*>(job.reduce), job.totals, wg, job.G, job.K,
+                                               job.max_slots, job.partial, job.planes);
     SVDI_LAUNCH_CHECK();
 }
 
