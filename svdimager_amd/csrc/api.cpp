@@ -307,7 +307,7 @@ Enqueued image_prepare(svdi_context* ctx, const SampleInput& in, const svdi_opti
     }
     const size_t P = hp.batch_slabs * static_cast<size_t>(K);
     e.planes = static_cast<float2*>(ctx->ws.get(Workspace::kPlanes, P * G * G * sizeof(float2)));
-    e.rowfft = static_cast<float2*>(ctx->ws.get(Workspace::kRowFft, P * G * hp.cols * sizeof(float2)));
+    e.rowfft = static_cast<float2*>(ctx->ws.get(Workspace::kRowFft, P * fft_row_elems(G, hp.cols) * sizeof(float2)));
     e.colfft = static_cast<float2*>(ctx->ws.get(Workspace::kColFft, P * hp.rows * hp.cols * sizeof(float2)));
     float* conv = static_cast<float*>(ctx->ws.get(Workspace::kConv, (N / 2 + 1) * sizeof(float)));
     e.conv = conv;
@@ -359,8 +359,7 @@ Enqueued image_prepare(svdi_context* ctx, const SampleInput& in, const svdi_opti
     ip.slab_half = hp.dev.slab_half_range;
     ip.r3_centre = hp.dev.r3_centre;
     ip.inv_num_samples = 1.0f / static_cast<float>(in.num_samples);
-    ip.rows = static_cast<int>(hp.rows);
-    ip.cols = static_cast<int>(hp.cols);
+    ip.win = fft_window(G, hp.row_lo, hp.rows, hp.cols);
     ip.row_lo = static_cast<int>(hp.row_lo);
     ip.col_lo = static_cast<int>(hp.col_lo);
     ip.signed_out = o.output == SVDI_OUTPUT_SIGNED;
@@ -398,7 +397,8 @@ void image_post(svdi_context* ctx, CallState& cs, Enqueued& e, size_t start, siz
     const HostPlan& hp = cs.hp;
     const size_t Pb = nb * static_cast<size_t>(hp.num_terms);
     size_t tok = stage_begin(ctx, 3);
-    launch_fft2_inverse(ctx, e.planes, Pb, hp.grid_size, hp.row_lo, hp.rows, hp.col_lo, hp.cols, e.rowfft, e.colfft);
+    launch_fft2_inverse(ctx, e.planes, Pb, hp.grid_size, hp.row_lo, hp.rows, hp.col_lo, hp.cols, e.rowfft, e.colfft,
+                        e.ip.win);
     stage_end(ctx, tok);
     e.ip.P = static_cast<int>(Pb);
     e.ip.slab_start = static_cast<int>(start);
@@ -1428,9 +1428,12 @@ int svdi_fft2_inverse(svdi_context* ctx, const void* planes, size_t num_planes, 
         DeviceGuard g(ctx->device);
         begin_call(ctx);
         float2* rowfft = static_cast<float2*>(
-            ctx->ws.get(Workspace::kRowFft, num_planes * grid_size * cols * sizeof(float2)));
+            ctx->ws.get(Workspace::kRowFft, num_planes * fft_row_elems(grid_size, cols) * sizeof(float2)));
+        FftWindow win;                                     // row-major
+        win.rows = static_cast<int>(rows);
+        win.cols = static_cast<int>(cols);
         launch_fft2_inverse(ctx, static_cast<const float2*>(planes), num_planes, grid_size, row_lo, rows, col_lo,
-                            cols, rowfft, static_cast<float2*>(out));
+                            cols, rowfft, static_cast<float2*>(out), win);
         SVDI_HIP(hipStreamSynchronize(ctx->stream));
     });
 }

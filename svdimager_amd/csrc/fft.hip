@@ -2,7 +2,8 @@
 // cufftPlanMany + cufftExecC2C(CUFFT_INVERSE) (SVDIntegratedImager.cu:1658-1676, 1713).
 //
 // Two LDS-staged passes of a mixed-radix Stockham FFT (radix 8/4/2/3/5 kernels plus a direct
-// butterfly for other primes up to 13).  G = ceil(3N/2) is 3 * 2^k for the usual image sizes.
+// butterfly for other primes up to 13).  G = ceil(3N/2) is 3 * 2^k for the usual image sizes; 1536,
+// 3072 and 6144 have passes of their own around a 1536-point transform held by one wavefront.
 // Only the central N x N of each transformed G x G plane is read by the image pass, so the row
 // pass keeps the central `cols` output columns and the column pass transforms just those
 // columns and keeps the central `rows` outputs.
@@ -345,19 +346,31 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// kTwStride: the table holds e^{2 pi i t / (1536 kTwStride)} (W_1536^m = tw[kTwStride m]).
+// Twiddles of the 1536-point wavefront transform in the order in which lanes ask for them, so that
+// each request reads 64 consecutive entries (from the one table of W_1536^m the lanes of a request
+// lie up to 64 lines apart, which bound the passes): W^{l k1} at [k1][l], W_64^{b c} at [c][q], q = 24 b +
+// k1 (the place of (k1, b) below), and W_24^{v s} at [8 v + s].
+struct Fft1536Tables {
+    const float2 *lane, *cross, *w24;
+};
+constexpr int kTabLane = 24 * 64, kTabCross = 8 * 192, kTab24 = 24;
+constexpr int kTabAll = kTabLane + kTabCross + kTab24;
+__device__ __forceinline__ Fft1536Tables fft1536_tables(const float2* __restrict__ t) {
+    return {t, t + kTabLane, t + kTabLane + kTabCross};
+}
+
 // fft1536_wave_regs takes the lane's inputs already in registers: y[v][u] = x[64 (3u + v) + l].
-template <int kTwStride = 1, class Store>
-__device__ __forceinline__ void fft1536_wave_regs(float2 (&y)[3][8], float2* tile, const float2* __restrict__ tw,
+template <class Store>
+__device__ __forceinline__ void fft1536_wave_regs(float2 (&y)[3][8], float2* tile, const Fft1536Tables& tw,
                                                   int lane, Store&& store) {
     // 24-point DFT over n1 = 3u + v, k1 = s + 8t: 8-point DFTs over u, times W_24^{v s}, then
-    // 3-point DFTs over v.  W_24^m = tw[64 m].
+    // 3-point DFTs over v.
 #pragma unroll
     for (int v = 0; v < 3; ++v) dft8(y[v]);
 #pragma unroll
     for (int v = 1; v < 3; ++v)
 #pragma unroll
-        for (int s8 = 1; s8 < 8; ++s8) y[v][s8] = cmul(y[v][s8], tw[kTwStride * 64 * v * s8]);
+        for (int s8 = 1; s8 < 8; ++s8) y[v][s8] = cmul(y[v][s8], tw.w24[8 * v + s8]);
 #pragma unroll
     for (int s8 = 0; s8 < 8; ++s8) {
         float2 t3[3] = {y[0][s8], y[1][s8], y[2][s8]};
@@ -366,7 +379,7 @@ __device__ __forceinline__ void fft1536_wave_regs(float2 (&y)[3][8], float2* til
         for (int t = 0; t < 3; ++t) {
             const int k1 = s8 + 8 * t;
             // times W^{l k1} (l k1 < 1536), into the tile at [k1][l]
-            tile[k1 * kTileStride + lane] = k1 == 0 ? t3[t] : cmul(t3[t], tw[kTwStride * lane * k1]);
+            tile[k1 * kTileStride + lane] = k1 == 0 ? t3[t] : cmul(t3[t], tw.lane[k1 * 64 + lane]);
         }
     }
     wave_lds_fence();
@@ -384,7 +397,7 @@ __device__ __forceinline__ void fft1536_wave_regs(float2 (&y)[3][8], float2* til
         const int q = lane + 64 * j, k1 = q % 24, b = q / 24;
         dft8(w[j]);
 #pragma unroll
-        for (int c = 1; c < 8; ++c) w[j][c] = cmul(w[j][c], tw[kTwStride * 24 * b * c]);
+        for (int c = 1; c < 8; ++c) w[j][c] = cmul(w[j][c], tw.cross[c * 192 + q]);
 #pragma unroll
         for (int c = 0; c < 8; ++c) tile[k1 * kTileStride + 8 * b + c] = w[j][c];
     }
@@ -408,8 +421,8 @@ __device__ __forceinline__ void fft1536_wave_regs(float2 (&y)[3][8], float2* til
     }
 }
 
-template <int kTwStride = 1, class Load, class Store>
-__device__ __forceinline__ void fft1536_wave(float2* tile, const float2* __restrict__ tw, int lane,
+template <class Load, class Store>
+__device__ __forceinline__ void fft1536_wave(float2* tile, const Fft1536Tables& tw, int lane,
                                              Load&& load, Store&& store) {
     float2 y[3][8];                                // y[v][u] = x[64 (3u + v) + l]
 #pragma unroll
@@ -417,26 +430,7 @@ __device__ __forceinline__ void fft1536_wave(float2* tile, const float2* __restr
 #pragma unroll
         for (int v = 0; v < 3; ++v) y[v][u] = load(64 * (3 * u + v) + lane);
     wave_lds_fence();                              // the tile may be where the loads came from
-    fft1536_wave_regs<kTwStride>(y, tile, tw, lane, store);
-}
-
-// Row pass for G = 1536: one wavefront per row of the P x G rows; loads stride 64 per lane and
-// stores of consecutive k across lanes are coalesced; only the columns col_lo .. col_lo + cols - 1
-// are stored.
-__global__ void __launch_bounds__(64 * kFftWaves)
-k_fft_rows_1536(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tw,
-                int total_rows, int col_lo, int cols) {
-    constexpr int G = 1536;
-    __shared__ float2 tile_all[kFftWaves][24 * kTileStride];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int row = blockIdx.x * kFftWaves + wave;
-    if (row >= total_rows) return;                 // whole wavefronts; no workgroup barrier below
-    const float2* src = in + static_cast<size_t>(row) * G;
-    float2* dst = out + static_cast<size_t>(row) * cols - col_lo;
-    fft1536_wave(tile_all[wave], tw, lane, [&](int n) { return src[n]; },
-                 [&](int k, float2 v) {
-                     if (k >= col_lo && k < col_lo + cols) dst[k] = v;
-                 });
+    fft1536_wave_regs(y, tile, tw, lane, store);
 }
 
 // Workgroups are dealt to the 8 XCDs round-robin in launch order, each XCD with its own L2.
@@ -451,89 +445,145 @@ __device__ __forceinline__ int xcd_local_tile(int linear, int total) {
     return x * q + min(x, r) + local;
 }
 
-// Column pass of 1536-point transforms: one workgroup per (half-plane, strip of kColStrip
-// columns).  The strip is read into LDS with the columns side by side (row segments of
-// kColStrip columns), each wavefront transforms one column in place (the column's LDS region is
-// also its exchange tile), and the output rows in the window row_lo .. row_lo + rows - 1 are
-// written back as row segments.  kSplit = 1: G = 1536, the half-planes are the planes and
-// transform index k is output row k.  kSplit = 2: G = 3072 after the row pass's radix-2 step;
-// half-plane q holds a (q even) or b (q odd) of plane q / 2, and k is output row 2 k + q % 2
-// (twiddles W_1536^m = tw[2 m]).
-constexpr int kColStrip = 4;
-constexpr int kColLen = 24 * kTileStride;          // float2 per column region (>= 1536)
+// G = 1536 s, s = 1, 2 or 4: the column direction's radix-s step (decimation in frequency) is done
+// in the row pass, on the row-transformed rows x_n, x_{n + 1536}, ...: sub-plane q holds
+// y_q[n] = W^{n q} sum_m W_s^{m q} x_{n + 1536 m}, n < 1536, W = e^{2 pi i / G}, and its 1536-point
+// column transform gives the output rows s k + q.  Between the passes element (n, c) of sub-plane i lies
+// at i sub_stride + n row_stride + (c / 8) block_stride + c % 8.  For s > 1 the columns are in blocks,
+// [sub-plane][block][n][8], which the column pass reads as contiguous runs (48 planes of 3072^2: rows 1.49
+// + columns 0.87 ms, against 1.34 + 1.17 row-major); for s = 1 the planes are row-major (8 planes of
+// 1536^2: 54 + 51 us, against 62 + 47 in blocks).
+constexpr int kBlockCols = 8;                      // 64-byte row segments
+constexpr int kSub = 1536;
+struct MidLayout {
+    size_t sub_stride;
+    int row_stride, block_stride;
+    __device__ __forceinline__ size_t row(size_t sub, int n) const { return sub * sub_stride + static_cast<size_t>(n) * row_stride; }
+    __device__ __forceinline__ size_t col(int kc) const {
+        return static_cast<size_t>(kc / kBlockCols) * block_stride + kc % kBlockCols;
+    }
+};
 
-template <int kSplit>
-__global__ void __launch_bounds__(64 * kColStrip)
-k_fft_cols_1536(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tw,
-                int cols, int row_lo, int rows, int strips) {
-    constexpr int H = 1536;
-    __shared__ float2 strip[kColStrip * kColLen];
-    const int tile = xcd_local_tile(blockIdx.x, gridDim.x);
-    const int q = tile / strips;
-    const int plane = q / kSplit, parity = q - plane * kSplit;
-    const int c0 = (tile - q * strips) * kColStrip;
-    const int nc = min(kColStrip, cols - c0);
-    const float2* src = in + static_cast<size_t>(q) * H * cols + c0;
-    {
-        // Element (r, c) of the strip: thread t = (r mod 64) kColStrip + c loads rows r0 + 64 j,
-        // all 24 loads issued before the first LDS store.
-        constexpr int kLoads = H / 64;
-        const int c = threadIdx.x % kColStrip, r0 = threadIdx.x / kColStrip;
-        if (c < nc) {
-            float2 v[kLoads];
-#pragma unroll
-            for (int j = 0; j < kLoads; ++j) v[j] = src[static_cast<size_t>(r0 + 64 * j) * cols + c];
-#pragma unroll
-            for (int j = 0; j < kLoads; ++j) strip[c * kColLen + r0 + 64 * j] = v[j];
-        }
-    }
-    __syncthreads();
+// Row pass for G = 1536: one wavefront per row of the P x G rows; loads stride 64 per lane are
+// coalesced; only the columns col_lo .. col_lo + cols - 1 are stored.
+__global__ void __launch_bounds__(64 * kFftWaves)
+k_fft_rows_1536(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tab,
+                int total_rows, int col_lo, int cols, MidLayout mid) {
+    constexpr int G = 1536;
+    __shared__ float2 tile_all[kFftWaves][24 * kTileStride];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (wave < nc) {
-        float2* col = strip + wave * kColLen;
-        fft1536_wave<kSplit>(col, tw, lane, [&](int n) { return col[n]; }, [&](int k, float2 v) { col[k] = v; });
-    }
-    __syncthreads();
-    // Transform outputs k_lo .. k_lo + nk - 1 land in the window (output row kSplit k + parity).
-    const int k_lo = max(0, (row_lo - parity + kSplit - 1) / kSplit);
-    const int nk = min(H, (row_lo + rows - parity + kSplit - 1) / kSplit) - k_lo;
-    float2* dst = out + static_cast<size_t>(plane) * rows * cols + c0;
+    const int row = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * kFftWaves + wave));
+    if (row >= total_rows) return;                 // whole wavefronts; no workgroup barrier below
+    const float2* src = in + static_cast<size_t>(row) * G;
+    const int plane = row / G, n = row - plane * G;
+    float2* dst = out + mid.row(plane, n);
+    fft1536_wave(tile_all[wave], fft1536_tables(tab), lane, [&](int m) { return src[m]; },
+                 [&](int k, float2 v) {
+                     const int kc = k - col_lo;
+                     if (kc >= 0 && kc < cols) dst[mid.col(kc)] = v;
+                 });
+}
+
+// Barrier for data exchanged through LDS: global loads and stores stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Column pass of the 1536-point transforms of column blocks (s sub-planes per plane), bound by memory:
+// persistent workgroups, one per CU, a wavefront per column of the block.  The block is read into LDS, each
+// wavefront transforms one column in place (the column's LDS region is also its exchange tile), and
+// the output rows s k + q in the window row_lo .. row_lo + rows - 1 are written.  The next block's
+// loads are issued before the transforms, which take their twiddles from LDS so that they wait
+// for no global load, and stay in flight across the barriers: with one workgroup per CU the memory
+// pipe is otherwise idle while it computes (with a workgroup per block and the twiddles gathered from
+// global memory: 8 planes of 1536^2 56 us, now 52; 48 of 3072^2 1.48 ms, 0.89; 8 of 6144^2, which then
+// had half transforms by pairs of wavefronts, 1.86 ms, 0.59).  Output element (row r, column c) of plane p goes to
+// p plane_stride + (c / 8) block_stride + r row_stride + c % 8 in a row-major plane (split_rows = 0), or,
+// with row_stride = 8 and split_rows = rows / s, to row q split_rows + k of its column block
+// (FftWindow).
+constexpr int kColLen = 24 * kTileStride;          // float2 per column region (>= 1536)
+constexpr size_t kColsLds = sizeof(float2) * (kBlockCols * kColLen + kTabLane + kTabCross);
+struct ColsOut {
+    size_t plane_stride, block_stride;
+    int row_stride, split_rows;
+};
+
+__global__ void __launch_bounds__(64 * kBlockCols)
+k_fft_cols_1536(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tab,
+                int s, int tiles, int nblk, int cols, int row_lo, int rows, MidLayout mid, ColsOut o) {
+    constexpr int H = kSub, kThreadsC = 64 * kBlockCols, kLoads = H / 64;
+    extern __shared__ float2 cols_lds[];
+    float2* strip = cols_lds;
+    float2* tab_lds = cols_lds + kBlockCols * kColLen;
+    for (int t = threadIdx.x; t < kTabLane + kTabCross; t += kThreadsC) tab_lds[t] = tab[t];
+    const Fft1536Tables tw = {tab_lds, tab_lds + kTabLane, tab + kTabLane + kTabCross};
+    // Tiles (plane, q, block) are dealt so that an XCD's workgroups work on neighbouring blocks.
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int c = threadIdx.x % kBlockCols, r0 = threadIdx.x / kBlockCols;
+    // Element (r, c) of a block: thread t = (r mod 64) kBlockCols + c loads rows r0 + 64 j.
+    float2 v[kLoads];
+    auto load = [&](int tile) {
+        const int sub = tile / nblk;
+        const float2* src = in + mid.row(sub, r0) + static_cast<size_t>(tile - sub * nblk) * mid.block_stride + c;
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) v[j] = src[static_cast<size_t>(64 * j) * mid.row_stride];
+    };
+    int tile = xcd_local_tile(blockIdx.x, gridDim.x);
+    if (tile < tiles) load(tile);
+    for (; tile < tiles; tile += gridDim.x) {
+        lds_barrier();                             // the block before this one has been written out
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) strip[c * kColLen + r0 + 64 * j] = v[j];
+        lds_barrier();
+        if (tile + static_cast<int>(gridDim.x) < tiles) load(tile + gridDim.x);
+        {
+            float2* col = strip + wave * kColLen;
+            fft1536_wave(col, tw, lane, [&](int n) { return col[n]; }, [&](int k, float2 x) { col[k] = x; });
+        }
+        lds_barrier();
+        // Transform outputs k_lo .. k_lo + nk - 1 land in the window.
+        const int sub = tile / nblk, blk = tile - sub * nblk;
+        const int plane = sub / s, q = sub - plane * s;
+        const int k_lo = max(0, (row_lo - q + s - 1) / s);
+        const int nk = min(H, (row_lo + rows - q + s - 1) / s) - k_lo;
+        if (blk * kBlockCols + c < cols) {
+            float2* dst = out + plane * o.plane_stride + blk * o.block_stride + c;
 #pragma unroll 8
-    for (int t = threadIdx.x; t < nk * kColStrip; t += 64 * kColStrip) {
-        const int k = k_lo + t / kColStrip, c = t % kColStrip;
-        const int r = kSplit * k + parity - row_lo;
-        if (c < nc && r >= 0 && r < rows) dst[static_cast<size_t>(r) * cols + c] = strip[c * kColLen + k];
+            for (int k = r0; k < nk; k += kThreadsC / kBlockCols) {
+                const int r = o.split_rows != 0 ? q * o.split_rows + k : s * (k_lo + k) + q - row_lo;
+                dst[static_cast<size_t>(r) * o.row_stride] = strip[c * kColLen + k_lo + k];
+            }
+        }
     }
 }
 
-// G = 3072 = 2 x 1536, a radix-2 step in each direction around 1536-point transforms.
-// Along a row (decimation in time): E and O are the transforms of the even and odd samples
-// (twiddles W_1536^m = tw[2 m] of the 3072-point table), X[k] = E[k] + W^k O[k] and
-// X[k + 1536] = E[k] - W^k O[k], W = e^{2 pi i / 3072}.  Along a column (decimation in
-// frequency, done in the row pass on the row-transformed rows x_n): a_n = x_n + x_{n + 1536} and
-// b_n = (x_n - x_{n + 1536}) W^n for n < 1536; the 1536-point column transforms of a and b give
-// the even and odd output rows, X[2 k] = A[k] and X[2 k + 1] = B[k].
-
 // Row pass for G = 3072: one workgroup per (plane, n < 1536) transforms rows n and n + 1536, a
-// pair of wavefronts per row (even samples, odd samples, each into its own LDS tile), combines
-// them and stores a_n as row n and b_n as row 1536 + n of the plane's output (the columns
-// col_lo .. col_lo + cols - 1).
+// pair of wavefronts per row, by decimation in time: E and O are the transforms of the even and odd
+// samples (each into its own LDS tile), X[k] = E[k] + W^k O[k] and X[k + 1536] = E[k] - W^k O[k],
+// W = e^{2 pi i / 3072}.  The column direction's step gives a_n = x_n + x_{n + 1536} and
+// b_n = (x_n - x_{n + 1536}) W^n, stored as row n of the plane's two sub-planes (the columns col_lo ..
+// col_lo + cols - 1).  (Decimation in frequency, whose loads are whole runs, took 1.61 ms for 1.51: its
+// extra LDS exchange costs more than the half-used lines, which the second wavefront finds in L2.)
 __global__ void __launch_bounds__(256)
 k_fft_rows_3072(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tw,
-                int col_lo, int cols) {
+                const float2* __restrict__ tab,
+                int col_lo, int cols, MidLayout mid) {
     constexpr int G = 3072, H = 1536;
     __shared__ float2 tile_all[4][24 * kTileStride];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int plane = blockIdx.x / H, n = blockIdx.x - plane * H;
+    const int tile_id = xcd_local_tile(blockIdx.x, gridDim.x);
+    const int plane = tile_id / H, n = tile_id - plane * H;
     const int which = wave >> 1, half = wave & 1;               // row n or n + 1536; even or odd
     const float2* src = in + (static_cast<size_t>(plane) * G + n + which * H) * G;
     float2* tile = tile_all[wave];
-    fft1536_wave<2>(tile, tw, lane, [&](int m) { return src[2 * m + half]; },
+    fft1536_wave(tile, fft1536_tables(tab), lane, [&](int m) { return src[2 * m + half]; },
                     [&](int k, float2 v) { tile[k] = v; });
     __syncthreads();
     const float2 wn = tw[n];
-    float2* dst_a = out + (static_cast<size_t>(plane) * G + n) * cols - col_lo;
-    float2* dst_b = dst_a + static_cast<size_t>(H) * cols;
+    float2* dst_a = out + mid.row(2 * plane, n);
+    float2* dst_b = out + mid.row(2 * plane + 1, n);
     for (int k = threadIdx.x; k < H; k += 256) {
         const float2 wk = tw[k];
         const float2 en = tile_all[0][k], on = cmul(tile_all[1][k], wk);
@@ -541,120 +591,97 @@ k_fft_rows_3072(const float2* __restrict__ in, float2* __restrict__ out, const f
         const float2 xn0 = cadd(en, on), xn1 = csub(en, on);      // row n at columns k, k + 1536
         const float2 xm0 = cadd(em, om), xm1 = csub(em, om);      // row n + 1536
         if (k >= col_lo && k < col_lo + cols) {
-            dst_a[k] = cadd(xn0, xm0);
-            dst_b[k] = cmul(csub(xn0, xm0), wn);
+            const size_t i = mid.col(k - col_lo);
+            dst_a[i] = cadd(xn0, xm0);
+            dst_b[i] = cmul(csub(xn0, xm0), wn);
         }
         const int k1 = k + H;
         if (k1 >= col_lo && k1 < col_lo + cols) {
-            dst_a[k1] = cadd(xn1, xm1);
-            dst_b[k1] = cmul(csub(xn1, xm1), wn);
+            const size_t i = mid.col(k1 - col_lo);
+            dst_a[i] = cadd(xn1, xm1);
+            dst_b[i] = cmul(csub(xn1, xm1), wn);
         }
     }
 }
 
-// Row pass for G = 6144 = 4 x 1536: one workgroup per row, wavefront j transforming the samples
-// x[4 m + j] (m < 1536, the 1536-point wavefront transform with a stride-4 twiddle table) into
-// F_j, then a radix-4 step: with W = e^{2 pi i / 6144} and k = k0 + 1536 q (k0 < 1536, q < 4),
-// X[k] = sum_j W^{j k} F_j[k0] = sum_j i^{j q} (W^{j k0} F_j[k0]).  Only the columns
-// col_lo .. col_lo + cols - 1 are stored; the column pass is the general one.
-__global__ void __launch_bounds__(256)
+// Row pass for G = 6144 = 4 x 1536: one workgroup per (plane, n < 1536) transforms the four rows
+// n + 1536 m, two at a time with four wavefronts each: wavefront j of a row transforms the samples
+// x[4 i + j] (i < 1536, the 1536-point wavefront transform) into F_j,
+// then a radix-4 step along the row: with W = e^{2 pi i / 6144} and k = k0 + 1536 p (k0 < 1536,
+// p < 4), X[k] = sum_j W^{j k} F_j[k0] = sum_j i^{j p} (W^{j k0} F_j[k0]).  Every thread keeps the
+// sums of the column direction's radix-4 step for its twelve columns k = threadIdx.x + 512 i in
+// registers over the four rows and stores them as row n of the plane's four sub-planes (the columns
+// col_lo .. col_lo + cols - 1).  A row pass that took two rows had left half of the column step to the
+// column pass (8 planes: 1.20 + 1.86 ms for both passes, now 1.45 + 0.59).
+constexpr int kRows6Threads = 512;
+constexpr size_t kRows6Lds = sizeof(float2) * 8 * 24 * kTileStride;
+__global__ void __launch_bounds__(kRows6Threads)
 k_fft_rows_6144(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tw,
-                int col_lo, int cols) {
-    constexpr int G = 6144, H = 1536;
-    __shared__ float2 tile_all[4][24 * kTileStride];
+                const float2* __restrict__ tab,
+                int col_lo, int cols, MidLayout mid) {
+    constexpr int G = 6144, H = 1536, kTile = 24 * kTileStride, kPer = H / kRows6Threads;
+    extern __shared__ float2 rows6_lds[];          // [row of the pair][residue j][kTile]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const size_t row = blockIdx.x;
-    const float2* src = in + row * G;
-    float2* tile = tile_all[wave];
-    fft1536_wave<4>(tile, tw, lane, [&](int m) { return src[4 * m + wave]; },
-                    [&](int k, float2 v) { tile[k] = v; });
-    __syncthreads();
-    float2* dst = out + row * static_cast<size_t>(cols) - col_lo;
-    for (int k0 = threadIdx.x; k0 < H; k0 += 256) {
-        const float2 g0 = tile_all[0][k0];
-        const float2 g1 = cmul(tile_all[1][k0], tw[k0]);
-        const float2 g2 = cmul(tile_all[2][k0], tw[2 * k0]);
-        const float2 g3 = cmul(tile_all[3][k0], tw[3 * k0]);
-        const float2 s02 = cadd(g0, g2), d02 = csub(g0, g2);
-        const float2 s13 = cadd(g1, g3), d13 = csub(g1, g3);
-        const float2 id13 = make_float2(-d13.y, d13.x);          // i (g1 - g3)
-        const float2 x[4] = {cadd(s02, s13), cadd(d02, id13), csub(s02, s13), csub(d02, id13)};
+    const int tile_id = xcd_local_tile(blockIdx.x, gridDim.x);
+    const int plane = tile_id / H, n = tile_id - plane * H;
+    float2 y[4][kPer][4];                          // [q][i][p]
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int k = k0 + H * q;
-            if (k >= col_lo && k < col_lo + cols) dst[k] = x[q];
+    for (int half = 0; half < 2; ++half) {         // rows m = half and half + 2
+        {
+            const float2* src = in + (static_cast<size_t>(plane) * G + n + (half + 2 * (wave >> 2)) * H) * G;
+            float2* tile = rows6_lds + wave * kTile;
+            fft1536_wave(tile, fft1536_tables(tab), lane, [&](int i) { return src[4 * i + (wave & 3)]; },
+                            [&](int k, float2 v) { tile[k] = v; });
         }
-    }
-}
-
-// Column pass for G = 6144 = 4 x 1536: decimation in frequency along the column, then four
-// 1536-point transforms.  With W = e^{2 pi i / 6144} and n < 1536,
-//   y_q[n] = W^{n q} sum_m i^{m q} x[n + 1536 m],   X[4 k + q] = sum_n y_q[n] W_1536^{n k}.
-// One workgroup per (plane, strip of kColStrip6 columns): the strip is read into LDS (column c's
-// rows 1536 m .. 1536 m + 1535 in its region m), wavefront (c, q) forms its 24 values of y_q in
-// registers from the four regions, and after a workgroup barrier transforms them in place in
-// region q (the region doubles as the exchange tile); the output rows of the window are written
-// back as row segments of the strip.
-constexpr int kColStrip6 = 3;
-constexpr int kCols6Threads = 64 * 4 * kColStrip6;
-constexpr size_t kCols6Lds = sizeof(float2) * kColStrip6 * 4 * kColLen;
-
-__global__ void __launch_bounds__(kCols6Threads)
-k_fft_cols_6144(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tw,
-                int cols, int row_lo, int rows, int strips) {
-    constexpr int G = 6144, H = 1536;
-    constexpr int kRowsPerPass = kCols6Threads / kColStrip6;      // 256
-    constexpr int kPasses = G / kRowsPerPass;                      // 24
-    extern __shared__ float2 lds6[];                               // [column][region m][kColLen]
-    const int tile = xcd_local_tile(blockIdx.x, gridDim.x);
-    const int plane = tile / strips;
-    const int c0 = (tile - plane * strips) * kColStrip6;
-    const int nc = min(kColStrip6, cols - c0);
-    {
-        const float2* src = in + static_cast<size_t>(plane) * G * cols + c0;
-        const int c = threadIdx.x % kColStrip6, r0 = threadIdx.x / kColStrip6;
-        if (c < nc) {
-            float2 v[kPasses];
+        __syncthreads();
 #pragma unroll
-            for (int j = 0; j < kPasses; ++j) v[j] = src[static_cast<size_t>(r0 + kRowsPerPass * j) * cols + c];
+        for (int i = 0; i < kPer; ++i) {
+            const int k0 = threadIdx.x + kRows6Threads * i;
+            float2 x[2][4];                        // the pair's rows at k0 + 1536 p
 #pragma unroll
-            for (int j = 0; j < kPasses; ++j) {
-                const int r = r0 + kRowsPerPass * j;
-                lds6[(c * 4 + r / H) * kColLen + r % H] = v[j];
+            for (int r = 0; r < 2; ++r) {
+                const float2* t = rows6_lds + 4 * r * kTile;
+                const float2 g0 = t[k0];
+                const float2 g1 = cmul(t[kTile + k0], tw[k0]);
+                const float2 g2 = cmul(t[2 * kTile + k0], tw[2 * k0]);
+                const float2 g3 = cmul(t[3 * kTile + k0], tw[3 * k0]);
+                const float2 s02 = cadd(g0, g2), d02 = csub(g0, g2);
+                const float2 s13 = cadd(g1, g3), id13 = mul_i(csub(g1, g3));
+                x[r][0] = cadd(s02, s13);
+                x[r][1] = cadd(d02, id13);
+                x[r][2] = csub(s02, s13);
+                x[r][3] = csub(d02, id13);
+            }
+            // y_0 and y_2 take +- (x_1 + x_3), y_1 and y_3 take +- i (x_1 - x_3).
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const float2 sum = cadd(x[0][p], x[1][p]), dif = csub(x[0][p], x[1][p]);
+                if (half == 0) {
+                    y[0][i][p] = sum;
+                    y[1][i][p] = dif;
+                } else {
+                    const float2 s = y[0][i][p], d = y[1][i][p], id = mul_i(dif);
+                    y[0][i][p] = cadd(s, sum);
+                    y[2][i][p] = csub(s, sum);
+                    y[1][i][p] = cadd(d, id);
+                    y[3][i][p] = csub(d, id);
+                }
             }
         }
+        if (half == 0) __syncthreads();
     }
-    __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int c = wave >> 2, q = wave & 3;
-    float2 y[3][8];
-    if (c < nc) {
-        const float2* col = lds6 + c * 4 * kColLen;
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+    for (int q = 0; q < 4; ++q) {
+        float2* dst = out + mid.row(4 * static_cast<size_t>(plane) + q, n);
+        const float2 wq = tw[q * n];
 #pragma unroll
-            for (int v = 0; v < 3; ++v) {
-                const int n = 64 * (3 * u + v) + lane;
-                const float2 x0 = col[n], x1 = col[kColLen + n], x2 = col[2 * kColLen + n], x3 = col[3 * kColLen + n];
-                float2 t;
-                if (q == 0) t = cadd(cadd(x0, x2), cadd(x1, x3));
-                else if (q == 1) t = cadd(csub(x0, x2), mul_i(csub(x1, x3)));
-                else if (q == 2) t = csub(cadd(x0, x2), cadd(x1, x3));
-                else t = csub(csub(x0, x2), mul_i(csub(x1, x3)));
-                y[v][u] = q == 0 ? t : cmul(t, tw[n * q]);
+        for (int i = 0; i < kPer; ++i)
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const int kc = threadIdx.x + kRows6Threads * i + H * p - col_lo;
+                if (kc >= 0 && kc < cols)
+                    dst[mid.col(kc)] = q == 0 ? y[q][i][p] : cmul(y[q][i][p], wq);
             }
-    }
-    __syncthreads();                               // every region read before any is rewritten
-    if (c < nc) {
-        float2* region = lds6 + (c * 4 + q) * kColLen;
-        fft1536_wave_regs<4>(y, region, tw, lane, [&](int k, float2 v) { region[k] = v; });
-    }
-    __syncthreads();
-    float2* dst = out + static_cast<size_t>(plane) * rows * cols + c0;
-    for (int t = threadIdx.x; t < rows * kColStrip6; t += kCols6Threads) {
-        const int r = t / kColStrip6, cc = t - r * kColStrip6;
-        const int gr = row_lo + r;                                 // output row 4 k + q
-        if (cc < nc) dst[static_cast<size_t>(r) * cols + cc] = lds6[(cc * 4 + (gr & 3)) * kColLen + (gr >> 2)];
     }
 }
 
@@ -751,31 +778,94 @@ bool factorize(int n, FftStages& st) {
 
 }  // namespace
 
-// Twiddles e^{2 pi i t / G}, t < G, from FP64 sincospi, rounded to FP32.
-__global__ void k_twiddles(float2* __restrict__ tw, int G) {
+// Twiddles e^{2 pi i t / G}, t < G, from FP64 sincospi, rounded to FP32, and behind them (for G = 1536
+// s) the tables of the 1536-point wavefront transform (Fft1536Tables).
+__global__ void k_twiddles(float2* __restrict__ tw, int G, int total) {
     const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= G) return;
+    if (t >= total) return;
+    double turn = static_cast<double>(t) / static_cast<double>(G);
+    if (t >= G) {
+        const int i = t - G, j = i - kTabLane, m = j - kTabCross;
+        int k;                                     // W_1536^k
+        if (j < 0) k = (i / 64) * (i % 64);
+        else if (m < 0) k = 24 * (j / 192) * (j % 192 / 24);
+        else k = 64 * (m / 8) * (m % 8);
+        turn = static_cast<double>(k) / kSub;
+    }
     double sn, cs;
-    sincospi(2.0 * static_cast<double>(t) / static_cast<double>(G), &sn, &cs);
+    sincospi(2.0 * turn, &sn, &cs);
     tw[t] = make_float2(static_cast<float>(cs), static_cast<float>(sn));
 }
+
+// The split s of G = 1536 s (0: another G).
+static int fft_split(size_t G) { return G == 1536 ? 1 : G == 3072 ? 2 : G == 6144 ? 4 : 0; }
+static size_t twiddle_elems(size_t G) { return G + (fft_split(G) != 0 ? kTabAll : 0); }
 
 // The twiddle table of G in the context's workspace, computed on the stream (no host copy, no
 // synchronisation) when G or the table's address changed since the last call.
 void fft_prepare(svdi_context* ctx, size_t G) {
-    float2* d = static_cast<float2*>(ctx->ws.get(Workspace::kTwiddles, G * sizeof(float2)));
+    const size_t total = twiddle_elems(G);
+    float2* d = static_cast<float2*>(ctx->ws.get(Workspace::kTwiddles, total * sizeof(float2)));
     if (ctx->twiddle_n == G && ctx->twiddle_at == d) return;
-    k_twiddles<<<static_cast<unsigned>((G + 255) / 256), 256, 0, ctx->stream>>>(d, static_cast<int>(G));
+    k_twiddles<<<static_cast<unsigned>((total + 255) / 256), 256, 0, ctx->stream>>>(d, static_cast<int>(G),
+                                                                                 static_cast<int>(total));
     SVDI_LAUNCH_CHECK();
     ctx->twiddle_n = G;
     ctx->twiddle_at = d;
 }
 
+size_t fft_row_elems(size_t G, size_t cols) {
+    return G * (fft_split(G) != 0 ? (cols + kBlockCols - 1) / kBlockCols * kBlockCols : cols);
+}
+
+FftWindow fft_window(size_t G, size_t row_lo, size_t rows, size_t cols) {
+    FftWindow w;
+    w.rows = static_cast<int>(rows);
+    w.cols = static_cast<int>(cols);
+    const size_t s = static_cast<size_t>(fft_split(G));
+    if (s != 0 && cols % kBlockCols == 0 && rows % s == 0 && row_lo % s == 0) w.split = static_cast<int>(s);
+    return w;
+}
+
 void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size_t G,
                          size_t row_lo, size_t rows, size_t col_lo, size_t cols,
-                         float2* row_out, float2* out) {
+                         float2* row_out, float2* out, const FftWindow& win) {
     fft_prepare(ctx, G);
-    const float2* tw = static_cast<const float2*>(ctx->ws.get(Workspace::kTwiddles, G * sizeof(float2)));
+    const float2* tw = static_cast<const float2*>(ctx->ws.get(Workspace::kTwiddles, twiddle_elems(G) * sizeof(float2)));
+    const float2* tab = tw + G;
+    const int split = fft_split(G);
+    if (split != 0) {
+        const int nblk = static_cast<int>((cols + kBlockCols - 1) / kBlockCols);
+        const int clo = static_cast<int>(col_lo), nc = static_cast<int>(cols);
+        MidLayout mid;
+        mid.sub_stride = static_cast<size_t>(kSub) * nblk * kBlockCols;
+        mid.row_stride = split == 1 ? nblk * kBlockCols : kBlockCols;
+        mid.block_stride = split == 1 ? kBlockCols : kSub * kBlockCols;
+        if (split == 4) {
+            allow_dynamic_lds(reinterpret_cast<const void*>(&k_fft_rows_6144), kRows6Lds);
+            k_fft_rows_6144<<<static_cast<unsigned>(P * kSub), kRows6Threads, kRows6Lds, ctx->stream>>>(planes, row_out, tw,
+                                                                                                     tab, clo, nc, mid);
+        } else if (split == 2) {
+            k_fft_rows_3072<<<static_cast<unsigned>(P * kSub), 256, 0, ctx->stream>>>(planes, row_out, tw, tab, clo, nc, mid);
+        } else {
+            const int total_rows = static_cast<int>(P * G);
+            k_fft_rows_1536<<<static_cast<unsigned>((total_rows + kFftWaves - 1) / kFftWaves), 64 * kFftWaves, 0,
+                              ctx->stream>>>(planes, row_out, tab, total_rows, clo, nc, mid);
+        }
+        SVDI_LAUNCH_CHECK();
+        const int tiles = static_cast<int>(P) * split * nblk;
+        ColsOut o;
+        o.plane_stride = rows * cols;
+        o.block_stride = win.split != 0 ? rows * kBlockCols : kBlockCols;
+        o.row_stride = win.split != 0 ? kBlockCols : nc;
+        o.split_rows = win.split != 0 ? static_cast<int>(rows) / split : 0;
+        allow_dynamic_lds(reinterpret_cast<const void*>(&k_fft_cols_1536), kColsLds);
+        const int grid = std::min(tiles, std::max(1, ctx->cu_count));
+        k_fft_cols_1536<<<static_cast<unsigned>(grid), 64 * kBlockCols, kColsLds, ctx->stream>>>(
+            row_out, out, tab, split, tiles, nblk, nc, static_cast<int>(row_lo), static_cast<int>(rows), mid, o);
+        SVDI_LAUNCH_CHECK();
+        return;
+    }
     FftStages st;
     const size_t per = 2 * padded_len(G) * sizeof(float2);     // one transform, ping-pong
     const size_t twb = G * sizeof(float2);
@@ -818,37 +908,13 @@ void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size
     auto cols_fn = inplace ? &k_fft_cols<true> : &k_fft_cols<false>;
     allow_dynamic_lds(reinterpret_cast<const void*>(rows_fn), lds);
     allow_dynamic_lds(reinterpret_cast<const void*>(cols_fn), lds);
-    if (G == 6144) {
-        k_fft_rows_6144<<<static_cast<unsigned>(P * G), 256, 0, ctx->stream>>>(
-            planes, row_out, tw, static_cast<int>(col_lo), static_cast<int>(cols));
-    } else if (G == 3072) {
-        k_fft_rows_3072<<<static_cast<unsigned>(P * 1536), 256, 0, ctx->stream>>>(
-            planes, row_out, tw, static_cast<int>(col_lo), static_cast<int>(cols));
-    } else if (G == 1536) {
-        const int total_rows = static_cast<int>(P * G);
-        k_fft_rows_1536<<<static_cast<unsigned>((total_rows + kFftWaves - 1) / kFftWaves), 64 * kFftWaves, 0,
-                          ctx->stream>>>(planes, row_out, tw, total_rows, static_cast<int>(col_lo),
-                                         static_cast<int>(cols));
-    } else {
+    {
         dim3 gr(static_cast<unsigned>((G + batch - 1) / batch), static_cast<unsigned>(P));
         rows_fn<<<gr, threads, lds, ctx->stream>>>(planes, row_out, st, tw, batch, static_cast<int>(col_lo),
                                                    static_cast<int>(cols));
     }
     SVDI_LAUNCH_CHECK();
-    if (G == 6144) {
-        const int strips = static_cast<int>((cols + kColStrip6 - 1) / kColStrip6);
-        allow_dynamic_lds(reinterpret_cast<const void*>(&k_fft_cols_6144), kCols6Lds);
-        k_fft_cols_6144<<<static_cast<unsigned>(strips * P), kCols6Threads, kCols6Lds, ctx->stream>>>(
-            row_out, out, tw, static_cast<int>(cols), static_cast<int>(row_lo), static_cast<int>(rows), strips);
-    } else if (G == 3072) {
-        const int strips = static_cast<int>((cols + kColStrip - 1) / kColStrip);
-        k_fft_cols_1536<2><<<static_cast<unsigned>(strips * 2 * P), 64 * kColStrip, 0, ctx->stream>>>(
-            row_out, out, tw, static_cast<int>(cols), static_cast<int>(row_lo), static_cast<int>(rows), strips);
-    } else if (G == 1536) {
-        const int strips = static_cast<int>((cols + kColStrip - 1) / kColStrip);
-        k_fft_cols_1536<1><<<static_cast<unsigned>(strips * P), 64 * kColStrip, 0, ctx->stream>>>(
-            row_out, out, tw, static_cast<int>(cols), static_cast<int>(row_lo), static_cast<int>(rows), strips);
-    } else {
+    {
         const int strips = static_cast<int>((cols + width - 1) / width);
         const unsigned gc = static_cast<unsigned>(strips * P);
         cols_fn<<<gc, threads, lds, ctx->stream>>>(row_out, out, st, tw, width, static_cast<int>(cols),

@@ -90,8 +90,8 @@ __device__ __forceinline__ bool image_pixel(const float2* __restrict__ planes, c
         ++lr;
     }
     const long gr = lr - ip.row_lo, gc = lc - ip.col_lo;
-    const size_t plane_stride = static_cast<size_t>(ip.rows) * ip.cols;
-    const float2* px = planes + static_cast<size_t>(gr) * ip.cols + gc;
+    const size_t plane_stride = static_cast<size_t>(ip.win.rows) * ip.win.cols;
+    const float2* px = planes + ip.win.index(static_cast<int>(gr), static_cast<int>(gc));
     float2 m[KMAX];
     auto load_slab = [&](int ls) {
 #pragma unroll

@@ -294,9 +294,24 @@ bool grid_windows_supported(const SampleInput& in, const GridParams& gp);
 
 // fft.hip
 void fft_prepare(svdi_context* ctx, size_t G);
+// float2 elements of a plane's row-transformed columns (launch_fft2_inverse's row_out).
+size_t fft_row_elems(size_t G, size_t cols);
+// Layout of a transformed plane's window: row-major (split = 0), or, for G = 1536 s (split = s), the
+// order in which the column pass produces it: columns in blocks of eight, and in a block the rows
+// s k + q by q, then k.
+struct FftWindow {
+    int rows = 0, cols = 0, split = 0;
+    __host__ __device__ size_t index(int r, int c) const {
+        if (split == 0) return static_cast<size_t>(r) * cols + c;
+        const int k = r / split, q = r - k * split;
+        return (static_cast<size_t>(c / 8) * rows + q * (rows / split) + k) * 8 + c % 8;
+    }
+};
+// The layout in which the image pass takes a window (row-major where the blocked one does not fit).
+FftWindow fft_window(size_t G, size_t row_lo, size_t rows, size_t cols);
 void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size_t G,
                          size_t row_lo, size_t rows, size_t col_lo, size_t cols,
-                         float2* row_out, float2* out);
+                         float2* row_out, float2* out, const FftWindow& win);
 
 // image.hip
 void launch_conv_corr(svdi_context* ctx, size_t N, size_t G, int archive_variant, float* conv);
@@ -309,7 +324,7 @@ struct ImageParams {
     float cell;
     float r3_min, slab_width, slab_half, r3_centre;
     float inv_num_samples;
-    int rows, cols;         // window sizes of the transformed planes
+    FftWindow win;          // layout of the transformed planes
     int row_lo, col_lo;
     int signed_out;
     int lin_q0, lin_r0;     // (G G / 2 + G / 2) = lin_q0 G + lin_r0 (set by launch_image)
