@@ -252,7 +252,7 @@ void launch_plan(svdi_context* ctx, const SampleInput& in, Semantics sem, size_t
     // r3 partials: from the row rotation (snapshot input) or a reduction over Bin.
     float* r3p;
     int r3_blocks;
-    char* misc = static_cast<char*>(ctx->ws.get(Workspace::kMisc, 1 << 20));
+    char* misc = static_cast<char*>(ctx->ws.get(Workspace::kMisc, 12 * 1024));
     if (in.r3_partials != nullptr) {
         r3p = const_cast<float*>(in.r3_partials);
         r3_blocks = in.r3_blocks;
@@ -263,8 +263,8 @@ void launch_plan(svdi_context* ctx, const SampleInput& in, Semantics sem, size_t
         SVDI_LAUNCH_CHECK();
     }
     const int t3_blocks = 512;
-    float* t3max = reinterpret_cast<float*>(misc + 64 * 1024);
-    uint32_t* t3valid = reinterpret_cast<uint32_t*>(misc + 128 * 1024);
+    float* t3max = reinterpret_cast<float*>(misc + 8 * 1024);
+    uint32_t* t3valid = reinterpret_cast<uint32_t*>(misc + 10 * 1024);
     const float* vin = in.from_snapshot ? in.geo->vin : in.vin_dev;
     k_t3_stats<<<t3_blocks, kThreads, 0, ctx->stream>>>(vin, image_size, cell, t3max, t3valid);
     SVDI_LAUNCH_CHECK();

@@ -294,6 +294,7 @@ bool grid_windows_supported(const SampleInput& in, const GridParams& gp);
 
 // fft.hip
 void fft_prepare(svdi_context* ctx, size_t G);
+size_t fft_table_bytes(size_t G);
 // float2 elements of a plane's row-transformed columns (launch_fft2_inverse's row_out).
 size_t fft_row_elems(size_t G, size_t cols);
 // Layout of a transformed plane's window: row-major (split = 0), or, for G = 1536 s (split = s), the

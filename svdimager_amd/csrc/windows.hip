@@ -1892,9 +1892,9 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     // Wavefront items: one per window at most.  Pieces (and partial slots): at most one per dense
     // half, of which there are at most records / (coop_min + 1), plus records / coop_cap.  The slots
     // of the worst case are bounded to kMaxPartialBytes (in the fixed scratch range to what is left but
-    // for the items and the FFT's twiddles) by a coarser shape.
+    // for the items and the FFT's tables) by a coarser shape.
     const size_t slot_bytes = static_cast<size_t>(gp.K) * kDenseCells * sizeof(float2) + sizeof(WItem);
-    const size_t reserve = nwt * (sizeof(WItem) + sizeof(WReduce)) + static_cast<size_t>(gp.G) * sizeof(float2) + (64u << 10);
+    const size_t reserve = nwt * (sizeof(WItem) + sizeof(WReduce)) + fft_table_bytes(static_cast<size_t>(gp.G)) + (32u << 10);
     const size_t left = ctx->ws.arena_left();
     const size_t partial_bytes = std::min(kMaxPartialBytes, left > reserve ? left - reserve : 0);
     auto slots = [&]() { return max_records / wg.coop_cap + std::min(2 * nwt, max_records / (wg.coop_min + 1)) + 1; };
