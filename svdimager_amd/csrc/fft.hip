@@ -45,16 +45,16 @@ struct FftStages {
 __device__ __forceinline__ int pidx(int i) { return i + (i >> 5); }
 __host__ __device__ inline size_t padded_len(size_t n) { return n + n / 32 + 1; }
 
-__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ float2 mul_i(float2 a) { return make_float2(-a.y, a.x); }   // i * a
+// Complex values are float2, or double2 where a butterfly is formed in FP64 (stage_inplace).
+template <class V> __device__ __forceinline__ V cmul(V a, V b) { return V(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+template <class V> __device__ __forceinline__ V cadd(V a, V b) { return V(a.x + b.x, a.y + b.y); }
+template <class V> __device__ __forceinline__ V csub(V a, V b) { return V(a.x - b.x, a.y - b.y); }
+template <class V> __device__ __forceinline__ V mul_i(V a) { return V(-a.y, a.x); }   // i * a
 
 // out[k] = sum_r v[r] e^{+2 pi i r k / R}
-__device__ __forceinline__ void dft2(float2* v) {
-    const float2 a = v[0], b = v[1];
+template <class V>
+__device__ __forceinline__ void dft2(V* v) {
+    const V a = v[0], b = v[1];
     v[0] = cadd(a, b);
     v[1] = csub(a, b);
 }
@@ -70,9 +70,10 @@ __device__ __forceinline__ void dft3(float2* v) {
     v[2] = csub(m, is);
 }
 
-__device__ __forceinline__ void dft4(float2* v) {
-    const float2 y0 = cadd(v[0], v[2]), y1 = csub(v[0], v[2]);
-    const float2 y2 = cadd(v[1], v[3]), y3 = mul_i(csub(v[1], v[3]));
+template <class V>
+__device__ __forceinline__ void dft4(V* v) {
+    const V y0 = cadd(v[0], v[2]), y1 = csub(v[0], v[2]);
+    const V y2 = cadd(v[1], v[3]), y3 = mul_i(csub(v[1], v[3]));
     v[0] = cadd(y0, y2);
     v[2] = csub(y0, y2);
     v[1] = cadd(y1, y3);
@@ -98,17 +99,18 @@ __device__ __forceinline__ void dft5(float2* v) {
     v[3] = csub(m2, mul_i(n2));
 }
 
-__device__ __forceinline__ void dft8(float2* v) {
-    const float h = 0.70710678118654752440f;
-    float2 a[4], b[4];
+template <class V>
+__device__ __forceinline__ void dft8(V* v) {
+    const decltype(v->x) h = 0.70710678118654752440;
+    V a[4], b[4];
     for (int r = 0; r < 4; ++r) {
         a[r] = cadd(v[r], v[r + 4]);
         b[r] = csub(v[r], v[r + 4]);
     }
     // b[r] *= e^{+2 pi i r / 8}
-    b[1] = make_float2(h * (b[1].x - b[1].y), h * (b[1].x + b[1].y));
+    b[1] = V(h * (b[1].x - b[1].y), h * (b[1].x + b[1].y));
     b[2] = mul_i(b[2]);
-    b[3] = make_float2(-h * (b[3].x + b[3].y), h * (b[3].x - b[3].y));
+    b[3] = V(-h * (b[3].x + b[3].y), h * (b[3].x - b[3].y));
     dft4(a);
     dft4(b);
     for (int m = 0; m < 4; ++m) {
@@ -128,8 +130,8 @@ __device__ __forceinline__ void dft_generic(float2* v, int R, const float2* __re
     for (int k = 0; k < R; ++k) v[k] = y[k];
 }
 
-template <int R>
-__device__ __forceinline__ void dft_fixed(float2* v) {
+template <int R, class V>
+__device__ __forceinline__ void dft_fixed(V* v) {
     if constexpr (R == 2) dft2(v);
     else if constexpr (R == 3) dft3(v);
     else if constexpr (R == 4) dft4(v);
@@ -188,11 +190,16 @@ __device__ void stage_generic(const float2* src, float2* dst, int ntrans, int n,
 
 // In-place form of a radix-R stage: every butterfly of the stage (at most kMaxB per thread) is
 // read and transformed into registers, then, after a barrier, written back to the same buffer.
-// Half the LDS of the ping-pong form, so twice the transforms per workgroup.
+// Half the LDS of the ping-pong form, so twice the transforms per workgroup.  V: the type of the
+// butterfly's arithmetic (double2 rounds once per stage, where values go back to LDS; FP64 runs at the
+// rate of plain FP32 here).
 constexpr int kMaxB = 4;
 constexpr int kInplaceThreads = 512;
 
-template <int R>
+template <class V>
+__device__ __forceinline__ V widen(float2 a) { return V(a.x, a.y); }
+
+template <int R, class V>
 __device__ __forceinline__ void stage_inplace(float2* buf, int ntrans, int n, int pn, int ns,
                                               FastDiv by_m, FastDiv by_ns, const float2* tw) {
     const int m = n / R;
@@ -210,10 +217,13 @@ __device__ __forceinline__ void stage_inplace(float2* buf, int ntrans, int n, in
             const int jq = static_cast<int>(by_ns.div(j));
             const int jm = j - jq * ns;
             const float2* in = buf + tr * pn;
-            v[b][0] = in[pidx(j)];
+            V x[R];
+            x[0] = widen<V>(in[pidx(j)]);
 #pragma unroll
-            for (int r = 1; r < R; ++r) v[b][r] = cmul(in[pidx(j + r * m)], tw[jm * r * tstep]);
-            dft_fixed<R>(v[b]);
+            for (int r = 1; r < R; ++r) x[r] = cmul(widen<V>(in[pidx(j + r * m)]), widen<V>(tw[jm * r * tstep]));
+            dft_fixed<R>(x);
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[b][r] = make_float2(static_cast<float>(x[r].x), static_cast<float>(x[r].y));
             obase[b] = (tr << 20) | (jq * ns * R + jm);     // tr < 16, index < 2^20
         }
     }
@@ -229,6 +239,8 @@ __device__ __forceinline__ void stage_inplace(float2* buf, int ntrans, int n, in
     __syncthreads();
 }
 
+// (double2: radices 2, 4 and 8 only.)
+template <class V = float2>
 __device__ void stockham_inplace(float2* buf, int ntrans, int pn, const FftStages& st, const float2* tw) {
     const int n = st.n;
     int ns = 1;
@@ -236,11 +248,15 @@ __device__ void stockham_inplace(float2* buf, int ntrans, int pn, const FftStage
         const int R = st.radix[stage];
         const FastDiv bm = st.by_m[stage], bn = st.by_ns[stage];
         switch (R) {
-            case 2: stage_inplace<2>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 3: stage_inplace<3>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 4: stage_inplace<4>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 5: stage_inplace<5>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
-            default: stage_inplace<8>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
+            case 2: stage_inplace<2, V>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
+            case 3:
+                if constexpr (sizeof(V) == sizeof(float2)) stage_inplace<3, V>(buf, ntrans, n, pn, ns, bm, bn, tw);
+                break;
+            case 4: stage_inplace<4, V>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
+            case 5:
+                if constexpr (sizeof(V) == sizeof(float2)) stage_inplace<5, V>(buf, ntrans, n, pn, ns, bm, bn, tw);
+                break;
+            default: stage_inplace<8, V>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
         }
         ns *= R;
     }
@@ -730,8 +746,10 @@ k_fft_cols(const float2* __restrict__ in, float2* __restrict__ out, FftStages st
 // n k = (n^2 + k^2 - (k - n)^2) / 2 gives X[k] = c[k] sum_n (x[n] c[n]) conj(c[k - n]), a circular
 // convolution of length M = 2^m >= 2 G - 1, done by two + transforms of length M in LDS:
 // z = conj(F(x c) B), X[k] = c[k] conj(F(z)[k]), where B = F(conj(c)) / M, conj(c) continued evenly.
-// Rows + columns of the planes of a 301^2 image (453^2): 46 + 29 us, as direct DFTs 518 + 304; the error
-// against 64 bits is 2.3e-7 rms of the output there, the direct sums' was 5.4e-7.
+// Rows + columns of the planes of a 301^2 image (453^2): 54 + 37 us, as direct DFTs 518 + 304.  The butterflies
+// are FP64: with FP32 ones (46 + 29 us) the transform's error was already below the direct sums' (2.3e-7
+// rms of white planes' output for 5.4e-7, now 1.5e-7), but the image's was 3 % above theirs, now 24 %
+// below.
 struct BlueTables {
     const float2 *chirp, *tw, *spec;               // c[G], W_M[M], B[M]
 };
@@ -770,14 +788,14 @@ __device__ __forceinline__ void blue_transforms(float2* lds, const FftStages& st
         buf[tr * pn + pidx(n)] = make_float2(0.f, 0.f);
     }
     __syncthreads();
-    stockham_inplace(buf, ntrans, pn, st, tw);
+    stockham_inplace<double2>(buf, ntrans, pn, st, tw);
     for (int t = threadIdx.x; t < M * ntrans; t += kInplaceThreads) {
         const int tr = t / M, k = t - tr * M;
         float2* at = buf + tr * pn + pidx(k);
         *at = cconj(cmul(*at, tb.spec[k]));
     }
     __syncthreads();
-    stockham_inplace(buf, ntrans, pn, st, tw);
+    stockham_inplace<double2>(buf, ntrans, pn, st, tw);
     for (int t = threadIdx.x; t < nk * ntrans; t += kInplaceThreads) {
         int tr, k;
         split(t, nk, tr, k);
