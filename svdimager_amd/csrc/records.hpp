@@ -75,6 +75,22 @@ SVDI_HD RecordWords rec_encode(int base1, float q1, int base2, float q2, float s
     return r;
 }
 
+// Records of a coarse bin (several row classes of a window column) keep the row cell relative to the
+// coarse bin's first row instead, row_shift = (the class's home window row's first row) - (that row)
+// more: -16 .. 111 in seven bits, the highest of them in place of the column cell's sign copy (a
+// column cell is in -16 .. 15 there).
+SVDI_HD void rec_to_coarse(RecordWords& r, int row_shift) {
+    const uint32_t row = static_cast<uint32_t>((static_cast<int32_t>(r.w[2]) >> 26) + row_shift + 16);
+    r.w[2] = (r.w[2] & 0x03ffffffu) | (row << 26);
+    r.w[3] = (r.w[3] & 0x7fffffffu) | (((row >> 6) & 1u) << 31);
+}
+SVDI_HD int rec_coarse_row(uint32_t w2, uint32_t w3) { return static_cast<int>((w2 >> 26) | ((w3 >> 31) << 6)) - 16; }
+SVDI_HD void rec_from_coarse(RecordWords& r, int row_shift) {
+    const uint32_t row = static_cast<uint32_t>(rec_coarse_row(r.w[2], r.w[3]) + row_shift);
+    r.w[2] = (r.w[2] & 0x03ffffffu) | (row << 26);
+    r.w[3] = (r.w[3] & 0x7fffffffu) | ((r.w[3] & 0x40000000u) << 1);
+}
+
 // Decoders (the window kernel inlines the same expressions).
 SVDI_HD int rec_cell(uint32_t w) { return static_cast<int32_t>(w) >> 26; }
 SVDI_HD uint32_t rec_frac_bits(uint32_t w) { return (w >> 8) & ((1u << kRecFracBits) - 1u); }

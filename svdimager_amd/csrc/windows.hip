@@ -28,8 +28,10 @@
 // LDS histograms kept per block; a prefix over the blocks and a scan of the bin totals give each
 // block its first slot in every bin, and one more pass over its samples writes the records
 // (position relative to the class's home window row / the window column, s, v).  When the bins
-// do not fit in one LDS histogram they are split into bands of consecutive bins, and each band
-// is a separate set of workgroups that reads the block's samples and handles only its own bins.
+// do not fit in one LDS histogram, runs of eight classes are binned together first and each such
+// coarse bin's records are then sorted by class (k_sub_bins).  Coarse bins that still do not fit are
+// split into bands of consecutive bins, and each band is a separate set of workgroups that reads the
+// block's samples and handles only its own bins.
 #include "sample.hpp"
 #include "scan.hpp"
 #include "es_poly.hpp"
@@ -53,6 +55,8 @@ constexpr int kBinPerThread = 16;        // samples per thread, preprocessed inp
 constexpr int kLdsBins = 36864;          // largest block-local histogram (144 KB of LDS)
 constexpr size_t kMaxBlockHistBytes = size_t(1) << 31;   // per-block histograms of all bands
 constexpr size_t kMaxPartialBytes = size_t(1) << 29;     // partial slots of the dense halves
+constexpr int kSupLog2 = 3;              // row classes binned together when the bins pass kLdsBins
+constexpr int kSup = 1 << kSupLog2;
 constexpr int kChunk = 32;               // samples per MFMA reduction step
 constexpr int kStride = 36;              // floats per c staging row (32 samples + pad)
 constexpr int kStrideH = 40;             // halves per ES staging row (32 samples + pad, 16-byte rows)
@@ -108,8 +112,11 @@ struct WinGeom {
     int nwin;        // nw * nw
     int nwin_total;  // nslabs * nwin
     int nbins;       // nslabs * nw * nh, ordered (slab, window column, row class)
+    int sup_log2;    // log2 of the row classes that are binned together (0, or kSupLog2)
+    int sup_rows;    // ceil(nh / 2^sup_log2)
+    int lbins;       // bins of the count and scatter passes: nslabs * nw * sup_rows
     int use_lds;     // block histograms in LDS (else one global atomic per record)
-    int band_bins;   // bins per LDS band (<= kLdsBins); band y covers [y band_bins, ...)
+    int band_bins;   // bins per LDS band (<= kLdsBins); band y covers [y band_bins, ...) of lbins
     uint32_t coop_min;   // records up to which a window is one wavefront item
     uint32_t coop_cap;   // records per workgroup piece
 };
@@ -158,7 +165,7 @@ __device__ __forceinline__ void for_sample_bins(const SampleInput& in, const Gri
         const int col0 = f.local_slab * wg.nw;
         const int wb0 = static_cast<int>(static_cast<uint32_t>(f.b0) / kWin);
         const int wb1 = static_cast<int>(static_cast<uint32_t>(f.b0 + f.nb - 1) / kWin);
-        for (int wb = wb0; wb <= wb1; ++wb) fn(f, (col0 + wb) * wg.nh + h, h, wb);
+        for (int wb = wb0; wb <= wb1; ++wb) fn(f, (col0 + wb) * wg.sup_rows + (h >> wg.sup_log2), h, wb);
     };
     if constexpr (kSnap) {
         if (in.quad_rows) {
@@ -283,11 +290,11 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v) {
 // Bins [lo, lo + n) of LDS band blockIdx.y.
 __device__ __forceinline__ void lds_band(const WinGeom& wg, int& lo, int& n) {
     lo = static_cast<int>(blockIdx.y) * wg.band_bins;
-    n = min(wg.band_bins, wg.nbins - lo);
+    n = min(wg.band_bins, wg.lbins - lo);
 }
 
 // Bin counts: per (block, band) in an LDS histogram (dynamic LDS) written to
-// blockhist[block * nbins + bin] for the band's bins, and the (block, band)'s record total to
+// blockhist[block * lbins + bin] for the band's bins, and the (block, band)'s record total to
 // blocktot[band * blocks + block] (without LDS histograms the counts go straight to counts[bin]).
 // kHist16: 16-bit counters, two bins per LDS word (bin b in the half b & 1 of word b / 2, added
 // to by a 32-bit atomic of 1 << 16 (b & 1)), for blocks of fewer than 65536 samples: a sample
@@ -322,7 +329,7 @@ k_win_count(SampleInput in, GridParams gp, WinGeom wg, uint32_t* __restrict__ co
     });
     const uint32_t tot = block_sum(cnt);          // (its barrier also ends the histogram's atomics)
     if (threadIdx.x == 0) blocktot[static_cast<size_t>(blockIdx.y) * gridDim.x + blk] = tot;
-    CountT* row = blockhist + blk * wg.nbins + lo;
+    CountT* row = blockhist + blk * wg.lbins + lo;
     for (int b = threadIdx.x; b < n; b += kBinThreads)
         row[b] = static_cast<CountT>(kHist16 ? (hist[b >> 1] >> ((b & 1) << 4)) & 0xffffu : hist[b]);
 }
@@ -429,6 +436,8 @@ k_win_scatter(SampleInput in, GridParams gp, WinGeom wg, const uint32_t* __restr
         // keeps its home's first cell 0, with the largest fraction instead.
         if (wb > 0 && f.b0 >= wb * kWin && static_cast<int32_t>(w.w[3]) < 0)
             w.w[3] = (((1u << kRecFracBits) - 1u) << 8) | (w.w[3] & 0xffu);
+        if (wg.sup_log2 != 0)
+            rec_to_coarse(w, kWin * home - ((h >> wg.sup_log2) << (wg.sup_log2 + wg.cls_log2)));
         rec.put(slot, w);
     };
     const size_t blk = blockIdx.x;
@@ -441,7 +450,7 @@ k_win_scatter(SampleInput in, GridParams gp, WinGeom wg, const uint32_t* __restr
     }
     int lo, n;
     lds_band(wg, lo, n);
-    const uint32_t* row = blockhist + blk * wg.nbins + lo;
+    const uint32_t* row = blockhist + blk * wg.lbins + lo;
     for (int b = threadIdx.x; b < n; b += kBinThreads) hist[b] = row[b];
     __syncthreads();
     uint32_t cnt = 0;
@@ -456,6 +465,151 @@ k_win_scatter(SampleInput in, GridParams gp, WinGeom wg, const uint32_t* __restr
     if (threadIdx.x == 0 && tot != blocktot[static_cast<size_t>(blockIdx.y) * gridDim.x + blk])
         atomicOr(err, kErrBinMismatch);
     block_max_to(m, vmax_bits);
+}
+
+// The records of the coarse bins (kSup row classes of a window column) sorted by class, and the
+// offsets boff of all bins.  A wavefront takes a piece of at most kSubPiece records of one coarse
+// bin into registers, ranks the records of each class by ballots and writes them to the class's range.
+// A coarse bin of one piece needs nothing else; the classes of larger ones are counted first
+// (kCount) in cls, and `used` hands out their slots to the pieces.  k_sub_list lists the pieces, those
+// of the larger coarse bins from the front and the others from the back, so that the wavefronts share
+// the few coarse bins near the uv centre, with thousands of pieces, evenly (16.7 M samples at 4096^2: 343 us;
+// given out by a fixed rule over groups of 256 coarse bins 543).
+// Bound by HBM: records read once (twice in coarse bins of several pieces) and written once.
+constexpr int kSubLoads = 8;
+constexpr int kSubPiece = 64 * kSubLoads;
+constexpr int kSubWaves = 4;             // wavefronts per workgroup
+constexpr int kSubGroupsPerCu = 4;
+
+// (bin, first record of the bin, piece number, records of the piece; pieces of one-piece coarse bins,
+// empty ones among them, are at the list's end.)
+struct SubPiece {
+    uint32_t bin, lo, piece, n;
+};
+
+// counts[0], [1]: pieces listed from the front and from the back.  A coarse bin of n records has
+// max(1, ceil(n / kSubPiece)) pieces, so `cap` = lbins + max_records / kSubPiece holds them all.
+__global__ void __launch_bounds__(256)
+k_sub_list(const uint32_t* __restrict__ coff, WinGeom wg, uint32_t limit, SubPiece* __restrict__ list, uint32_t cap,
+           uint32_t* __restrict__ counts, uint32_t* __restrict__ boff) {
+    const int bin = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+    if (bin == 0) boff[wg.nbins] = coff[wg.lbins];
+    uint32_t lo = 0, n = 0;
+    if (bin < wg.lbins) {
+        lo = min(coff[bin], limit);
+        n = min(coff[bin + 1], limit) - lo;
+    }
+    const bool single = bin < wg.lbins && n <= static_cast<uint32_t>(kSubPiece);
+    const uint64_t singles = __ballot(single);
+    uint32_t base = 0;
+    if (lane == 0 && singles != 0) base = atomicAdd(&counts[1], static_cast<uint32_t>(__popcll(singles)));
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (single) {
+        const uint32_t at = base + __popcll(singles & ((1ull << lane) - 1));
+        if (at < cap) list[cap - 1 - at] = {static_cast<uint32_t>(bin), lo, 0u, n};
+    }
+    // The larger ones' pieces: one reservation per wavefront, then all its lanes list a coarse bin's.
+    const uint32_t pieces = bin < wg.lbins && !single ? (n + kSubPiece - 1) / kSubPiece : 0u;
+    uint32_t incl = pieces;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t v = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += v;
+    }
+    base = 0;
+    if (lane == 63 && incl != 0) base = atomicAdd(&counts[0], incl);
+    const uint32_t first = __builtin_amdgcn_readlane(base, 63) + incl - pieces;
+    uint64_t todo = __ballot(pieces != 0);
+    while (todo != 0) {
+        const int i = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const uint32_t b_lo = __builtin_amdgcn_readlane(lo, i), b_n = __builtin_amdgcn_readlane(n, i);
+        const uint32_t b_first = __builtin_amdgcn_readlane(first, i), b_pieces = __builtin_amdgcn_readlane(pieces, i);
+        for (uint32_t p = lane; p < b_pieces; p += 64)
+            if (b_first + p < cap)
+                list[b_first + p] = {static_cast<uint32_t>(bin - lane + i), b_lo, p,
+                                     min(b_n - p * kSubPiece, static_cast<uint32_t>(kSubPiece))};
+    }
+}
+
+template <bool kCount>
+__global__ void __launch_bounds__(kSubWaves * 64)
+k_sub_bins(const SubPiece* __restrict__ list, uint32_t cap, const uint32_t* __restrict__ counts, WinGeom wg,
+           const uint4* __restrict__ coarse, uint32_t* __restrict__ cls, uint32_t* __restrict__ used,
+           uint32_t* __restrict__ boff, WRecords rec, uint32_t limit) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * kSubWaves + (threadIdx.x >> 6));
+    const uint32_t nwaves = gridDim.x * kSubWaves;
+    const int my = lane & (kSup - 1);                      // the class that this lane counts
+    const uint32_t multi = min(counts[0], cap);
+    const uint32_t total = kCount ? multi : min(multi + counts[1], cap);
+    // Lanes of class c among those whose class bits are (b0, b1, b2).
+    auto among = [](uint64_t b0, uint64_t b1, uint64_t b2, int c) {
+        return ((c & 1) ? b0 : ~b0) & ((c & 2) ? b1 : ~b1) & ((c & 4) ? b2 : ~b2);
+    };
+    auto piece = [&](uint32_t t) { return list[t < multi ? t : cap - 1 - (t - multi)]; };
+    auto load = [&](const SubPiece& s, uint4 (&q)[kSubLoads]) {
+        const uint4* src = coarse + s.lo + s.piece * kSubPiece;
+#pragma unroll
+        for (int r = 0; r < kSubLoads; ++r)
+            if (64u * r + lane < s.n) q[r] = src[64 * r + lane];
+    };
+    uint32_t t = wave;
+    if (t >= total) return;
+    SubPiece s = piece(t), s_next = s;
+    uint4 q[kSubLoads];
+    load(s, q);
+    if (t + nwaves < total) s_next = piece(t + nwaves);
+    for (;;) {
+        // The classes, then (the row cells are not needed for anything else) the records as they are
+        // written, so that the next piece's loads can be requested behind them.
+        int c[kSubLoads];
+        uint32_t cnt = 0;
+        const int col = static_cast<int>(s.bin) / wg.sup_rows, sup = static_cast<int>(s.bin) - col * wg.sup_rows;
+#pragma unroll
+        for (int r = 0; r < kSubLoads; ++r) {
+            const bool valid = 64u * r + lane < s.n;
+            c[r] = valid ? min(max(rec_coarse_row(q[r].z, q[r].w) >> wg.cls_log2, 0), kSup - 1) : 0;
+            const uint64_t b0 = __ballot(c[r] & 1), b1 = __ballot(c[r] & 2), b2 = __ballot(c[r] & 4);
+            cnt += __popcll(among(b0, b1, b2, my) & __ballot(valid));
+        }
+        if constexpr (kCount) {
+            if (lane < kSup && cnt != 0) atomicAdd(&cls[kSup * s.bin + lane], cnt);
+        } else {
+            const bool single = t >= multi;
+            const uint32_t tot = single ? cnt : cls[kSup * s.bin + my];
+            uint32_t start = s.lo;                         // first slot of class `my`
+#pragma unroll
+            for (int k = 0; k < kSup - 1; ++k) {
+                const uint32_t u = __builtin_amdgcn_readlane(tot, k);
+                start += my > k ? u : 0u;
+            }
+            const int h = kSup * sup + my;
+            if (s.piece == 0 && lane < kSup && h < wg.nh) boff[col * wg.nh + h] = start;
+            if (!single && lane < kSup && cnt != 0) start += atomicAdd(&used[kSup * s.bin + lane], cnt);
+#pragma unroll
+            for (int r = 0; r < kSubLoads; ++r) {
+                const bool valid = 64u * r + lane < s.n;
+                const uint64_t b0 = __ballot(c[r] & 1), b1 = __ballot(c[r] & 2), b2 = __ballot(c[r] & 4);
+                const uint64_t in = __ballot(valid);
+                const uint64_t same = among(b0, b1, b2, c[r]) & in;
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(same >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(same), 0u));
+                const uint32_t slot = __shfl(start, c[r], 64) + rank;
+                if (valid && slot < limit) {
+                    const int h0 = kSup * sup + c[r];
+                    RecordWords w = {{q[r].x, q[r].y, q[r].z, q[r].w}};
+                    rec_from_coarse(w, ((kSup * sup) << wg.cls_log2) - ((((h0 << wg.cls_log2) + 8) >> 4) * kWin));
+                    rec.put(slot, w);
+                }
+                start += __popcll(among(b0, b1, b2, my) & in);
+            }
+        }
+        t += nwaves;
+        if (t >= total) break;
+        s = s_next;
+        load(s, q);
+        if (t + nwaves < total) s_next = piece(t + nwaves);
+    }
 }
 
 // Record range of window w (slab, wa, wb): bnd[j] = first record of the window's class j
@@ -1841,18 +1995,36 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     unsigned blocks;
     if (in.from_snapshot) blocks = static_cast<unsigned>((in.num_rows + kBinRows - 1) / kBinRows);
     else blocks = static_cast<unsigned>((S + kBinThreads * kBinPerThread - 1) / (kBinThreads * kBinPerThread));
+    // Bins that pass the LDS histogram are counted and scattered as coarse bins of eight row classes,
+    // whose records k_sub_bins then sorts by class: one pass over the samples where there were up to
+    // eight, for one more over the records.  16.7 M samples at 4096^2 (294,912 bins): count, scatter and
+    // offsets 1.77 ms, now 0.70; 3.8 M at 2048^2 in three slabs 396 us, now 310.  The records wait in the planes, which nothing has written yet; if
+    // these are too small, in LDS bands of the bins themselves.
+    const size_t sub_bins = static_cast<size_t>(gp.nslabs) * wg.nw * ((wg.nh + kSup - 1) / kSup);
+    const uint32_t sub_cap = static_cast<uint32_t>(sub_bins + max_records / kSubPiece);
+    const size_t sub_bytes = sub_cap * sizeof(SubPiece);
+    const size_t planes_bytes = static_cast<size_t>(gp.nslabs) * gp.K * gp.G * gp.G * sizeof(float2);
+    const bool coarse = nbins > static_cast<size_t>(kLdsBins) && max_records * sizeof(uint4) + sub_bytes <= planes_bytes;
+    wg.sup_log2 = coarse ? kSupLog2 : 0;
+    wg.sup_rows = (wg.nh + (1 << wg.sup_log2) - 1) >> wg.sup_log2;
+    const size_t lbins = static_cast<size_t>(gp.nslabs) * wg.nw * wg.sup_rows;
+    wg.lbins = static_cast<int>(lbins);
     // LDS bands of at most kLdsBins bins, unless the per-block histograms would pass
     // kMaxBlockHistBytes (then one global atomic per record).
-    const size_t nbands = (nbins + kLdsBins - 1) / kLdsBins;
-    wg.use_lds = static_cast<size_t>(blocks) * nbins * sizeof(uint32_t) <= kMaxBlockHistBytes ? 1 : 0;
-    wg.band_bins = static_cast<int>((nbins + nbands - 1) / nbands);
+    const size_t nbands = (lbins + kLdsBins - 1) / kLdsBins;
+    wg.use_lds = static_cast<size_t>(blocks) * lbins * sizeof(uint32_t) <= kMaxBlockHistBytes ? 1 : 0;
+    wg.band_bins = static_cast<int>((lbins + nbands - 1) / nbands);
     const unsigned bands = wg.use_lds ? static_cast<unsigned>(nbands) : 1u;
-    const size_t nhist = wg.use_lds ? static_cast<size_t>(blocks) * nbins : 1;
+    const size_t nhist = wg.use_lds ? static_cast<size_t>(blocks) * lbins : 1;
     const size_t bin_lds = wg.use_lds ? static_cast<size_t>(wg.band_bins) * sizeof(uint32_t) : 0;
     const dim3 bin_grid(blocks, bands);
 
-    // counts[0, nbins) | counts[nbins + 2, +8) = totals.
-    uint32_t* counts = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinCounts, (nbins + 12) * sizeof(uint32_t)));
+    // counts[0, lbins) | counts[lbins + 2, +8) = totals, [+8, +10) = the coarse bins' pieces | the coarse bins' class counts and the slots
+    // handed out, kSup lbins each.
+    const size_t nsub = coarse ? kSup * lbins : 0;
+    const size_t ncleared = lbins + 12 + 2 * nsub;
+    uint32_t* counts = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinCounts, ncleared * sizeof(uint32_t)));
+    uint32_t* sub_counts = counts + lbins + 12;
     // Per-block record offsets (the counts themselves when 32-bit), the (block, band) record
     // totals, then the 16-bit per-block counts when a block has fewer than 65536 samples (a
     // bin's count per block is at most its sample count).
@@ -1865,16 +2037,19 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     uint32_t* blocktot = blockhist + nhist;
     uint16_t* blockcount16 = count16 ? reinterpret_cast<uint16_t*>(blocktot + ntot) : nullptr;
     uint32_t* boff = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinOffsets, (nbins + 8) * sizeof(uint32_t)));
-    uint32_t* cursor = static_cast<uint32_t*>(
-        ctx->ws.get(Workspace::kBinCursor, (nbins + 8 + nwt + (wg.use_lds ? kBinSegs * nbins : 0)) * sizeof(uint32_t)));
-    uint32_t* multi = cursor + nbins + 8;                  // windows with several pieces
-    uint32_t* segsum = multi + nwt;                        // [kBinSegs][nbins]
+    // The coarse bins' offsets, or those of the bins themselves; cursors (without LDS histograms); the
+    // windows with several pieces; segment sums [kBinSegs][lbins].
+    uint32_t* cursor = static_cast<uint32_t*>(ctx->ws.get(
+        Workspace::kBinCursor, (lbins + 8 + nwt + (wg.use_lds ? kBinSegs * lbins : 0) + (coarse ? lbins + 8 : 0)) * sizeof(uint32_t)));
+    uint32_t* multi = cursor + lbins + 8;
+    uint32_t* segsum = multi + nwt;
+    uint32_t* coff = coarse ? segsum + (wg.use_lds ? kBinSegs * lbins : 0) : boff;
     const size_t ncounts = (3 * kItemClasses + 2) * nwt;
     uint32_t* sums = static_cast<uint32_t*>(
-        ctx->ws.get(Workspace::kScanSums, scan_blocks(std::max(nbins, ncounts)) * sizeof(uint32_t)));
+        ctx->ws.get(Workspace::kScanSums, scan_blocks(std::max(lbins, ncounts)) * sizeof(uint32_t)));
     uint32_t* icount = static_cast<uint32_t*>(ctx->ws.get(Workspace::kItemCounts, (ncounts + 8) * sizeof(uint32_t)));
     uint32_t* ioff = static_cast<uint32_t*>(ctx->ws.get(Workspace::kItemOffsets, (ncounts + 8) * sizeof(uint32_t)));
-    uint32_t* totals = counts + nbins + 2;
+    uint32_t* totals = counts + lbins + 2;
     WRecords rec;
     rec.r = static_cast<uint4*>(ctx->ws.get(Workspace::kRecPos, max_records * sizeof(uint4)));
 
@@ -1911,7 +2086,7 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
         ctx->ws.get(Workspace::kWinPartial, (max_slots * piece_floats2 + 64) * sizeof(float2)));
     float2* trash = partial + max_slots * piece_floats2;
 
-    launch_fill(ctx, reinterpret_cast<float*>(counts), nbins + 12, 0.0f);
+    launch_fill(ctx, reinterpret_cast<float*>(counts), ncleared, 0.0f);
     // 16-bit LDS histograms (two bins per word) when there are also more blocks than CUs, so that
     // two can share a CU.  With one block per CU the halved LDS gains nothing and the packing
     // costs a little (snapshot rows at 64 channels: 35.9 against 33.9 us; preprocessed samples:
@@ -1932,24 +2107,50 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
         else count(&k_win_count<false, false, uint32_t>, blockhist);
     }
     SVDI_LAUNCH_CHECK();
-    const unsigned seg_grid = static_cast<unsigned>((kBinSegs * nbins + 255) / 256);
+    const unsigned seg_grid = static_cast<unsigned>((kBinSegs * lbins + 255) / 256);
     if (wg.use_lds) {
         if (count16)
             k_bin_seg_sums<uint16_t><<<seg_grid, 256, 0, ctx->stream>>>(blockcount16, static_cast<int>(blocks),
-                                                                       wg.nbins, segsum, counts);
+                                                                       wg.lbins, segsum, counts);
         else
-            k_bin_seg_sums<uint32_t><<<seg_grid, 256, 0, ctx->stream>>>(blockhist, static_cast<int>(blocks), wg.nbins,
+            k_bin_seg_sums<uint32_t><<<seg_grid, 256, 0, ctx->stream>>>(blockhist, static_cast<int>(blocks), wg.lbins,
                                                                        segsum, counts);
         SVDI_LAUNCH_CHECK();
     }
-    launch_exclusive_scan(ctx, counts, boff, wg.use_lds ? nullptr : cursor, sums, nbins);
+    launch_exclusive_scan(ctx, counts, coff, wg.use_lds ? nullptr : cursor, sums, lbins);
     if (wg.use_lds) {
         if (count16)
             k_bin_block_offsets<uint16_t><<<seg_grid, 256, 0, ctx->stream>>>(
-                blockcount16, blockhist, static_cast<int>(blocks), wg.nbins, segsum, boff);
+                blockcount16, blockhist, static_cast<int>(blocks), wg.lbins, segsum, coff);
         else
             k_bin_block_offsets<uint32_t><<<seg_grid, 256, 0, ctx->stream>>>(
-                blockhist, blockhist, static_cast<int>(blocks), wg.nbins, segsum, boff);
+                blockhist, blockhist, static_cast<int>(blocks), wg.lbins, segsum, coff);
+        SVDI_LAUNCH_CHECK();
+    }
+    const uint32_t limit = static_cast<uint32_t>(max_records);
+    const WRecords scattered = coarse ? WRecords{reinterpret_cast<uint4*>(planes)} : rec;
+    SubPiece* sub_list = reinterpret_cast<SubPiece*>(reinterpret_cast<uint4*>(planes) + max_records);
+    if (in.from_snapshot) {
+        allow_dynamic_lds(reinterpret_cast<const void*>(&k_win_scatter<true>), bin_lds);
+        k_win_scatter<true><<<bin_grid, kBinThreads, bin_lds, ctx->stream>>>(in, gp, wg, blockhist, blocktot, cursor,
+                                                                         scattered, limit, totals + 4, ctx->dev_err);
+    } else {
+        allow_dynamic_lds(reinterpret_cast<const void*>(&k_win_scatter<false>), bin_lds);
+        k_win_scatter<false><<<bin_grid, kBinThreads, bin_lds, ctx->stream>>>(in, gp, wg, blockhist, blocktot, cursor,
+                                                                          scattered, limit, totals + 4, ctx->dev_err);
+    }
+    SVDI_LAUNCH_CHECK();
+    if (coarse) {
+        k_sub_list<<<static_cast<unsigned>((lbins + 255) / 256), 256, 0, ctx->stream>>>(coff, wg, limit, sub_list, sub_cap,
+                                                                                       totals + 8, boff);
+        SVDI_LAUNCH_CHECK();
+        const unsigned sub_grid = static_cast<unsigned>(std::min<size_t>(ctx->cu_count * kSubGroupsPerCu,
+                                                                         (sub_cap + kSubWaves - 1) / kSubWaves));
+        k_sub_bins<true><<<sub_grid, kSubWaves * 64, 0, ctx->stream>>>(sub_list, sub_cap, totals + 8, wg, scattered.r,
+                                                                       sub_counts, sub_counts + nsub, boff, rec, limit);
+        SVDI_LAUNCH_CHECK();
+        k_sub_bins<false><<<sub_grid, kSubWaves * 64, 0, ctx->stream>>>(sub_list, sub_cap, totals + 8, wg, scattered.r,
+                                                                        sub_counts, sub_counts + nsub, boff, rec, limit);
         SVDI_LAUNCH_CHECK();
     }
     k_win_item_counts<<<static_cast<unsigned>((nwt + 255) / 256), 256, 0, ctx->stream>>>(boff, wg, icount, multi, totals);
@@ -1957,17 +2158,6 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     launch_exclusive_scan(ctx, icount, ioff, nullptr, sums, ncounts);
     k_win_item_write<<<static_cast<unsigned>((max_items + 255) / 256), 256, 0, ctx->stream>>>(
         boff, ioff, multi, wg, items, static_cast<uint32_t>(max_items), red, totals);
-    SVDI_LAUNCH_CHECK();
-    const uint32_t limit = static_cast<uint32_t>(max_records);
-    if (in.from_snapshot) {
-        allow_dynamic_lds(reinterpret_cast<const void*>(&k_win_scatter<true>), bin_lds);
-        k_win_scatter<true><<<bin_grid, kBinThreads, bin_lds, ctx->stream>>>(in, gp, wg, blockhist, blocktot, cursor,
-                                                                         rec, limit, totals + 4, ctx->dev_err);
-    } else {
-        allow_dynamic_lds(reinterpret_cast<const void*>(&k_win_scatter<false>), bin_lds);
-        k_win_scatter<false><<<bin_grid, kBinThreads, bin_lds, ctx->stream>>>(in, gp, wg, blockhist, blocktot, cursor,
-                                                                          rec, limit, totals + 4, ctx->dev_err);
-    }
     SVDI_LAUNCH_CHECK();
 
     WindowJob job;
