@@ -45,13 +45,9 @@ namespace {
 
 constexpr int kWin = 16;                 // window side in cells
 constexpr int kMaxClasses = 6;           // classes per window: 24 / class height (4 or 8)
-constexpr int kBinThreads = 1024;        // binning blocks: 256 rows x 4 channel groups at a time
-constexpr int kBinRowSets = 2;           // row sets of 256 per block (fewer, larger blocks: the
-                                         // per-block histograms are written and read back whole)
-constexpr int kBinRowsPerSet = 256;
-constexpr int kBinRows = kBinRowSets * kBinRowsPerSet;
-constexpr int kBinChanGroups = kBinThreads / kBinRowsPerSet;
-constexpr int kBinPerThread = 16;        // samples per thread, preprocessed input
+constexpr int kBinThreads = 1024;        // binning blocks
+constexpr int kBinRowsMost = 512;        // rows of a block, snapshot input: 64 .. 512
+constexpr int kBinPerThreadMost = 16;    // samples per thread, preprocessed input: 1 .. 16
 constexpr int kLdsBins = 36864;          // largest block-local histogram (144 KB of LDS)
 constexpr size_t kMaxBlockHistBytes = size_t(1) << 31;   // per-block histograms of all bands
 constexpr size_t kMaxPartialBytes = size_t(1) << 29;     // partial slots of the dense halves
@@ -117,6 +113,8 @@ struct WinGeom {
     int lbins;       // bins of the count and scatter passes: nslabs * nw * sup_rows
     int use_lds;     // block histograms in LDS (else one global atomic per record)
     int band_bins;   // bins per LDS band (<= kLdsBins); band y covers [y band_bins, ...) of lbins
+    int block_size;  // binning blocks: rows (snapshot input), samples per thread (preprocessed)
+    int set_rows;    // rows of a block read at a time (64 or 256; snapshot rows read one by one)
     uint32_t coop_min;   // records up to which a window is one wavefront item
     uint32_t coop_cap;   // records per workgroup piece
 };
@@ -149,10 +147,10 @@ struct WRecords {
 
 // Every (sample, bin) pair of this block's samples: one row class h = a0 / c (c the class
 // height), and the window columns b0 / 16 .. (b0 + nb - 1) / 16 that the clipped footprint meets
-// (at most two).  Snapshot input: 512 consecutive rows in two sets of 256, each row split over 4
-// threads that take every fourth channel (a wavefront reads 64 consecutive rows of one channel:
-// coalesced), loading four samples before working on the first.  Preprocessed input: 16384
-// consecutive samples, 16 per thread at a stride of the block size.  kVis = false (snapshot
+// (at most two).  Snapshot input: block_size consecutive rows, in sets of set_rows, each row split over
+// kBinThreads / set_rows threads that take every so many channels (a wavefront reads 64 consecutive
+// rows of one channel: coalesced), loading four samples before working on the first.  Preprocessed
+// input: block_size consecutive samples per thread, at a stride of kBinThreads.  kVis = false (snapshot
 // input): neither visibilities nor weights are loaded and f.vw is zero; the bins depend on flags
 // and geometry only (samples are kept unless both polarisations are flagged, V = 0 when the
 // weights sum to zero), so both passes keep the same samples.
@@ -170,11 +168,11 @@ __device__ __forceinline__ void for_sample_bins(const SampleInput& in, const Gri
     if constexpr (kSnap) {
         if (in.quad_rows) {
             // Four consecutive rows of one channel per thread (one 16-byte load per FP32 array,
-            // 4 bytes per flag array; a wavefront reads 256 consecutive rows), 128 row quads x 8
-            // channel groups; the next channel's loads are issued before this one is binned.
-            constexpr int kQuads = kBinRows / 4;
-            constexpr int kQuadGroups = kBinThreads / kQuads;
-            const size_t row0 = blk * kBinRows + 4 * (threadIdx.x % kQuads);
+            // 4 bytes per flag array), 128 row quads x 8 channel groups in blocks of 512 rows (16 x
+            // 64 in blocks of 64); the next channel's loads are issued before this one is binned.
+            const uint32_t quads_log2 = 31 - __builtin_clz(static_cast<uint32_t>(wg.block_size) / 4);
+            const uint32_t quad_groups = kBinThreads >> quads_log2;
+            const size_t row0 = blk * wg.block_size + 4 * (threadIdx.x & ((1u << quads_log2) - 1));
             if (row0 >= in.num_rows) return;          // (num_rows % 4 == 0: quads are whole)
             struct QuadLoad {
                 double nu;
@@ -201,7 +199,7 @@ __device__ __forceinline__ void for_sample_bins(const SampleInput& in, const Gri
                 return q;
             };
             auto lane4 = [](const float4& v, int r) { return r == 0 ? v.x : r == 1 ? v.y : r == 2 ? v.z : v.w; };
-            size_t chan = threadIdx.x / kQuads;
+            size_t chan = threadIdx.x >> quads_log2;
             if (chan >= in.num_channels) return;
             QuadLoad cur = load(chan);
             double geo[4][3];
@@ -209,9 +207,9 @@ __device__ __forceinline__ void for_sample_bins(const SampleInput& in, const Gri
             for (int r = 0; r < 4; ++r)
 #pragma unroll
                 for (int k = 0; k < 3; ++k) geo[r][k] = in.rot[3 * (row0 + r) + k];
-            for (; chan < in.num_channels; chan += kQuadGroups) {
+            for (; chan < in.num_channels; chan += quad_groups) {
                 QuadLoad nxt = cur;
-                if (chan + kQuadGroups < in.num_channels) nxt = load(chan + kQuadGroups);
+                if (chan + quad_groups < in.num_channels) nxt = load(chan + quad_groups);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     SnapLoad s;
@@ -232,28 +230,29 @@ __device__ __forceinline__ void for_sample_bins(const SampleInput& in, const Gri
             return;
         }
         constexpr int kBatch = 4;
-        for (int set = 0; set < kBinRowSets; ++set) {
-        const size_t row = blk * kBinRows + set * kBinRowsPerSet + (threadIdx.x % kBinRowsPerSet);
+        const uint32_t groups = kBinThreads / static_cast<uint32_t>(wg.set_rows);
+        for (int set = 0; set < wg.block_size; set += wg.set_rows) {
+        const size_t row = blk * wg.block_size + set + (threadIdx.x & (wg.set_rows - 1));
         if (row >= in.num_rows) return;
         const double ru = in.rot[3 * row], rv = in.rot[3 * row + 1], rw = in.rot[3 * row + 2];
-        for (size_t c0 = threadIdx.x / kBinRowsPerSet; c0 < in.num_channels; c0 += kBatch * kBinChanGroups) {
+        for (size_t c0 = threadIdx.x / static_cast<uint32_t>(wg.set_rows); c0 < in.num_channels; c0 += kBatch * groups) {
             SnapLoad ld[kBatch] = {};
 #pragma unroll
             for (int u = 0; u < kBatch; ++u) {
-                const size_t chan = c0 + u * kBinChanGroups;
+                const size_t chan = c0 + u * groups;
                 if (chan < in.num_channels) ld[u] = load_snapshot_sample<kVis, kVis>(in, row + chan * in.num_rows, chan);
             }
 #pragma unroll
             for (int u = 0; u < kBatch; ++u) {
-                const size_t chan = c0 + u * kBinChanGroups;
+                const size_t chan = c0 + u * groups;
                 Footprint f;
                 if (chan < in.num_channels && finish_snapshot_sample<true>(gp, ru, rv, rw, ld[u], f)) bins_of(f);
             }
         }
         }
     } else {
-        const size_t base = blk * kBinThreads * kBinPerThread + threadIdx.x;
-        for (int j = 0; j < kBinPerThread; ++j) {
+        const size_t base = blk * kBinThreads * wg.block_size + threadIdx.x;
+        for (int j = 0; j < wg.block_size; ++j) {
             const size_t idx = base + static_cast<size_t>(j) * kBinThreads;
             if (idx >= in.num_samples) return;
             Footprint f;
@@ -1976,6 +1975,44 @@ bool grid_windows_supported(const SampleInput& in, const GridParams& gp) {
     return 2 * in.num_samples < (1ull << 31);             // records: at most two per sample
 }
 
+// The binning's block size (WinGeom) and the number of blocks.  A block's time goes with its samples
+// and, for its histogram, with the bins (about 3.7 ns a sample in the scatter and count passes together
+// with 3 ns for ten bins), one block per CU at a time; every block also costs 14 bytes per bin of counts
+// and offsets in memory.  So a snapshot that does not fill the chip with the largest blocks takes smaller
+// ones (scatter + count of 1.4 M samples in 29,377 rows at 1000^2: 58 blocks 114 us, 230 blocks 56; of 5.2 M
+// in 81,103 rows at 512^2: 159 blocks 171, 254 blocks 127), as long as its histograms do not cost more.  Rows read four
+// at a time take powers of two (their threads are dealt by shifts).
+static unsigned choose_bin_blocks(const svdi_context* ctx, const SampleInput& in, WinGeom& wg) {
+    // (Channels below sixteen would leave most of sixteen groups of threads idle.)
+    wg.set_rows = in.num_channels > 8 ? 64 : 256;
+    const size_t units = in.from_snapshot ? in.num_rows : (in.num_samples + kBinThreads - 1) / kBinThreads;
+    // Samples of a unit, a block's idle groups of threads included.
+    auto unit_samples = [&](int size) {
+        if (!in.from_snapshot) return static_cast<size_t>(kBinThreads);
+        const size_t groups = kBinThreads / (in.quad_rows ? size / 4 : wg.set_rows);
+        return (in.num_channels + groups - 1) / groups * groups;
+    };
+    const int most = in.from_snapshot ? kBinRowsMost : kBinPerThreadMost;
+    auto blocks_of = [&](int size) { return (units + size - 1) / static_cast<size_t>(size); };
+    wg.block_size = most;
+    // (The fixed scratch range keeps the largest blocks: fewer histograms.)
+    if (ctx->ws.arena_left() == SIZE_MAX) {
+        double best = 0.0;
+        const int step = in.from_snapshot ? (in.quad_rows ? 64 : wg.set_rows) : 1;
+        for (int size = most; size >= step; size = in.from_snapshot && in.quad_rows ? size / 2 : size - step) {
+            const size_t blocks = blocks_of(size);
+            const size_t rounds = (blocks + ctx->cu_count - 1) / ctx->cu_count;
+            const double bins = static_cast<double>(wg.lbins);
+            const double ns = rounds * (3.7 * static_cast<double>(size * unit_samples(size)) + 0.3 * std::min(bins, 1.0 * kLdsBins)) +
+                              blocks * bins * 0.0035;
+            if (size != most && (ns >= best || blocks * bins * sizeof(uint32_t) > kMaxBlockHistBytes / 8)) continue;
+            best = ns;
+            wg.block_size = size;
+        }
+    }
+    return static_cast<unsigned>(blocks_of(wg.block_size));
+}
+
 WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp, float2* planes) {
     if (gp.K < 1 || gp.K > kMaxTerms) throw std::logic_error("term count out of range");
     if (!grid_windows_supported(in, gp)) throw UnsupportedError("grid or sample count too large for the window gridder");
@@ -1992,9 +2029,6 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     const size_t max_records = 2 * S;                      // one row class, at most two window columns
     const size_t nbins = nbins_sz;
     const size_t nwt = static_cast<size_t>(wg.nwin_total);
-    unsigned blocks;
-    if (in.from_snapshot) blocks = static_cast<unsigned>((in.num_rows + kBinRows - 1) / kBinRows);
-    else blocks = static_cast<unsigned>((S + kBinThreads * kBinPerThread - 1) / (kBinThreads * kBinPerThread));
     // Bins that pass the LDS histogram are counted and scattered as coarse bins of eight row classes,
     // whose records k_sub_bins then sorts by class: one pass over the samples where there were up to
     // eight, for one more over the records.  16.7 M samples at 4096^2 (294,912 bins): count, scatter and
@@ -2009,6 +2043,7 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     wg.sup_rows = (wg.nh + (1 << wg.sup_log2) - 1) >> wg.sup_log2;
     const size_t lbins = static_cast<size_t>(gp.nslabs) * wg.nw * wg.sup_rows;
     wg.lbins = static_cast<int>(lbins);
+    const unsigned blocks = choose_bin_blocks(ctx, in, wg);
     // LDS bands of at most kLdsBins bins, unless the per-block histograms would pass
     // kMaxBlockHistBytes (then one global atomic per record).
     const size_t nbands = (lbins + kLdsBins - 1) / kLdsBins;
@@ -2028,8 +2063,7 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     // Per-block record offsets (the counts themselves when 32-bit), the (block, band) record
     // totals, then the 16-bit per-block counts when a block has fewer than 65536 samples (a
     // bin's count per block is at most its sample count).
-    const size_t block_samples = in.from_snapshot ? static_cast<size_t>(kBinRows) * in.num_channels
-                                                  : static_cast<size_t>(kBinThreads) * kBinPerThread;
+    const size_t block_samples = static_cast<size_t>(wg.block_size) * (in.from_snapshot ? in.num_channels : kBinThreads);
     const bool count16 = wg.use_lds && block_samples < 65536;
     const size_t ntot = static_cast<size_t>(blocks) * bands;
     uint32_t* blockhist = static_cast<uint32_t*>(ctx->ws.get(
