@@ -1,9 +1,9 @@
 // Batched 2D inverse DFT (sign +, unnormalised) of the moment planes, replacing
 // cufftPlanMany + cufftExecC2C(CUFFT_INVERSE) (SVDIntegratedImager.cu:1658-1676, 1713).
 //
-// Two LDS-staged passes of a mixed-radix Stockham FFT (radix 8/4/2/3/5 kernels plus a direct
-// butterfly for other primes up to 13).  G = ceil(3N/2) is 3 * 2^k for the usual image sizes; 1536,
-// 3072 and 6144 have passes of their own around a 1536-point transform held by one wavefront.
+// Two LDS-staged passes of a mixed-radix Stockham FFT (radices of 2 to 16, for lengths with prime
+// factors up to 13).  G = ceil(3N/2) is 3 * 2^k for the usual image sizes; 1536, 3072 and 6144 have
+// passes of their own around a 1536-point transform held by one wavefront.
 // Only the central N x N of each transformed G x G plane is read by the image pass, so the row
 // pass keeps the central `cols` output columns and the column pass transforms just those
 // columns and keeps the central `rows` outputs.
@@ -15,9 +15,7 @@
 namespace svdi {
 namespace {
 
-constexpr int kThreads = 256;
 constexpr int kMaxStages = 24;
-constexpr int kMaxRadix = 16;
 
 // Quotient q = n / d for 0 <= n < 2^27 and d <= 2^13 as (n * ceil(2^40 / d)) >> 40: the error
 // term n / 2^40 stays below 1 / d, so the floor is exact without an integer divide.
@@ -80,23 +78,62 @@ __device__ __forceinline__ void dft4(V* v) {
     v[3] = csub(y1, y3);
 }
 
-__device__ __forceinline__ void dft5(float2* v) {
-    // e^{2 pi i k / 5}: c1 = cos(2pi/5), c2 = cos(4pi/5), s1 = sin(2pi/5), s2 = sin(4pi/5)
-    const float c1 = 0.30901699437494742410f, c2 = -0.80901699437494742410f;
-    const float s1 = 0.95105651629515357212f, s2 = 0.58778525229247312917f;
-    const float2 a1 = cadd(v[1], v[4]), b1 = csub(v[1], v[4]);
-    const float2 a2 = cadd(v[2], v[3]), b2 = csub(v[2], v[3]);
+// cos and sin of 2 pi num / den, for constants.
+constexpr double turn_cos(int num, int den) {
+    num %= den;
+    if (2 * num > den) num = den - num;                // cos(-x) = cos x
+    const bool neg = 4 * num > den;                    // cos(pi - x) = -cos x
+    const double x = 6.283185307179586476925 * (neg ? 0.5 - static_cast<double>(num) / den : static_cast<double>(num) / den);
+    double term = 1.0, sum = 1.0;
+    for (int k = 1; k <= 12; ++k) {
+        term *= -x * x / ((2 * k - 1) * (2 * k));
+        sum += term;
+    }
+    return neg ? -sum : sum;
+}
+constexpr double turn_sin(int num, int den) { return turn_cos(4 * num + 3 * den, 4 * den); }   // sin x = cos(x - pi/2)
+
+// Odd prime P: out_k, out_{P-k} = v_0 + sum_j cos(2 pi j k / P) (v_j + v_{P-j}) +- i sum_j sin(2 pi j k / P)
+// (v_j - v_{P-j}).
+template <int P>
+struct TurnTable {
+    float c[P], s[P];
+    constexpr TurnTable() : c(), s() {
+        for (int i = 0; i < P; ++i) {
+            c[i] = static_cast<float>(turn_cos(i, P));
+            s[i] = static_cast<float>(turn_sin(i, P));
+        }
+    }
+};
+template <int P>
+__device__ __forceinline__ void dft_prime(float2* v) {
+    constexpr TurnTable<P> t;
+    constexpr int H = (P - 1) / 2;
+    float2 a[H], b[H];
     const float2 x0 = v[0];
-    const float2 m1 = make_float2(x0.x + c1 * a1.x + c2 * a2.x, x0.y + c1 * a1.y + c2 * a2.y);
-    const float2 m2 = make_float2(x0.x + c2 * a1.x + c1 * a2.x, x0.y + c2 * a1.y + c1 * a2.y);
-    // i * (s1 b1 + s2 b2) and i * (s2 b1 - s1 b2)
-    const float2 n1 = make_float2(s1 * b1.x + s2 * b2.x, s1 * b1.y + s2 * b2.y);
-    const float2 n2 = make_float2(s2 * b1.x - s1 * b2.x, s2 * b1.y - s1 * b2.y);
-    v[0] = make_float2(x0.x + a1.x + a2.x, x0.y + a1.y + a2.y);
-    v[1] = cadd(m1, mul_i(n1));
-    v[4] = csub(m1, mul_i(n1));
-    v[2] = cadd(m2, mul_i(n2));
-    v[3] = csub(m2, mul_i(n2));
+    float2 all = x0;
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+        a[j] = cadd(v[j + 1], v[P - 1 - j]);
+        b[j] = csub(v[j + 1], v[P - 1 - j]);
+        all = cadd(all, a[j]);
+    }
+    v[0] = all;
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+        float2 m = x0, n = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int j = 0; j < H; ++j) {
+            const int i = (j + 1) * k % P;
+            m.x += t.c[i] * a[j].x;
+            m.y += t.c[i] * a[j].y;
+            n.x += t.s[i] * b[j].x;
+            n.y += t.s[i] * b[j].y;
+        }
+        const float2 in = mul_i(n);
+        v[k] = cadd(m, in);
+        v[P - k] = csub(m, in);
+    }
 }
 
 template <class V>
@@ -119,78 +156,76 @@ __device__ __forceinline__ void dft8(V* v) {
     }
 }
 
-__device__ __forceinline__ void dft_generic(float2* v, int R, const float2* __restrict__ tw, int n) {
-    float2 y[kMaxRadix];
-    const int step = n / R;                 // e^{2 pi i q / R} = tw[q * n / R]
-    for (int k = 0; k < R; ++k) {
-        float2 acc = v[0];
-        for (int q = 1; q < R; ++q) acc = cadd(acc, cmul(v[q], tw[((q * k) % R) * step]));
-        y[k] = acc;
+template <int R, class V>
+__device__ __forceinline__ void dft_fixed(V* v);
+
+// R = A^2: X[k1 + A k2] = sum_{n2 < A} W_A^{n2 k2} (W_R^{n2 k1} sum_{n1 < A} W_A^{n1 k1} v[A n1 + n2]).
+template <int A>
+__device__ __forceinline__ void dft_square(float2* v) {
+    constexpr TurnTable<A * A> t;
+    float2 y[A][A];
+#pragma unroll
+    for (int n2 = 0; n2 < A; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < A; ++n1) y[n2][n1] = v[A * n1 + n2];
+        dft_fixed<A>(y[n2]);
+#pragma unroll
+        for (int k1 = 1; k1 < A; ++k1)
+            if (n2 != 0) y[n2][k1] = cmul(y[n2][k1], make_float2(t.c[n2 * k1], t.s[n2 * k1]));
     }
-    for (int k = 0; k < R; ++k) v[k] = y[k];
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+        float2 z[A];
+#pragma unroll
+        for (int n2 = 0; n2 < A; ++n2) z[n2] = y[n2][k1];
+        dft_fixed<A>(z);
+#pragma unroll
+        for (int k2 = 0; k2 < A; ++k2) v[k1 + A * k2] = z[k2];
+    }
+}
+
+// R = A B with A and B coprime (Good and Thomas): with n = B n1 + A n2 mod R and k = k1 mod A = k2 mod B,
+// W_R^{n k} = W_A^{n1 k1} W_B^{n2 k2}: no twiddles, so no roundings but those of the factors.
+template <int A, int B>
+__device__ __forceinline__ void dft_coprime(float2* v) {
+    float2 y[B][A];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < A; ++n1) y[n2][n1] = v[(B * n1 + A * n2) % (A * B)];
+        dft_fixed<A>(y[n2]);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+        float2 z[B];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) z[n2] = y[n2][k1];
+        dft_fixed<B>(z);
+#pragma unroll
+        for (int k = 0; k < A * B; ++k)
+            if (k % A == k1) v[k] = z[k % B];
+    }
 }
 
 template <int R, class V>
 __device__ __forceinline__ void dft_fixed(V* v) {
     if constexpr (R == 2) dft2(v);
-    else if constexpr (R == 3) dft3(v);
     else if constexpr (R == 4) dft4(v);
-    else if constexpr (R == 5) dft5(v);
-    else dft8(v);
+    else if constexpr (R == 8) dft8(v);
+    else if constexpr (R == 3) dft3(v);
+    else if constexpr (R == 5 || R == 7 || R == 11 || R == 13) dft_prime<R>(v);
+    else if constexpr (R == 16) dft_square<4>(v);
+    else if constexpr (R == 9) dft_square<3>(v);
+    else if constexpr (R == 15) dft_coprime<3, 5>(v);
+    else if constexpr (R == 12) dft_coprime<4, 3>(v);
+    else dft_coprime<2, R / 2>(v);                     // 6, 10, 14
 }
 
-// One Stockham stage of radix R over ntrans transforms of length n (LDS src -> LDS dst, each
-// transform `pn` float2 apart, padded): butterfly j reads src[j + r m], twiddles by
-// e^{+2 pi i (j mod ns) r / (ns R)} (table tw in LDS: tw[t] = e^{2 pi i t / n}), and writes
-// dst[(j / ns) ns R + (j mod ns) + r ns].
-template <int R>
-__device__ __forceinline__ void stage_fixed(const float2* src, float2* dst, int ntrans, int n, int pn,
-                                            int ns, FastDiv by_m, FastDiv by_ns, const float2* tw) {
-    const int m = n / R;
-    const int tstep = n / (ns * R);
-    const int total = ntrans * m;
-    for (int t = threadIdx.x; t < total; t += blockDim.x) {
-        const int tr = static_cast<int>(by_m.div(t));
-        const int j = t - tr * m;
-        const int jq = static_cast<int>(by_ns.div(j));
-        const int jm = j - jq * ns;
-        const float2* in = src + tr * pn;
-        float2* out = dst + tr * pn;
-        float2 v[R];
-        v[0] = in[pidx(j)];
-#pragma unroll
-        for (int r = 1; r < R; ++r) v[r] = cmul(in[pidx(j + r * m)], tw[jm * r * tstep]);
-        dft_fixed<R>(v);
-        const int d = jq * ns * R + jm;
-#pragma unroll
-        for (int r = 0; r < R; ++r) out[pidx(d + r * ns)] = v[r];
-    }
-}
-
-__device__ void stage_generic(const float2* src, float2* dst, int ntrans, int n, int pn, int ns, int R,
-                              FastDiv by_m, FastDiv by_ns, const float2* tw) {
-    const int m = n / R;
-    const int tstep = n / (ns * R);
-    const int total = ntrans * m;
-    for (int t = threadIdx.x; t < total; t += blockDim.x) {
-        const int tr = static_cast<int>(by_m.div(t));
-        const int j = t - tr * m;
-        const int jq = static_cast<int>(by_ns.div(j));
-        const int jm = j - jq * ns;
-        const float2* in = src + tr * pn;
-        float2* out = dst + tr * pn;
-        float2 v[kMaxRadix];
-        v[0] = in[pidx(j)];
-        for (int r = 1; r < R; ++r) v[r] = cmul(in[pidx(j + r * m)], tw[jm * r * tstep]);
-        dft_generic(v, R, tw, n);
-        const int d = jq * ns * R + jm;
-        for (int r = 0; r < R; ++r) out[pidx(d + r * ns)] = v[r];
-    }
-}
-
-// In-place form of a radix-R stage: every butterfly of the stage (at most kMaxB per thread) is
-// read and transformed into registers, then, after a barrier, written back to the same buffer.
-// Half the LDS of the ping-pong form, so twice the transforms per workgroup.  V: the type of the
+// One Stockham stage of radix R over ntrans transforms of length n in LDS, `pn` float2 apart and
+// padded: butterfly j reads element j + r m (m = n / R), times e^{+2 pi i (j mod ns) r / (ns R)} (table
+// tw in LDS: tw[t] = e^{2 pi i t / n}), and writes (j / ns) ns R + (j mod ns) + r ns.  In place: every
+// butterfly of the stage (at most kMaxB per thread) is read and transformed into registers, then,
+// after a barrier, written back to the same buffer.  V: the type of the
 // butterfly's arithmetic (double2 rounds once per stage, where values go back to LDS; FP64 runs at the
 // rate of plain FP32 here).
 constexpr int kMaxB = 4;
@@ -239,53 +274,18 @@ __device__ __forceinline__ void stage_inplace(float2* buf, int ntrans, int n, in
     __syncthreads();
 }
 
-// (double2: radices 2, 4 and 8 only.)
-template <class V = float2>
+// (Radices 4 and 8: factorize_pow2.)
+template <class V>
 __device__ void stockham_inplace(float2* buf, int ntrans, int pn, const FftStages& st, const float2* tw) {
     const int n = st.n;
     int ns = 1;
     for (int stage = 0; stage < st.count; ++stage) {
         const int R = st.radix[stage];
         const FastDiv bm = st.by_m[stage], bn = st.by_ns[stage];
-        switch (R) {
-            case 2: stage_inplace<2, V>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 3:
-                if constexpr (sizeof(V) == sizeof(float2)) stage_inplace<3, V>(buf, ntrans, n, pn, ns, bm, bn, tw);
-                break;
-            case 4: stage_inplace<4, V>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 5:
-                if constexpr (sizeof(V) == sizeof(float2)) stage_inplace<5, V>(buf, ntrans, n, pn, ns, bm, bn, tw);
-                break;
-            default: stage_inplace<8, V>(buf, ntrans, n, pn, ns, bm, bn, tw); break;
-        }
+        if (R == 4) stage_inplace<4, V>(buf, ntrans, n, pn, ns, bm, bn, tw);
+        else stage_inplace<8, V>(buf, ntrans, n, pn, ns, bm, bn, tw);
         ns *= R;
     }
-}
-
-// ntrans transforms of length n, `pn` float2 apart in src (LDS, padded).  Returns the buffer
-// that holds the result (src or dst).
-__device__ float2* stockham(float2* src, float2* dst, int ntrans, int pn, const FftStages& st,
-                            const float2* tw) {
-    const int n = st.n;
-    int ns = 1;
-    for (int stage = 0; stage < st.count; ++stage) {
-        const int R = st.radix[stage];
-        const FastDiv bm = st.by_m[stage], bn = st.by_ns[stage];
-        switch (R) {
-            case 2: stage_fixed<2>(src, dst, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 3: stage_fixed<3>(src, dst, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 4: stage_fixed<4>(src, dst, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 5: stage_fixed<5>(src, dst, ntrans, n, pn, ns, bm, bn, tw); break;
-            case 8: stage_fixed<8>(src, dst, ntrans, n, pn, ns, bm, bn, tw); break;
-            default: stage_generic(src, dst, ntrans, n, pn, ns, R, bm, bn, tw); break;
-        }
-        __syncthreads();
-        float2* tmp = src;
-        src = dst;
-        dst = tmp;
-        ns *= R;
-    }
-    return src;
 }
 
 // put(t, get(t)) for t = threadIdx.x, + blockDim.x, ... < n, with the gets of kCopyBatch
@@ -305,44 +305,125 @@ __device__ __forceinline__ void copy_batched(int n, Get&& get, Put&& put) {
     for (; t < n; t += step) put(t, get(t));
 }
 
-// LDS of a pass: the twiddle table (n float2), then two ping-pong buffers of ntrans padded
-// transforms.
 __device__ __forceinline__ const float2* load_twiddles(float2* lds, const float2* __restrict__ tw, int n) {
     copy_batched(n, [&](int t) { return tw[t]; }, [&](int t, float2 v) { lds[t] = v; });
     return lds;
 }
 
-// Row pass: planes [P][G][G] -> row_out [P][G][cols] (output columns col_lo .. col_lo+cols-1).
-// kInplace: radices 2/3/4/5/8 only, one LDS buffer, kInplaceThreads threads.
-template <bool kInplace>
-__global__ void __launch_bounds__(kInplace ? kInplaceThreads : kThreads)
-k_fft_rows(const float2* __restrict__ in, float2* __restrict__ out, FftStages st,
-           const float2* __restrict__ tw_g, int batch, int col_lo, int cols) {
-    extern __shared__ float2 lds[];
-    const int G = st.n;
-    const int pn = static_cast<int>(padded_len(G));
-    const float2* tw = load_twiddles(lds, tw_g, G);
-    float2* buf0 = lds + G;
-    float2* buf1 = kInplace ? buf0 : buf0 + batch * pn;
-    const size_t plane = blockIdx.y;
-    const int row0 = blockIdx.x * batch;
-    const int nrows = min(batch, G - row0);
-    const float2* src = in + (plane * G + row0) * static_cast<size_t>(G);
-    for (int r = 0; r < nrows; ++r)
-        copy_batched(G, [&](int c) { return src[static_cast<size_t>(r) * G + c]; },
-                     [&](int c, float2 v) { buf0[r * pn + pidx(c)] = v; });
-    __syncthreads();
-    const float2* res;
-    if constexpr (kInplace) {
-        stockham_inplace(buf0, nrows, pn, st, tw);
-        res = buf0;
-    } else {
-        res = stockham(buf0, buf1, nrows, pn, st, tw);
+// Barrier for data exchanged through LDS: global loads and stores stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Passes of the lengths without a kernel of their own.  A workgroup takes ntrans transforms (rows, or
+// neighbouring columns) through the Stockham stages; the first stage's butterflies are read from
+// memory and the last one's written to memory, so that a length of two to four stages goes through
+// LDS one to three times.  Bound by LDS traffic and index arithmetic, which go with the number of stages, and by
+// how many wavefronts hide them: radices of up to 16 in registers keep the stages few, and the registers of
+// one or two butterflies (kHoldLess or kHoldMore elements a thread, held between reading and writing, as a
+// stage is in place) keep the wavefronts many.  Rows + columns of eight planes, before (radices of up to 8,
+// every stage from and to LDS; 7 and above a loop over a private array) and now: 768^2 31 + 21 -> 21 + 15
+// us, 1500^2 103 + 81 -> 77 + 50, 2304^2 480 -> 133 + 173 (both), 3024^2 3590 -> 309 + 292 (both).
+constexpr int kHoldLess = 16, kHoldMore = 20;
+constexpr int kPassThreads = 1024;
+constexpr int kPassElems = 6200;                   // of a workgroup's transforms, if it can choose
+constexpr size_t kPassLds = 160 << 10;
+constexpr int kRadices[] = {16, 15, 14, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+
+// Padding of a pass's LDS: one float2 per 16, so that first stages with an even radix (stride R) spread
+// over the banks, and transforms an odd multiple of four apart, so that four neighbouring elements
+// of eight columns do.
+__device__ __forceinline__ int pass_idx(int i) { return i + (i >> 4); }
+__host__ __device__ inline int pass_len(int n) { return ((n + n / 16 + 1 + 3) & ~7) + 4; }
+
+template <int R, int kHold, bool kRows, class Get, class Put>
+__device__ __forceinline__ void pass_stage(float2* buf, int ntrans, int n, int pn, int ns, FastDiv by_m, FastDiv by_ns,
+                                           const float2* tw, bool first, bool last, Get&& get, Put&& put) {
+    constexpr int B = kHold / R;
+    const int m = n / R, tstep = n / (ns * R), total = ntrans * m;
+    const int threads = static_cast<int>(blockDim.x);
+    // (Opaque, so that no radix's index arithmetic is moved out of the loop over tiles, where those of
+    // all radices together would not fit the registers.)
+    int tid = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(tid));
+    float2 v[B][R];
+    int at[B], tr_of[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        const int t = tid + b * threads;
+        at[b] = -1;
+        if (t < total) {
+            // Rows: consecutive threads take consecutive elements; columns: consecutive columns.
+            const int tr = kRows ? static_cast<int>(by_m.div(t)) : t & (ntrans - 1);
+            const int j = kRows ? t - tr * m : t >> (31 - __builtin_clz(ntrans));
+            tr_of[b] = tr;
+            if (first) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) v[b][r] = get(tr, j + r * m);
+                at[b] = j * R;
+            } else {
+                const int jq = static_cast<int>(by_ns.div(j)), jm = j - jq * ns;
+                const float2* in = buf + tr * pn;
+                v[b][0] = in[pass_idx(j)];
+#pragma unroll
+                for (int r = 1; r < R; ++r) v[b][r] = cmul(in[pass_idx(j + r * m)], tw[jm * r * tstep]);
+                at[b] = jq * ns * R + jm;
+            }
+        }
     }
-    float2* dst = out + (plane * G + row0) * static_cast<size_t>(cols);
-    for (int r = 0; r < nrows; ++r)
-        for (int c = threadIdx.x; c < cols; c += blockDim.x)
-            dst[static_cast<size_t>(r) * cols + c] = res[r * pn + pidx(col_lo + c)];
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+        if (b * threads < total) dft_fixed<R>(v[b]);   // (the same for the whole workgroup)
+    if (last) {
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+            if (at[b] >= 0)
+#pragma unroll
+                for (int r = 0; r < R; ++r) put(tr_of[b], at[b] + r * ns, v[b][r]);
+        return;
+    }
+    lds_barrier();                                 // the stage (or the last tile) has been read
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+        if (at[b] >= 0)
+#pragma unroll
+            for (int r = 0; r < R; ++r) buf[tr_of[b] * pn + pass_idx(at[b] + r * ns)] = v[b][r];
+    lds_barrier();
+}
+
+template <int kHold, bool kRows, class Get, class Put>
+__device__ __forceinline__ void pass_transforms(float2* buf, int ntrans, const FftStages& st, const float2* tw, Get&& get,
+                                                Put&& put) {
+    const int n = st.n, pn = pass_len(n);
+    int ns = 1;
+    for (int stage = 0; stage < st.count; ++stage) {
+        const FastDiv bm = st.by_m[stage], bn = st.by_ns[stage];
+        const bool first = stage == 0, last = stage == st.count - 1;
+        const int R = st.radix[stage];
+        auto run = [&](auto radix) {
+            pass_stage<decltype(radix)::value, kHold, kRows>(buf, ntrans, n, pn, ns, bm, bn, tw, first, last, get, put);
+        };
+        switch (R) {
+            case 2: run(std::integral_constant<int, 2>()); break;
+            case 3: run(std::integral_constant<int, 3>()); break;
+            case 4: run(std::integral_constant<int, 4>()); break;
+            case 5: run(std::integral_constant<int, 5>()); break;
+            case 6: run(std::integral_constant<int, 6>()); break;
+            case 7: run(std::integral_constant<int, 7>()); break;
+            case 8: run(std::integral_constant<int, 8>()); break;
+            case 9: run(std::integral_constant<int, 9>()); break;
+            case 10: run(std::integral_constant<int, 10>()); break;
+            case 11: run(std::integral_constant<int, 11>()); break;
+            case 12: run(std::integral_constant<int, 12>()); break;
+            case 13: run(std::integral_constant<int, 13>()); break;
+            case 14: run(std::integral_constant<int, 14>()); break;
+            case 15: run(std::integral_constant<int, 15>()); break;
+            default: run(std::integral_constant<int, 16>()); break;
+        }
+        ns *= R;
+    }
 }
 
 // One 1536-point inverse transform per wavefront (G = 24 x 64), held in registers.  With
@@ -498,13 +579,6 @@ k_fft_rows_1536(const float2* __restrict__ in, float2* __restrict__ out, const f
                      const int kc = k - col_lo;
                      if (kc >= 0 && kc < cols) dst[mid.col(kc)] = v;
                  });
-}
-
-// Barrier for data exchanged through LDS: global loads and stores stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // Column pass of the 1536-point transforms of column blocks (s sub-planes per plane), bound by memory:
@@ -701,44 +775,53 @@ k_fft_rows_6144(const float2* __restrict__ in, float2* __restrict__ out, const f
     }
 }
 
-// Column pass: row_out [P][G][cols] -> out [P][rows][cols] (output rows row_lo .. row_lo+rows-1).
-// One workgroup per (plane, strip of `width` columns), strips ordered XCD-locally.
-template <bool kInplace>
-__global__ void __launch_bounds__(kInplace ? kInplaceThreads : kThreads)
-k_fft_cols(const float2* __restrict__ in, float2* __restrict__ out, FftStages st,
-           const float2* __restrict__ tw_g, int width, int cols, int row_lo, int rows, int strips) {
+// Row pass of the other lengths: planes [P][G][G] -> row_out [P][G][cols] (output columns col_lo ..
+// col_lo + cols - 1), `batch` rows of the P G at a time.  Workgroups walk the tiles, so that the twiddle
+// table is loaded once for several.
+template <int kHold>
+__global__ void __launch_bounds__(kPassThreads)
+k_fft_rows(const float2* __restrict__ in, float2* __restrict__ out, FftStages st, const float2* __restrict__ tw_g,
+           int total_rows, int batch, int tiles, int col_lo, int cols) {
     extern __shared__ float2 lds[];
     const int G = st.n;
-    const int pn = static_cast<int>(padded_len(G));
     const float2* tw = load_twiddles(lds, tw_g, G);
-    float2* buf0 = lds + G;
-    float2* buf1 = kInplace ? buf0 : buf0 + width * pn;
-    const int tile = xcd_local_tile(blockIdx.x, gridDim.x);
-    const size_t plane = tile / strips;
-    const int c0 = (tile - static_cast<int>(plane) * strips) * width;
-    const int nc = min(width, cols - c0);
-    const float2* src = in + plane * G * static_cast<size_t>(cols) + c0;
-    copy_batched(G * nc,
-                 [&](int t) {
-                     const int r = t / nc, c = t - r * nc;
-                     return src[static_cast<size_t>(r) * cols + c];
-                 },
-                 [&](int t, float2 v) {
-                     const int r = t / nc, c = t - r * nc;
-                     buf0[c * pn + pidx(r)] = v;
-                 });
-    __syncthreads();
-    const float2* res;
-    if constexpr (kInplace) {
-        stockham_inplace(buf0, nc, pn, st, tw);
-        res = buf0;
-    } else {
-        res = stockham(buf0, buf1, nc, pn, st, tw);
+    float2* buf = lds + G;
+    lds_barrier();
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int row0 = tile * batch;
+        const float2* src = in + static_cast<size_t>(row0) * G;
+        float2* dst = out + static_cast<size_t>(row0) * cols - col_lo;
+        pass_transforms<kHold, true>(buf, min(batch, total_rows - row0), st, tw,
+                              [&](int tr, int i) { return src[static_cast<size_t>(tr) * G + i]; },
+                              [&](int tr, int k, float2 v) {
+                                  if (k >= col_lo && k < col_lo + cols) dst[static_cast<size_t>(tr) * cols + k] = v;
+                              });
     }
-    float2* dst = out + plane * rows * static_cast<size_t>(cols) + c0;
-    for (int t = threadIdx.x; t < rows * nc; t += blockDim.x) {
-        const int r = t / nc, c = t - r * nc;
-        dst[static_cast<size_t>(r) * cols + c] = res[c * pn + pidx(row_lo + r)];
+}
+
+// Column pass: row_out [P][G][cols] -> out [P][rows][cols] (output rows row_lo .. row_lo + rows - 1).  A
+// tile is a strip of `width` (a power of two) columns of a plane, dealt XCD-locally; the last strip of a
+// plane repeats its last column in place of those past the end.
+template <int kHold>
+__global__ void __launch_bounds__(kPassThreads)
+k_fft_cols(const float2* __restrict__ in, float2* __restrict__ out, FftStages st, const float2* __restrict__ tw_g,
+           int width, int strips, int tiles, int cols, int row_lo, int rows) {
+    extern __shared__ float2 lds[];
+    const int G = st.n;
+    const float2* tw = load_twiddles(lds, tw_g, G);
+    float2* buf = lds + G;
+    lds_barrier();
+    for (int tile = xcd_local_tile(blockIdx.x, gridDim.x); tile < tiles; tile += gridDim.x) {
+        const int plane = tile / strips, c0 = (tile - plane * strips) * width;
+        const float2* src = in + plane * static_cast<size_t>(G) * cols + c0;
+        float2* dst = out + plane * static_cast<size_t>(rows) * cols + c0;
+        const int nc = cols - c0;
+        pass_transforms<kHold, false>(buf, width, st, tw,
+                               [&](int tr, int i) { return src[static_cast<size_t>(i) * cols + min(tr, nc - 1)]; },
+                               [&](int tr, int k, float2 v) {
+                                   const int r = k - row_lo;
+                                   if (r >= 0 && r < rows && tr < nc) dst[static_cast<size_t>(r) * cols + tr] = v;
+                               });
     }
 }
 
@@ -920,20 +1003,37 @@ void stage_divisors(FftStages& st) {
     }
 }
 
+// n in as few of the radices as do, of those the ones with the smallest sum, odd ones first (the first
+// stage's LDS writes, a stride of its radix apart, then meet no bank twice).  False: n has a prime factor above
+// 13 or is out of range.
+constexpr int kPassMax = 8192;                     // (twiddles and one transform: 134 KB of LDS)
 bool factorize(int n, FftStages& st) {
-    st.n = n;
-    st.count = 0;
-    int m = n;
-    const int pref[] = {8, 4, 2, 3, 5, 7, 11, 13};
-    for (int r : pref) {
-        while (m % r == 0 && m > 1) {
-            if (st.count == kMaxStages) return false;
-            st.radix[st.count++] = r;
-            m /= r;
+    if (n < 2 || n > kPassMax) return false;
+    int best[kMaxStages], pick[kMaxStages], best_count = kMaxStages, best_sum = 0;
+    auto search = [&](auto&& self, int rest, int depth, int sum, size_t from) -> void {
+        if (rest == 1) {
+            if (depth < best_count || (depth == best_count && sum < best_sum)) {
+                best_count = depth;
+                best_sum = sum;
+                std::copy(pick, pick + depth, best);
+            }
+            return;
         }
-    }
+        if (depth == best_count || depth + 1 == kMaxStages) return;
+        for (size_t i = from; i < sizeof kRadices / sizeof kRadices[0]; ++i) {
+            if (rest % kRadices[i] != 0) continue;
+            pick[depth] = kRadices[i];
+            self(self, rest / kRadices[i], depth + 1, sum + kRadices[i], i);
+        }
+    };
+    search(search, n, 0, 0, 0);
+    if (best_count == kMaxStages) return false;
+    std::stable_partition(best, best + best_count, [](int r) { return r % 2 != 0; });
+    st.n = n;
+    st.count = best_count;
+    std::copy(best, best + best_count, st.radix);
     stage_divisors(st);
-    return m == 1 && n <= 8192;
+    return true;
 }
 
 // n = 2^m >= 16 in radices 8 and 4 only: 8 8 4 4 for 8 8 8 2, so that twice the transforms fit a
@@ -1078,10 +1178,7 @@ void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size
         SVDI_LAUNCH_CHECK();
         return;
     }
-    const size_t per = 2 * padded_len(G) * sizeof(float2);     // one transform, ping-pong
-    const size_t twb = G * sizeof(float2);
-    const bool ok = factorize(static_cast<int>(G), st) && twb + per <= 160 * 1024;
-    if (!ok) {
+    if (!factorize(static_cast<int>(G), st)) {
         dim3 gr(static_cast<unsigned>((cols + 127) / 128), static_cast<unsigned>(G), static_cast<unsigned>(P));
         k_dft_rows_naive<<<gr, 128, 0, ctx->stream>>>(planes, row_out, static_cast<int>(G), tw,
                                                       static_cast<int>(col_lo), static_cast<int>(cols));
@@ -1093,45 +1190,59 @@ void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size
         SVDI_LAUNCH_CHECK();
         return;
     }
-    // In-place form when every radix has a fixed kernel and a stage's butterflies for at least
-    // one transform fit kMaxB per thread: transforms per workgroup = min over stages of
-    // kMaxB * threads / m, capped by 64 KB of LDS.
-    bool inplace = true;
-    int fit = 16;
+    // Transforms per workgroup: about kPassElems elements, so that two workgroups and more share a CU and one's
+    // loads run beside the other's stages; columns at least four (32-byte row segments) unless the LDS does
+    // not hold them; fewer where the workgroups would not fill the chip twice.  The threads: up to 512 with a
+    // butterfly or so each, more only where 512 could not hold a stage.
+    const int n = static_cast<int>(G);
+    int held[2] = {kHoldLess, kHoldMore};          // elements per thread, the least of the stages
     for (int i = 0; i < st.count; ++i) {
-        const int R = st.radix[i];
-        if (R != 2 && R != 3 && R != 4 && R != 5 && R != 8) inplace = false;
-        fit = std::min(fit, kMaxB * kInplaceThreads / (static_cast<int>(G) / R));
+        held[0] = std::min(held[0], kHoldLess / st.radix[i] * st.radix[i]);
+        held[1] = std::min(held[1], kHoldMore / st.radix[i] * st.radix[i]);
     }
-    const size_t one = padded_len(G) * sizeof(float2);
-    if (inplace && fit >= 1) {
-        fit = static_cast<int>(std::max<size_t>(1, std::min<size_t>(fit, (64 * 1024 > twb ? (64 * 1024 - twb) / one : 1))));
-    } else {
-        inplace = false;
-        const size_t budget = 128 * 1024;
-        const size_t room = budget > twb ? (budget - twb) / per : 0;
-        fit = static_cast<int>(std::max<size_t>(1, std::min<size_t>(16, room)));
-    }
-    const int batch = fit, width = fit;
-    const size_t lds = twb + static_cast<size_t>(fit) * (inplace ? one : per);
-    const int threads = inplace ? kInplaceThreads : kThreads;
-    auto rows_fn = inplace ? &k_fft_rows<true> : &k_fft_rows<false>;
-    auto cols_fn = inplace ? &k_fft_cols<true> : &k_fft_cols<false>;
-    allow_dynamic_lds(reinterpret_cast<const void*>(rows_fn), lds);
-    allow_dynamic_lds(reinterpret_cast<const void*>(cols_fn), lds);
-    {
-        dim3 gr(static_cast<unsigned>((G + batch - 1) / batch), static_cast<unsigned>(P));
-        rows_fn<<<gr, threads, lds, ctx->stream>>>(planes, row_out, st, tw, batch, static_cast<int>(col_lo),
-                                                   static_cast<int>(cols));
-    }
-    SVDI_LAUNCH_CHECK();
-    {
-        const int strips = static_cast<int>((cols + width - 1) / width);
-        const unsigned gc = static_cast<unsigned>(strips * P);
-        cols_fn<<<gc, threads, lds, ctx->stream>>>(row_out, out, st, tw, width, static_cast<int>(cols),
-                                                   static_cast<int>(row_lo), static_cast<int>(rows), strips);
-    }
-    SVDI_LAUNCH_CHECK();
+    const size_t one = static_cast<size_t>(pass_len(n)) * sizeof(float2), twb = G * sizeof(float2);
+    auto lds_of = [&](int ntrans) { return twb + ntrans * one; };
+    auto fit = [&](int most, int least, size_t transforms) {
+        int ntrans = most;
+        while (ntrans > least && (ntrans * n > kPassElems || transforms / ntrans < 2 * static_cast<size_t>(ctx->cu_count)))
+            ntrans /= 2;
+        while (ntrans > 1 && (ntrans * n > kPassThreads * std::max(held[0], held[1]) || lds_of(ntrans) > kPassLds)) ntrans /= 2;
+        return ntrans;
+    };
+    struct Shape {
+        int threads;
+        bool more;                                 // kHoldMore
+    };
+    auto shape_of = [&](int ntrans) {
+        const int elems = ntrans * n;
+        Shape s = {128, false};
+        while (s.threads < 512 && elems > s.threads * 8) s.threads *= 2;
+        if (elems > s.threads * held[0] && elems <= s.threads * held[1]) s.more = true;
+        while (elems > s.threads * held[s.more]) {
+            s.more = false;
+            s.threads *= 2;
+            if (s.threads == kPassThreads && elems > s.threads * held[0]) s.more = true;
+        }
+        return s;
+    };
+    auto grid_of = [&](int tiles, int ntrans, int threads) {
+        const int per_cu = static_cast<int>(std::min<size_t>(kPassLds / lds_of(ntrans), 2048 / threads));
+        return static_cast<unsigned>(std::min(tiles, std::max(1, ctx->cu_count * per_cu)));
+    };
+    const int c_lo = static_cast<int>(col_lo), nc = static_cast<int>(cols), nr = static_cast<int>(rows);
+    auto launch = [&](auto less, auto more, int ntrans, int tiles, auto... args) {
+        const Shape shape = shape_of(ntrans);
+        const auto kernel = shape.more ? more : less;
+        allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds_of(ntrans));
+        kernel<<<grid_of(tiles, ntrans, shape.threads), shape.threads, lds_of(ntrans), ctx->stream>>>(args...);
+        SVDI_LAUNCH_CHECK();
+    };
+    const int total_rows = static_cast<int>(P * G), batch = fit(16, 1, P * G), row_tiles = (total_rows + batch - 1) / batch;
+    launch(&k_fft_rows<kHoldLess>, &k_fft_rows<kHoldMore>, batch, row_tiles, planes, row_out, st, tw, total_rows, batch,
+           row_tiles, c_lo, nc);
+    const int width = fit(8, 4, P * cols), strips = (nc + width - 1) / width, col_tiles = strips * static_cast<int>(P);
+    launch(&k_fft_cols<kHoldLess>, &k_fft_cols<kHoldMore>, width, col_tiles, static_cast<const float2*>(row_out), out, st, tw,
+           width, strips, col_tiles, nc, static_cast<int>(row_lo), nr);
 }
 
 }  // namespace svdi
