@@ -1,6 +1,8 @@
 // Exclusive scan of a u32 array on the device (counts -> offsets), shared by the binning passes
-// of the gridders: per-block scans of 4096 elements, a one-block scan of the block totals, then
-// the block offsets added; out[n] receives the total and `cursor` (optional) a copy of out.
+// of the gridders: per-block scans of 4096 elements, then the block offsets added, each block
+// summing the totals before it itself (a one-block scan of the totals between the two, 2 to 5 us and a
+// launch, is left for more than kScanSelf blocks); out[n] receives the total and `cursor` (optional) a
+// copy of out.  One block is one launch.
 #pragma once
 
 #include "svdi_internal.hpp"
@@ -35,7 +37,8 @@ __device__ __forceinline__ uint32_t block_scan_1024(uint32_t v, uint32_t* s_wave
 }
 
 __global__ void __launch_bounds__(1024)
-k_scan_blocks(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint32_t* __restrict__ sums, uint32_t n) {
+k_scan_blocks(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint32_t* __restrict__ sums, uint32_t n,
+              uint32_t* __restrict__ cursor) {
     __shared__ uint32_t s_wave[16];
     const size_t base = static_cast<size_t>(blockIdx.x) * kScanBlock + threadIdx.x * kScanPer;
     uint32_t v[kScanPer], tot = 0;
@@ -46,10 +49,16 @@ k_scan_blocks(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint3
     const uint32_t incl = block_scan_1024(tot, s_wave);
     uint32_t run = incl - tot;
     for (int j = 0; j < kScanPer; ++j) {
-        if (base + j < n) out[base + j] = run;
+        if (base + j < n) {
+            out[base + j] = run;
+            if (cursor != nullptr && gridDim.x == 1) cursor[base + j] = run;
+        }
         run += v[j];
     }
-    if (threadIdx.x == 1023) sums[blockIdx.x] = incl;
+    if (threadIdx.x == 1023) {
+        sums[blockIdx.x] = incl;
+        if (gridDim.x == 1) out[n] = incl;
+    }
 }
 
 __global__ void __launch_bounds__(1024)
@@ -69,14 +78,33 @@ k_scan_sums(uint32_t* __restrict__ sums, int nblocks, uint32_t* __restrict__ gra
     if (threadIdx.x == 1023) *grand_total = incl;
 }
 
-__global__ void __launch_bounds__(256)
-k_scan_add(uint32_t* __restrict__ out, const uint32_t* __restrict__ sums, uint32_t n, uint32_t* __restrict__ cursor) {
-    const size_t i = blockIdx.x * static_cast<size_t>(256) + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t v = out[i] + sums[i / kScanBlock];
-    out[i] = v;
-    if (cursor != nullptr) cursor[i] = v;
+// sums: the blocks' totals, or (scanned) their exclusive scan with out[n] already written.
+__global__ void __launch_bounds__(1024)
+k_scan_add(uint32_t* __restrict__ out, const uint32_t* __restrict__ sums, uint32_t n, uint32_t* __restrict__ cursor, bool scanned) {
+    __shared__ uint32_t s_part[16];
+    uint32_t before = 0;
+    if (scanned) {
+        before = sums[blockIdx.x];
+    } else {
+        for (uint32_t i = threadIdx.x; i < blockIdx.x; i += 1024) before += sums[i];
+        for (int d = 32; d >= 1; d >>= 1) before += __shfl_xor(before, d, 64);
+        if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = before;
+        __syncthreads();
+        before = 0;
+        for (int k = 0; k < 16; ++k) before += s_part[k];
+        if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = before + sums[blockIdx.x];
+    }
+    const size_t base = static_cast<size_t>(blockIdx.x) * kScanBlock + threadIdx.x;
+    for (int j = 0; j < kScanPer; ++j) {
+        const size_t i = base + 1024 * j;
+        if (i >= n) break;
+        const uint32_t v = out[i] + before;
+        out[i] = v;
+        if (cursor != nullptr) cursor[i] = v;
+    }
 }
+
+constexpr size_t kScanSelf = 2048;
 
 inline size_t scan_blocks(size_t n) { return (n + kScanBlock - 1) / kScanBlock; }
 
@@ -87,11 +115,15 @@ inline void launch_exclusive_scan(svdi_context* ctx, const uint32_t* in, uint32_
     const size_t nb = scan_blocks(n);
     if (nb > (1ull << 30)) throw UnsupportedError("scan too large");
     const uint32_t n32 = static_cast<uint32_t>(n);
-    k_scan_blocks<<<static_cast<unsigned>(nb), 1024, 0, ctx->stream>>>(in, out, sums, n32);
+    k_scan_blocks<<<static_cast<unsigned>(nb), 1024, 0, ctx->stream>>>(in, out, sums, n32, cursor);
     SVDI_LAUNCH_CHECK();
-    k_scan_sums<<<1, 1024, 0, ctx->stream>>>(sums, static_cast<int>(nb), out + n);
-    SVDI_LAUNCH_CHECK();
-    k_scan_add<<<static_cast<unsigned>((n + 255) / 256), 256, 0, ctx->stream>>>(out, sums, n32, cursor);
+    if (nb == 1) return;
+    const bool scanned = nb > kScanSelf;
+    if (scanned) {
+        k_scan_sums<<<1, 1024, 0, ctx->stream>>>(sums, static_cast<int>(nb), out + n);
+        SVDI_LAUNCH_CHECK();
+    }
+    k_scan_add<<<static_cast<unsigned>(nb), 1024, 0, ctx->stream>>>(out, sums, n32, cursor, scanned);
     SVDI_LAUNCH_CHECK();
 }
 

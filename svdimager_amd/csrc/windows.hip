@@ -646,8 +646,8 @@ __device__ __forceinline__ WinRange window_range(const uint32_t* __restrict__ bo
 // coop_cap for pieces; the last class also the smaller and empty ones), so that the wavefronts
 // and workgroups finish together.
 // icount: [kItemClasses][nwin_total] wavefront items, [kItemClasses][2 nwin_total] pieces of the
-// halves, [2 nwin_total] partial slots; one exclusive scan gives the queue positions and slot
-// numbers.  totals[0] = records, [1] = wavefront items, [2] = (unused), [3] = pieces,
+// halves, [2 nwin_total] partial slots, [nwin_total] windows that k_win_reduce completes; one exclusive
+// scan gives the queue positions, slot numbers and places in k_win_reduce's list.  totals[0] = records, [1] = wavefront items, [2] = (unused), [3] = pieces,
 // [4] = max |v| bits, [5] = piece queue head, [6] = windows that k_win_reduce completes.
 constexpr int kItemClasses = 8;
 constexpr uint32_t kCoopMinDefault = 1024;
@@ -716,9 +716,14 @@ __device__ __forceinline__ WinSplit window_split(const uint32_t* __restrict__ bo
     return s;
 }
 
+// The queue classes of a window's wavefront item (-1: it has none) and of a dense half's pieces.
+__device__ __forceinline__ int wave_item_class(const WinGeom& wg, const WinSplit& s) {
+    return s.s_count > 0 || !s.reduced() ? item_class(s.s_count, 3 * wg.coop_min) : -1;
+}
+__device__ __forceinline__ int piece_class(const WinGeom& wg, const Pieces& p) { return item_class(p.per, wg.coop_cap); }
+
 __global__ void __launch_bounds__(256)
-k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __restrict__ icount,
-                  uint32_t* __restrict__ multi, uint32_t* __restrict__ totals) {
+k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __restrict__ icount, uint32_t* __restrict__ totals) {
     const int w = blockIdx.x * 256 + threadIdx.x;
     const int nwt = wg.nwin_total;
     if (w == 0) totals[0] = boff[wg.nbins];
@@ -726,7 +731,7 @@ k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __res
     uint32_t end;
     const WinRange x = window_range(boff, wg, w, end);
     const WinSplit s = window_split(boff, wg, w, x, end);
-    const int wcls = s.s_count > 0 || !s.reduced() ? item_class(s.s_count, 3 * wg.coop_min) : -1;
+    const int wcls = wave_item_class(wg, s);
     for (int k = 0; k < kItemClasses; ++k) icount[k * nwt + w] = k == wcls ? 1u : 0u;
     uint32_t* half = icount + kItemClasses * nwt;
     for (int j = 0; j < 2; ++j) {
@@ -734,12 +739,12 @@ k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __res
         Pieces p = {0u, 0u};
         if (s.dense[j]) {
             p = dense_pieces(wg, s.h[j + 1] - s.h[j]);
-            pcls = item_class(p.per, wg.coop_cap);
+            pcls = piece_class(wg, p);
         }
         for (int k = 0; k <= kItemClasses; ++k)
             half[(2 * k + j) * nwt + w] = k == pcls || k == kItemClasses ? p.count : 0u;
     }
-    if (s.reduced()) multi[atomicAdd(&totals[6], 1u)] = static_cast<uint32_t>(w);
+    half[(2 * kItemClasses + 2) * nwt + w] = s.reduced() ? 1u : 0u;
 }
 
 // A window that k_win_reduce completes: the partial slots of the halves that reach it (its lower
@@ -750,75 +755,83 @@ struct WReduce {
     uint32_t first[6], count[6];
 };
 
-// One thread per item: its (queue, class, window) entry of the counts is found by binary search
-// over the offsets; and one thread per window that k_win_reduce completes.
+// kItemLanes threads per window write its items at the places that the counts' offsets give them, the
+// first one the wavefront item and, for a window that k_win_reduce completes, its entry there.  Bound by
+// latency: two rounds of loads that no cache line serves twice, so few threads per window (SKA-Low
+// snapshot, 9,216 windows: 11 us with two, 18 with eight; a thread per item that looks its window up by
+// binary search over the offsets is a chain of 18 loads, 16 us).
+constexpr int kItemLanes = 2;
 __global__ void __launch_bounds__(256)
-k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__ ioff,
-                 const uint32_t* __restrict__ multi, WinGeom wg, WItem* __restrict__ items, uint32_t max_items,
-                 WReduce* __restrict__ red, uint32_t* __restrict__ totals) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__ ioff, WinGeom wg, WItem* __restrict__ items,
+                 uint32_t max_items, WReduce* __restrict__ red, uint32_t* __restrict__ totals) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int w = t / kItemLanes, sub = t % kItemLanes;
     const int nwt = wg.nwin_total;
     const int n = 3 * kItemClasses * nwt;
-    if (i < totals[6]) {                        // (a window is listed at most once: i < nwt)
-        const int w = static_cast<int>(multi[i]);
-        uint32_t end;
-        const WinRange x = window_range(boff, wg, w, end);
-        const WinSplit s = window_split(boff, wg, w, x, end);
-        WReduce r;
-        r.win = w;
-        r.add = s.s_count > 0 ? 1 : 0;
-        // (n + j nwt + w: the slots of half j of window w.)
-        const uint32_t records[6] = {s.dense[0] ? s.h[1] - s.h[0] : 0u, s.dense[1] ? s.h[2] - s.h[1] : 0u,
-                                     s.up, s.left[0], s.left[1], s.up_left};
-        const int at[6] = {n + w, n + nwt + w, n + nwt + w - wg.nw, n + w - 1, n + nwt + w - 1, n + nwt + w - wg.nw - 1};
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            r.count[k] = records[k] != 0 ? dense_pieces(wg, records[k]).count : 0u;
-            r.first[k] = records[k] != 0 ? ioff[at[k]] - ioff[n] : 0u;
-        }
-        red[i] = r;
-    }
-    const uint32_t nwave = ioff[kItemClasses * nwt];
-    const uint32_t nitems = min(ioff[n], max_items);
-    if (i == 0) {
-        totals[1] = min(nwave, nitems);
-        totals[3] = nitems - min(nwave, nitems);
-    }
-    if (i >= nitems) return;
-    int lo = 0, hi = n;                         // largest j with ioff[j] <= i
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) / 2;
-        if (ioff[mid] <= i) lo = mid;
-        else hi = mid;
-    }
-    const int row = lo / nwt;                   // wavefront class, then kItemClasses + 2 class + half
-    const int w = lo - row * nwt;
+    if (w >= nwt) return;
     uint32_t end;
     const WinRange x = window_range(boff, wg, w, end);
     const WinSplit s = window_split(boff, wg, w, x, end);
-    WItem t;
-    t.win = w;
+    // Every offset that the window can need is requested at once (at a valid place where it does not need it),
+    // not one behind another.  (n + j nwt + w: the slots of half j of window w.)
+    const uint32_t records[6] = {s.dense[0] ? s.h[1] - s.h[0] : 0u, s.dense[1] ? s.h[2] - s.h[1] : 0u,
+                                 s.up, s.left[0], s.left[1], s.up_left};
+    const int at[6] = {n + w, n + nwt + w, n + nwt + w - wg.nw, n + w - 1, n + nwt + w - 1, n + nwt + w - wg.nw - 1};
+    uint32_t slots[6], queue[2];
 #pragma unroll
-    for (int j = 0; j < kMaxClasses; ++j) t.bnd[j] = static_cast<int>(x.bnd[j]);
-    t.start = static_cast<int>(s.s0);
-    t.count = static_cast<int>(s.s_count);
-    t.hole = static_cast<int>(s.hole);
-    t.hole_len = static_cast<int>(s.hole_len);
-    t.slot = -1;
-    t.half = 0;
-    t.skip = s.skip();
-    if (row >= kItemClasses) {
-        const int j = (row - kItemClasses) & 1;
-        const uint32_t first = j ? s.h[1] : s.h[0], records = (j ? s.h[2] : s.h[1]) - first;
-        const Pieces p = dense_pieces(wg, records);
-        const uint32_t q = i - ioff[lo];
-        t.start = static_cast<int>(first + q * p.per);
-        t.count = static_cast<int>(min(p.per, records - q * p.per));
-        t.slot = static_cast<int>(ioff[n + j * nwt + w] - ioff[n] + q);
-        t.half = j;
-        t.skip = (s.skip() >> (j + 1)) & 1;
+    for (int k = 0; k < 6; ++k) slots[k] = ioff[records[k] != 0 ? at[k] : n];
+    Pieces pieces[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        pieces[j] = dense_pieces(wg, records[j]);
+        queue[j] = ioff[records[j] != 0 ? (kItemClasses + 2 * piece_class(wg, pieces[j]) + j) * nwt + w : n];
     }
-    items[i] = t;
+    const int wcls = wave_item_class(wg, s);
+    const uint32_t wave_at = ioff[wcls >= 0 ? wcls * nwt + w : n], slot0 = ioff[n], red0 = ioff[n + 2 * nwt];
+    const uint32_t red_at = ioff[n + 2 * nwt + w];
+    if (sub == 0 && s.reduced()) {
+        WReduce r;
+        r.win = w;
+        r.add = s.s_count > 0 ? 1 : 0;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            r.count[k] = records[k] != 0 ? dense_pieces(wg, records[k]).count : 0u;
+            r.first[k] = records[k] != 0 ? slots[k] - slot0 : 0u;
+        }
+        red[red_at - red0] = r;
+    }
+    WItem it;
+    it.win = w;
+#pragma unroll
+    for (int j = 0; j < kMaxClasses; ++j) it.bnd[j] = static_cast<int>(x.bnd[j]);
+    it.hole = static_cast<int>(s.hole);
+    it.hole_len = static_cast<int>(s.hole_len);
+    if (sub == 0 && wcls >= 0) {
+        it.start = static_cast<int>(s.s0);
+        it.count = static_cast<int>(s.s_count);
+        it.slot = -1;
+        it.half = 0;
+        it.skip = s.skip();
+        if (wave_at < max_items) items[wave_at] = it;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        if (records[j] == 0) continue;
+        it.half = j;
+        it.skip = (s.skip() >> (j + 1)) & 1;
+        for (uint32_t q = sub; q < pieces[j].count; q += kItemLanes) {
+            it.start = static_cast<int>(s.h[j] + q * pieces[j].per);
+            it.count = static_cast<int>(min(pieces[j].per, records[j] - q * pieces[j].per));
+            it.slot = static_cast<int>(slots[j] - slot0 + q);
+            if (queue[j] + q < max_items) items[queue[j] + q] = it;
+        }
+    }
+    if (t == 0) {
+        const uint32_t nwave = ioff[kItemClasses * nwt], nitems = min(slot0, max_items);
+        totals[1] = min(nwave, nitems);
+        totals[3] = nitems - min(nwave, nitems);
+        totals[6] = ioff[n + 3 * nwt] - red0;
+    }
 }
 
 // Partial slots: [term][kDenseRows rows][kDenseCols columns] from the half's first row and the
@@ -2071,14 +2084,12 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     uint32_t* blocktot = blockhist + nhist;
     uint16_t* blockcount16 = count16 ? reinterpret_cast<uint16_t*>(blocktot + ntot) : nullptr;
     uint32_t* boff = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinOffsets, (nbins + 8) * sizeof(uint32_t)));
-    // The coarse bins' offsets, or those of the bins themselves; cursors (without LDS histograms); the
-    // windows with several pieces; segment sums [kBinSegs][lbins].
+    // Cursors (without LDS histograms); segment sums [kBinSegs][lbins]; the coarse bins' offsets.
     uint32_t* cursor = static_cast<uint32_t*>(ctx->ws.get(
-        Workspace::kBinCursor, (lbins + 8 + nwt + (wg.use_lds ? kBinSegs * lbins : 0) + (coarse ? lbins + 8 : 0)) * sizeof(uint32_t)));
-    uint32_t* multi = cursor + lbins + 8;
-    uint32_t* segsum = multi + nwt;
+        Workspace::kBinCursor, (lbins + 8 + (wg.use_lds ? kBinSegs * lbins : 0) + (coarse ? lbins + 8 : 0)) * sizeof(uint32_t)));
+    uint32_t* segsum = cursor + lbins + 8;
     uint32_t* coff = coarse ? segsum + (wg.use_lds ? kBinSegs * lbins : 0) : boff;
-    const size_t ncounts = (3 * kItemClasses + 2) * nwt;
+    const size_t ncounts = (3 * kItemClasses + 3) * nwt;
     uint32_t* sums = static_cast<uint32_t*>(
         ctx->ws.get(Workspace::kScanSums, scan_blocks(std::max(lbins, ncounts)) * sizeof(uint32_t)));
     uint32_t* icount = static_cast<uint32_t*>(ctx->ws.get(Workspace::kItemCounts, (ncounts + 8) * sizeof(uint32_t)));
@@ -2187,11 +2198,11 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
                                                                         sub_counts, sub_counts + nsub, boff, rec, limit);
         SVDI_LAUNCH_CHECK();
     }
-    k_win_item_counts<<<static_cast<unsigned>((nwt + 255) / 256), 256, 0, ctx->stream>>>(boff, wg, icount, multi, totals);
+    k_win_item_counts<<<static_cast<unsigned>((nwt + 255) / 256), 256, 0, ctx->stream>>>(boff, wg, icount, totals);
     SVDI_LAUNCH_CHECK();
     launch_exclusive_scan(ctx, icount, ioff, nullptr, sums, ncounts);
-    k_win_item_write<<<static_cast<unsigned>((max_items + 255) / 256), 256, 0, ctx->stream>>>(
-        boff, ioff, multi, wg, items, static_cast<uint32_t>(max_items), red, totals);
+    k_win_item_write<<<static_cast<unsigned>((kItemLanes * nwt + 255) / 256), 256, 0, ctx->stream>>>(
+        boff, ioff, wg, items, static_cast<uint32_t>(max_items), red, totals);
     SVDI_LAUNCH_CHECK();
 
     WindowJob job;
