@@ -656,41 +656,65 @@ k_fft_cols_1536(const float2* __restrict__ in, float2* __restrict__ out, const f
 // b_n = (x_n - x_{n + 1536}) W^n, stored as row n of the plane's two sub-planes (the columns col_lo ..
 // col_lo + cols - 1).  (Decimation in frequency, whose loads are whole runs, took 1.61 ms for 1.51: its
 // extra LDS exchange costs more than the half-used lines, which the second wavefront finds in L2.)
-__global__ void __launch_bounds__(256)
+// As the 6144-point pass: persistent workgroups of two tiles at a time, the next tiles' rows requested as soon as the
+// transforms have taken the present ones, every twiddle in LDS (48 planes: a workgroup per tile 1.50 ms,
+// now 1.34).
+constexpr int kRows3Tiles = 2, kRows3Threads = 256 * kRows3Tiles;
+constexpr size_t kRows3Lds = sizeof(float2) * (4 * kRows3Tiles * 24 * kTileStride + kTabLane + kTabCross + kSub);
+__global__ void __launch_bounds__(kRows3Threads)
 k_fft_rows_3072(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tw,
-                const float2* __restrict__ tab,
-                int col_lo, int cols, MidLayout mid) {
-    constexpr int G = 3072, H = 1536;
-    __shared__ float2 tile_all[4][24 * kTileStride];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int tile_id = xcd_local_tile(blockIdx.x, gridDim.x);
-    const int plane = tile_id / H, n = tile_id - plane * H;
-    const int which = wave >> 1, half = wave & 1;               // row n or n + 1536; even or odd
-    const float2* src = in + (static_cast<size_t>(plane) * G + n + which * H) * G;
-    float2* tile = tile_all[wave];
-    fft1536_wave(tile, fft1536_tables(tab), lane, [&](int m) { return src[2 * m + half]; },
-                    [&](int k, float2 v) { tile[k] = v; });
-    __syncthreads();
-    const float2 wn = tw[n];
-    float2* dst_a = out + mid.row(2 * plane, n);
-    float2* dst_b = out + mid.row(2 * plane + 1, n);
-    for (int k = threadIdx.x; k < H; k += 256) {
-        const float2 wk = tw[k];
-        const float2 en = tile_all[0][k], on = cmul(tile_all[1][k], wk);
-        const float2 em = tile_all[2][k], om = cmul(tile_all[3][k], wk);
-        const float2 xn0 = cadd(en, on), xn1 = csub(en, on);      // row n at columns k, k + 1536
-        const float2 xm0 = cadd(em, om), xm1 = csub(em, om);      // row n + 1536
-        if (k >= col_lo && k < col_lo + cols) {
-            const size_t i = mid.col(k - col_lo);
-            dst_a[i] = cadd(xn0, xm0);
-            dst_b[i] = cmul(csub(xn0, xm0), wn);
+                const float2* __restrict__ tab, int pairs, int col_lo, int cols, MidLayout mid) {
+    constexpr int G = 3072, H = kSub, kTile = 24 * kTileStride;
+    extern __shared__ float2 rows3_lds[];          // [tile][row n or n + 1536][even or odd][kTile], tables, W^k
+    float2* tab_lds = rows3_lds + 4 * kRows3Tiles * kTile;
+    float2* step_tw = tab_lds + kTabLane + kTabCross;
+    for (int t = threadIdx.x; t < kTabLane + kTabCross; t += kRows3Threads) tab_lds[t] = tab[t];
+    for (int t = threadIdx.x; t < H; t += kRows3Threads) step_tw[t] = tw[t];
+    const Fft1536Tables tables = {tab_lds, tab_lds + kTabLane, tab + kTabLane + kTabCross};
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int which = (wave >> 1) & 1, half = wave & 1;         // row n or n + 1536; even or odd
+    float2* const tile_lds = rows3_lds + wave * kTile;
+    const float2* const pair_lds = rows3_lds + (wave & ~3) * kTile;
+    float2 x[3][8];
+    auto load = [&](int pair) {
+        const int tile_id = kRows3Tiles * pair + (wave >> 2), plane = tile_id / H, n = tile_id - plane * H;
+        const float2* src = in + (static_cast<size_t>(plane) * G + n + which * H) * G + half;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int v = 0; v < 3; ++v) x[v][u] = src[2 * (64 * (3 * u + v) + lane)];
+    };
+    int pair = xcd_local_tile(blockIdx.x, gridDim.x);
+    if (pair < pairs) load(pair);
+    lds_barrier();                                 // the tables
+    for (; pair < pairs; pair += gridDim.x) {
+        fft1536_wave_regs(x, tile_lds, tables, lane, [&](int k, float2 v) { tile_lds[k] = v; });
+        if (pair + static_cast<int>(gridDim.x) < pairs) load(pair + gridDim.x);
+        lds_barrier();
+        const int tile_id = kRows3Tiles * pair + (wave >> 2), plane = tile_id / H, n = tile_id - plane * H;
+        const float2 wn = tw[n];
+        float2* dst_a = out + mid.row(2 * static_cast<size_t>(plane), n);
+        float2* dst_b = out + mid.row(2 * static_cast<size_t>(plane) + 1, n);
+#pragma unroll
+        for (int k = threadIdx.x & 255; k < H; k += 256) {
+            const float2 wk = step_tw[k];
+            const float2 en = pair_lds[k], on = cmul(pair_lds[kTile + k], wk);
+            const float2 em = pair_lds[2 * kTile + k], om = cmul(pair_lds[3 * kTile + k], wk);
+            const float2 xn0 = cadd(en, on), xn1 = csub(en, on);      // row n at columns k, k + 1536
+            const float2 xm0 = cadd(em, om), xm1 = csub(em, om);      // row n + 1536
+            if (k >= col_lo && k < col_lo + cols) {
+                const size_t i = mid.col(k - col_lo);
+                dst_a[i] = cadd(xn0, xm0);
+                dst_b[i] = cmul(csub(xn0, xm0), wn);
+            }
+            const int k1 = k + H;
+            if (k1 >= col_lo && k1 < col_lo + cols) {
+                const size_t i = mid.col(k1 - col_lo);
+                dst_a[i] = cadd(xn1, xm1);
+                dst_b[i] = cmul(csub(xn1, xm1), wn);
+            }
         }
-        const int k1 = k + H;
-        if (k1 >= col_lo && k1 < col_lo + cols) {
-            const size_t i = mid.col(k1 - col_lo);
-            dst_a[i] = cadd(xn1, xm1);
-            dst_b[i] = cmul(csub(xn1, xm1), wn);
-        }
+        lds_barrier();                             // the rows have been read
     }
 }
 
@@ -702,28 +726,49 @@ k_fft_rows_3072(const float2* __restrict__ in, float2* __restrict__ out, const f
 // sums of the column direction's radix-4 step for its twelve columns k = threadIdx.x + 512 i in
 // registers over the four rows and stores them as row n of the plane's four sub-planes (the columns
 // col_lo .. col_lo + cols - 1).  A row pass that took two rows had left half of the column step to the
-// column pass (8 planes: 1.20 + 1.86 ms for both passes, now 1.45 + 0.59).
+// column pass (8 planes: 1.20 + 1.86 ms for both passes, then 1.39 + 0.59).
+// Bound by memory, as the column pass: persistent workgroups, one per CU, request the next two rows
+// as soon as a transform has taken the present ones into LDS, and keep every twiddle in LDS, so that nothing
+// waits behind those loads (eight planes: a workgroup per tile, twiddles from memory 1.39 ms, now
+// 1.12).
 constexpr int kRows6Threads = 512;
-constexpr size_t kRows6Lds = sizeof(float2) * 8 * 24 * kTileStride;
+constexpr size_t kRows6Lds = sizeof(float2) * (8 * 24 * kTileStride + kTabLane + kTabCross + 3 * kSub);
 __global__ void __launch_bounds__(kRows6Threads)
 k_fft_rows_6144(const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tw,
-                const float2* __restrict__ tab,
-                int col_lo, int cols, MidLayout mid) {
-    constexpr int G = 6144, H = 1536, kTile = 24 * kTileStride, kPer = H / kRows6Threads;
-    extern __shared__ float2 rows6_lds[];          // [row of the pair][residue j][kTile]
+                const float2* __restrict__ tab, int tiles, int col_lo, int cols, MidLayout mid) {
+    constexpr int G = 6144, H = kSub, kTile = 24 * kTileStride, kPer = H / kRows6Threads;
+    extern __shared__ float2 rows6_lds[];          // [row of the pair][residue j][kTile], tables, W^{j k}
+    float2* tab_lds = rows6_lds + 8 * kTile;
+    float2* step_tw = tab_lds + kTabLane + kTabCross;
+    for (int t = threadIdx.x; t < kTabLane + kTabCross; t += kRows6Threads) tab_lds[t] = tab[t];
+    for (int t = threadIdx.x; t < H; t += kRows6Threads)
+        for (int j = 1; j < 4; ++j) step_tw[(j - 1) * H + t] = tw[j * t];
+    const Fft1536Tables tables = {tab_lds, tab_lds + kTabLane, tab + kTabLane + kTabCross};
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int tile_id = xcd_local_tile(blockIdx.x, gridDim.x);
+    float2* const tile_lds = rows6_lds + wave * kTile;
+    // Samples of row n + (half + 2 (wave / 4)) H of the tile's plane, residue wave % 4.
+    float2 x0[3][8];
+    auto load = [&](int tile_id, int half) {
+        const int plane = tile_id / H, n = tile_id - plane * H;
+        const float2* src = in + (static_cast<size_t>(plane) * G + n + (half + 2 * (wave >> 2)) * H) * G + (wave & 3);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int v = 0; v < 3; ++v) x0[v][u] = src[4 * (64 * (3 * u + v) + lane)];
+    };
+    int tile_id = xcd_local_tile(blockIdx.x, gridDim.x);
+    if (tile_id < tiles) load(tile_id, 0);
+    lds_barrier();                                 // the tables
+    for (; tile_id < tiles; tile_id += gridDim.x) {
     const int plane = tile_id / H, n = tile_id - plane * H;
+    const int tile_next = tile_id + static_cast<int>(gridDim.x);
     float2 y[4][kPer][4];                          // [q][i][p]
 #pragma unroll
     for (int half = 0; half < 2; ++half) {         // rows m = half and half + 2
-        {
-            const float2* src = in + (static_cast<size_t>(plane) * G + n + (half + 2 * (wave >> 2)) * H) * G;
-            float2* tile = rows6_lds + wave * kTile;
-            fft1536_wave(tile, fft1536_tables(tab), lane, [&](int i) { return src[4 * i + (wave & 3)]; },
-                            [&](int k, float2 v) { tile[k] = v; });
-        }
-        __syncthreads();
+        fft1536_wave_regs(x0, tile_lds, tables, lane, [&](int k, float2 v) { tile_lds[k] = v; });
+        if (half == 0) load(tile_id, 1);
+        else if (tile_next < tiles) load(tile_next, 0);
+        lds_barrier();
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int k0 = threadIdx.x + kRows6Threads * i;
@@ -732,9 +777,9 @@ k_fft_rows_6144(const float2* __restrict__ in, float2* __restrict__ out, const f
             for (int r = 0; r < 2; ++r) {
                 const float2* t = rows6_lds + 4 * r * kTile;
                 const float2 g0 = t[k0];
-                const float2 g1 = cmul(t[kTile + k0], tw[k0]);
-                const float2 g2 = cmul(t[2 * kTile + k0], tw[2 * k0]);
-                const float2 g3 = cmul(t[3 * kTile + k0], tw[3 * k0]);
+                const float2 g1 = cmul(t[kTile + k0], step_tw[k0]);
+                const float2 g2 = cmul(t[2 * kTile + k0], step_tw[H + k0]);
+                const float2 g3 = cmul(t[3 * kTile + k0], step_tw[2 * H + k0]);
                 const float2 s02 = cadd(g0, g2), d02 = csub(g0, g2);
                 const float2 s13 = cadd(g1, g3), id13 = mul_i(csub(g1, g3));
                 x[r][0] = cadd(s02, s13);
@@ -758,7 +803,7 @@ k_fft_rows_6144(const float2* __restrict__ in, float2* __restrict__ out, const f
                 }
             }
         }
-        if (half == 0) __syncthreads();
+        lds_barrier();                             // the rows have been read
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -772,6 +817,7 @@ k_fft_rows_6144(const float2* __restrict__ in, float2* __restrict__ out, const f
                 if (kc >= 0 && kc < cols)
                     dst[mid.col(kc)] = q == 0 ? y[q][i][p] : cmul(y[q][i][p], wq);
             }
+    }
     }
 }
 
@@ -1131,10 +1177,14 @@ void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size
         mid.block_stride = split == 1 ? kBlockCols : kSub * kBlockCols;
         if (split == 4) {
             allow_dynamic_lds(reinterpret_cast<const void*>(&k_fft_rows_6144), kRows6Lds);
-            k_fft_rows_6144<<<static_cast<unsigned>(P * kSub), kRows6Threads, kRows6Lds, ctx->stream>>>(planes, row_out, tw,
-                                                                                                     tab, clo, nc, mid);
+            const int row_tiles = static_cast<int>(P) * kSub;
+            k_fft_rows_6144<<<static_cast<unsigned>(std::min(row_tiles, std::max(1, ctx->cu_count))), kRows6Threads, kRows6Lds,
+                              ctx->stream>>>(planes, row_out, tw, tab, row_tiles, clo, nc, mid);
         } else if (split == 2) {
-            k_fft_rows_3072<<<static_cast<unsigned>(P * kSub), 256, 0, ctx->stream>>>(planes, row_out, tw, tab, clo, nc, mid);
+            allow_dynamic_lds(reinterpret_cast<const void*>(&k_fft_rows_3072), kRows3Lds);
+            const int pairs = static_cast<int>(P) * kSub / kRows3Tiles;
+            k_fft_rows_3072<<<static_cast<unsigned>(std::min(pairs, std::max(1, ctx->cu_count))), kRows3Threads, kRows3Lds,
+                              ctx->stream>>>(planes, row_out, tw, tab, pairs, clo, nc, mid);
         } else {
             const int total_rows = static_cast<int>(P * G);
             k_fft_rows_1536<<<static_cast<unsigned>((total_rows + kFftWaves - 1) / kFftWaves), 64 * kFftWaves, 0,
