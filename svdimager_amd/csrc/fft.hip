@@ -43,7 +43,7 @@ struct FftStages {
 __device__ __forceinline__ int pidx(int i) { return i + (i >> 5); }
 __host__ __device__ inline size_t padded_len(size_t n) { return n + n / 32 + 1; }
 
-// Complex values are float2, or double2 where a butterfly is formed in FP64 (stage_inplace).
+// Complex values are float2, or double2 where a butterfly is formed in FP64 (the convolutions).
 template <class V> __device__ __forceinline__ V cmul(V a, V b) { return V(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
 template <class V> __device__ __forceinline__ V cadd(V a, V b) { return V(a.x + b.x, a.y + b.y); }
 template <class V> __device__ __forceinline__ V csub(V a, V b) { return V(a.x - b.x, a.y - b.y); }
@@ -95,13 +95,13 @@ constexpr double turn_sin(int num, int den) { return turn_cos(4 * num + 3 * den,
 
 // Odd prime P: out_k, out_{P-k} = v_0 + sum_j cos(2 pi j k / P) (v_j + v_{P-j}) +- i sum_j sin(2 pi j k / P)
 // (v_j - v_{P-j}).
-template <int P>
+template <int P, class T = float>
 struct TurnTable {
-    float c[P], s[P];
+    T c[P], s[P];
     constexpr TurnTable() : c(), s() {
         for (int i = 0; i < P; ++i) {
-            c[i] = static_cast<float>(turn_cos(i, P));
-            s[i] = static_cast<float>(turn_sin(i, P));
+            c[i] = static_cast<T>(turn_cos(i, P));
+            s[i] = static_cast<T>(turn_sin(i, P));
         }
     }
 };
@@ -160,10 +160,10 @@ template <int R, class V>
 __device__ __forceinline__ void dft_fixed(V* v);
 
 // R = A^2: X[k1 + A k2] = sum_{n2 < A} W_A^{n2 k2} (W_R^{n2 k1} sum_{n1 < A} W_A^{n1 k1} v[A n1 + n2]).
-template <int A>
-__device__ __forceinline__ void dft_square(float2* v) {
-    constexpr TurnTable<A * A> t;
-    float2 y[A][A];
+template <int A, class V>
+__device__ __forceinline__ void dft_square(V* v) {
+    constexpr TurnTable<A * A, decltype(v->x)> t;
+    V y[A][A];
 #pragma unroll
     for (int n2 = 0; n2 < A; ++n2) {
 #pragma unroll
@@ -171,11 +171,11 @@ __device__ __forceinline__ void dft_square(float2* v) {
         dft_fixed<A>(y[n2]);
 #pragma unroll
         for (int k1 = 1; k1 < A; ++k1)
-            if (n2 != 0) y[n2][k1] = cmul(y[n2][k1], make_float2(t.c[n2 * k1], t.s[n2 * k1]));
+            if (n2 != 0) y[n2][k1] = cmul(y[n2][k1], V(t.c[n2 * k1], t.s[n2 * k1]));
     }
 #pragma unroll
     for (int k1 = 0; k1 < A; ++k1) {
-        float2 z[A];
+        V z[A];
 #pragma unroll
         for (int n2 = 0; n2 < A; ++n2) z[n2] = y[n2][k1];
         dft_fixed<A>(z);
@@ -219,73 +219,6 @@ __device__ __forceinline__ void dft_fixed(V* v) {
     else if constexpr (R == 15) dft_coprime<3, 5>(v);
     else if constexpr (R == 12) dft_coprime<4, 3>(v);
     else dft_coprime<2, R / 2>(v);                     // 6, 10, 14
-}
-
-// One Stockham stage of radix R over ntrans transforms of length n in LDS, `pn` float2 apart and
-// padded: butterfly j reads element j + r m (m = n / R), times e^{+2 pi i (j mod ns) r / (ns R)} (table
-// tw in LDS: tw[t] = e^{2 pi i t / n}), and writes (j / ns) ns R + (j mod ns) + r ns.  In place: every
-// butterfly of the stage (at most kMaxB per thread) is read and transformed into registers, then,
-// after a barrier, written back to the same buffer.  V: the type of the
-// butterfly's arithmetic (double2 rounds once per stage, where values go back to LDS; FP64 runs at the
-// rate of plain FP32 here).
-constexpr int kMaxB = 4;
-constexpr int kInplaceThreads = 512;
-
-template <class V>
-__device__ __forceinline__ V widen(float2 a) { return V(a.x, a.y); }
-
-template <int R, class V>
-__device__ __forceinline__ void stage_inplace(float2* buf, int ntrans, int n, int pn, int ns,
-                                              FastDiv by_m, FastDiv by_ns, const float2* tw) {
-    const int m = n / R;
-    const int tstep = n / (ns * R);
-    const int total = ntrans * m;
-    float2 v[kMaxB][R];
-    int obase[kMaxB];
-#pragma unroll
-    for (int b = 0; b < kMaxB; ++b) {
-        const int t = threadIdx.x + b * kInplaceThreads;
-        obase[b] = -1;
-        if (t < total) {
-            const int tr = static_cast<int>(by_m.div(t));
-            const int j = t - tr * m;
-            const int jq = static_cast<int>(by_ns.div(j));
-            const int jm = j - jq * ns;
-            const float2* in = buf + tr * pn;
-            V x[R];
-            x[0] = widen<V>(in[pidx(j)]);
-#pragma unroll
-            for (int r = 1; r < R; ++r) x[r] = cmul(widen<V>(in[pidx(j + r * m)]), widen<V>(tw[jm * r * tstep]));
-            dft_fixed<R>(x);
-#pragma unroll
-            for (int r = 0; r < R; ++r) v[b][r] = make_float2(static_cast<float>(x[r].x), static_cast<float>(x[r].y));
-            obase[b] = (tr << 20) | (jq * ns * R + jm);     // tr < 16, index < 2^20
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < kMaxB; ++b) {
-        if (obase[b] < 0) continue;
-        float2* out = buf + (obase[b] >> 20) * pn;
-        const int d = obase[b] & 0xfffff;
-#pragma unroll
-        for (int r = 0; r < R; ++r) out[pidx(d + r * ns)] = v[b][r];
-    }
-    __syncthreads();
-}
-
-// (Radices 4 and 8: factorize_pow2.)
-template <class V>
-__device__ void stockham_inplace(float2* buf, int ntrans, int pn, const FftStages& st, const float2* tw) {
-    const int n = st.n;
-    int ns = 1;
-    for (int stage = 0; stage < st.count; ++stage) {
-        const int R = st.radix[stage];
-        const FastDiv bm = st.by_m[stage], bn = st.by_ns[stage];
-        if (R == 4) stage_inplace<4, V>(buf, ntrans, n, pn, ns, bm, bn, tw);
-        else stage_inplace<8, V>(buf, ntrans, n, pn, ns, bm, bn, tw);
-        ns *= R;
-    }
 }
 
 // put(t, get(t)) for t = threadIdx.x, + blockDim.x, ... < n, with the gets of kCopyBatch
@@ -875,87 +808,158 @@ k_fft_cols(const float2* __restrict__ in, float2* __restrict__ out, FftStages st
 // n k = (n^2 + k^2 - (k - n)^2) / 2 gives X[k] = c[k] sum_n (x[n] c[n]) conj(c[k - n]), a circular
 // convolution of length M = 2^m >= 2 G - 1, done by two + transforms of length M in LDS:
 // z = conj(F(x c) B), X[k] = c[k] conj(F(z)[k]), where B = F(conj(c)) / M, conj(c) continued evenly.
-// Rows + columns of the planes of a 301^2 image (453^2): 54 + 37 us, as direct DFTs 518 + 304.  The butterflies
-// are FP64: with FP32 ones (46 + 29 us) the transform's error was already below the direct sums' (2.3e-7
-// rms of white planes' output for 5.4e-7, now 1.5e-7), but the image's was 3 % above theirs, now 24 %
-// below.
+// The first stage is read from memory and the last one written to it; the last stage of the first
+// transform, the product with B and the first stage of the second, which takes the same elements, are one.
+// Rows + columns of the planes of a 301^2 image (453^2): 27 + 20 us; with every stage from and to LDS 54 + 37, as
+// direct DFTs 518 + 304.  The butterflies are FP64 (which runs at the rate of plain FP32 here) and rounded once a
+// stage: with FP32 ones the transform's error was already below the direct sums' (2.3e-7 rms of white planes'
+// output for 5.4e-7, now 1.5e-7), but the image's was 3 % above theirs, now 24 % below.
 struct BlueTables {
     const float2 *chirp, *tw, *spec;               // c[G], W_M[M], B[M]
 };
-__device__ __forceinline__ float2 cconj(float2 a) { return make_float2(a.x, -a.y); }
+__device__ __forceinline__ double2 widen(float2 a) { return make_double2(a.x, a.y); }
+__device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
+__device__ __forceinline__ float2 narrow(double2 a) { return make_float2(static_cast<float>(a.x), static_cast<float>(a.y)); }
 
-// The transforms of `ntrans` sequences: get(tr, n) reads x[n], put(tr, k, X[k]) takes the outputs
-// k_lo .. k_lo + nk - 1.  unit_n: consecutive threads take consecutive elements (else transforms).
-template <bool kUnitN, class Get, class Put>
-__device__ __forceinline__ void blue_transforms(float2* lds, const FftStages& st, const BlueTables& tb, int G,
-                                                int ntrans, int k_lo, int nk, Get&& get, Put&& put) {
-    const int M = st.n, pn = static_cast<int>(padded_len(M));
+// Radices of the first transform of length 2^E; the second's are the same in reverse.
+template <int E>
+struct BlueRadices {
+    static constexpr int count = E < 8 ? 2 : E < 12 ? 3 : 4;
+    static constexpr int r[4] = {E == 8 ? 4 : E == 9 || E == 10 || E == 12 ? 8 : 16, E == 10 || E == 11 ? 16 : 8,
+                                 E < 8 ? 1 : 8, E < 12 ? 1 : 8};
+    static constexpr int least = E == 8 ? 4 : 8;
+    static constexpr int per_transform = (1 << E) / least;         // threads
+};
+
+// The transforms of `ntrans` sequences (per_transform threads each): get(tr, n) reads x[n], put(tr, k, X[k])
+// takes the outputs k_lo .. k_lo + nk - 1.  kUnitN: consecutive threads take consecutive elements of x
+// and X (else transforms).
+template <int E, bool kUnitN, class Get, class Put>
+__device__ __forceinline__ void blue_transforms(float2* lds, const BlueTables& tb, int G, int ntrans, int k_lo, int nk,
+                                                Get&& get, Put&& put) {
+    using L = BlueRadices<E>;
+    constexpr int M = 1 << E;
+    const int pn = static_cast<int>(padded_len(M));
     const float2* tw = load_twiddles(lds, tb.tw, M);
     float2* buf = lds + M;
-    auto split = [&](int t, int len, int& tr, int& i) {
-        if constexpr (kUnitN) {
-            tr = t / len;
-            i = t - tr * len;
-        } else {
-            i = t / ntrans;
-            tr = t - i * ntrans;
+    const int tid = static_cast<int>(threadIdx.x);
+    lds_barrier();
+    // Butterfly j of transform tr of a stage with m butterflies a transform.
+    auto place = [&](int m, bool unit, int& tr, int& j) {
+        tr = unit ? tid / m : tid % ntrans;
+        j = unit ? tid % m : tid / ntrans;
+        return tr < ntrans && j < m;
+    };
+    auto write = [&](auto radix, int tr, int d, int ns, const double2* x, bool active) {
+        constexpr int R = decltype(radix)::value;
+        lds_barrier();                             // the stage has been read
+        if (active)
+#pragma unroll
+            for (int r = 0; r < R; ++r) buf[tr * pn + pidx(d + r * ns)] = narrow(x[r]);
+        lds_barrier();
+    };
+    auto read = [&](auto radix, int tr, int j, int ns, double2* x) {
+        constexpr int R = decltype(radix)::value, m = M / R;
+        const int jm = j & (ns - 1), tstep = M / (ns * R);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            x[r] = widen(buf[tr * pn + pidx(j + r * m)]);
+            if (r > 0) x[r] = cmul(x[r], widen(tw[jm * r * tstep]));
         }
     };
-    copy_batched(G * ntrans,
-                 [&](int t) {
-                     int tr, n;
-                     split(t, G, tr, n);
-                     return get(tr, n);
-                 },
-                 [&](int t, float2 v) {
-                     int tr, n;
-                     split(t, G, tr, n);
-                     buf[tr * pn + pidx(n)] = cmul(v, tb.chirp[n]);
-                 });
-    for (int t = threadIdx.x; t < (M - G) * ntrans; t += kInplaceThreads) {
-        const int tr = t / (M - G), n = G + t - tr * (M - G);
-        buf[tr * pn + pidx(n)] = make_float2(0.f, 0.f);
+    auto middle = [&](auto radix, int ns) {
+        constexpr int R = decltype(radix)::value;
+        int tr, j;
+        const bool active = place(M / R, true, tr, j);
+        double2 x[R];
+        if (active) {
+            read(radix, tr, j, ns, x);
+            dft_fixed<R>(x);
+        }
+        write(radix, tr, (j & ~(ns - 1)) * R + (j & (ns - 1)), ns, x, active);
+    };
+    using First = std::integral_constant<int, L::r[0]>;
+    using Last = std::integral_constant<int, L::r[L::count - 1]>;
+    {
+        constexpr int R = First::value, m = M / R;
+        int tr, j;
+        const bool active = place(m, kUnitN, tr, j);
+        double2 x[R];
+        if (active) {
+            float2 v[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[r] = j + r * m < G ? get(tr, j + r * m) : make_float2(0.f, 0.f);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                x[r] = j + r * m < G ? cmul(widen(v[r]), widen(tb.chirp[j + r * m])) : make_double2(0.0, 0.0);
+            dft_fixed<R>(x);
+        }
+        write(First(), tr, j * R, 1, x, active);
     }
-    __syncthreads();
-    stockham_inplace<double2>(buf, ntrans, pn, st, tw);
-    for (int t = threadIdx.x; t < M * ntrans; t += kInplaceThreads) {
-        const int tr = t / M, k = t - tr * M;
-        float2* at = buf + tr * pn + pidx(k);
-        *at = cconj(cmul(*at, tb.spec[k]));
+    if constexpr (L::count > 2) middle(std::integral_constant<int, L::r[1]>(), L::r[0]);
+    if constexpr (L::count > 3) middle(std::integral_constant<int, L::r[2]>(), L::r[0] * L::r[1]);
+    {
+        constexpr int R = Last::value, m = M / R;
+        int tr, j;
+        const bool active = place(m, true, tr, j);
+        double2 x[R];
+        if (active) {
+            read(Last(), tr, j, m, x);
+            dft_fixed<R>(x);
+#pragma unroll
+            for (int r = 0; r < R; ++r) x[r] = cconj(cmul(x[r], widen(tb.spec[j + r * m])));
+            dft_fixed<R>(x);
+        }
+        write(Last(), tr, j * R, 1, x, active);
     }
-    __syncthreads();
-    stockham_inplace<double2>(buf, ntrans, pn, st, tw);
-    for (int t = threadIdx.x; t < nk * ntrans; t += kInplaceThreads) {
-        int tr, k;
-        split(t, nk, tr, k);
-        put(tr, k, cmul(cconj(buf[tr * pn + pidx(k_lo + k)]), tb.chirp[k_lo + k]));
+    if constexpr (L::count > 3) middle(std::integral_constant<int, L::r[2]>(), L::r[3]);
+    if constexpr (L::count > 2) middle(std::integral_constant<int, L::r[1]>(), M / (L::r[0] * L::r[1]));
+    {
+        constexpr int R = First::value, m = M / R;
+        int tr, j;
+        if (!place(m, kUnitN, tr, j)) return;
+        double2 x[R];
+        read(First(), tr, j, m, x);
+        dft_fixed<R>(x);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int k = j + r * m - k_lo;
+            if (k >= 0 && k < nk) put(tr, k, narrow(cmul(cconj(x[r]), widen(tb.chirp[k_lo + k]))));
+        }
     }
 }
 
-__global__ void __launch_bounds__(kInplaceThreads)
-k_blue_rows(const float2* __restrict__ in, float2* __restrict__ out, FftStages st, BlueTables tb, int G, int batch,
+// Threads of a workgroup: several transforms' where that leaves several workgroups to a CU; columns twice the
+// rows', for longer row segments.
+template <int E>
+constexpr int blue_threads(bool rows) { return E == 13 ? 1024 : E == 12 || !rows ? 512 : 256; }
+
+template <int E>
+__global__ void __launch_bounds__(blue_threads<E>(true))
+k_blue_rows(const float2* __restrict__ in, float2* __restrict__ out, BlueTables tb, int G, int total_rows, int batch,
             int col_lo, int cols) {
     extern __shared__ float2 lds[];
     const int row0 = blockIdx.x * batch;
-    const float2* src = in + (static_cast<size_t>(blockIdx.y) * G + row0) * G;
-    float2* dst = out + (static_cast<size_t>(blockIdx.y) * G + row0) * cols;
-    blue_transforms<true>(lds, st, tb, G, min(batch, G - row0), col_lo, cols,
-                          [&](int tr, int n) { return src[static_cast<size_t>(tr) * G + n]; },
-                          [&](int tr, int k, float2 v) { dst[static_cast<size_t>(tr) * cols + k] = v; });
+    const float2* src = in + static_cast<size_t>(row0) * G;
+    float2* dst = out + static_cast<size_t>(row0) * cols;
+    blue_transforms<E, true>(lds, tb, G, min(batch, total_rows - row0), col_lo, cols,
+                             [&](int tr, int n) { return src[static_cast<size_t>(tr) * G + n]; },
+                             [&](int tr, int k, float2 v) { dst[static_cast<size_t>(tr) * cols + k] = v; });
 }
 
-__global__ void __launch_bounds__(kInplaceThreads)
-k_blue_cols(const float2* __restrict__ in, float2* __restrict__ out, FftStages st, BlueTables tb, int G, int width,
-            int cols, int row_lo, int rows, int strips) {
+template <int E>
+__global__ void __launch_bounds__(blue_threads<E>(false))
+k_blue_cols(const float2* __restrict__ in, float2* __restrict__ out, BlueTables tb, int G, int width, int cols, int row_lo,
+            int rows, int strips) {
     extern __shared__ float2 lds[];
     const int tile = xcd_local_tile(blockIdx.x, gridDim.x);
     const size_t plane = tile / strips;
     const int c0 = (tile - static_cast<int>(plane) * strips) * width;
     const float2* src = in + plane * G * static_cast<size_t>(cols) + c0;
     float2* dst = out + plane * rows * static_cast<size_t>(cols) + c0;
-    blue_transforms<false>(lds, st, tb, G, min(width, cols - c0), row_lo, rows,
-                           [&](int tr, int n) { return src[static_cast<size_t>(n) * cols + tr]; },
-                           [&](int tr, int k, float2 v) { dst[static_cast<size_t>(k) * cols + tr] = v; });
+    blue_transforms<E, false>(lds, tb, G, min(width, cols - c0), row_lo, rows,
+                              [&](int tr, int n) { return src[static_cast<size_t>(n) * cols + tr]; },
+                              [&](int tr, int k, float2 v) { dst[static_cast<size_t>(k) * cols + tr] = v; });
 }
 
 // The tables of BlueTables, contiguous, from FP64: one workgroup, B by a radix-2 transform in LDS (M
@@ -1082,17 +1086,6 @@ bool factorize(int n, FftStages& st) {
     return true;
 }
 
-// n = 2^m >= 16 in radices 8 and 4 only: 8 8 4 4 for 8 8 8 2, so that twice the transforms fit a
-// workgroup's registers.
-void factorize_pow2(int n, FftStages& st) {
-    st.n = n;
-    st.count = 0;
-    int e = __builtin_ctz(static_cast<unsigned>(n));
-    for (; e > 0 && e != 4 && e != 2; e -= 3) st.radix[st.count++] = 8;
-    for (; e > 0; e -= 2) st.radix[st.count++] = 4;
-    stage_divisors(st);
-}
-
 }  // namespace
 
 // Twiddles e^{2 pi i t / G}, t < G, from FP64 sincospi, rounded to FP32, and behind them (for G = 1536
@@ -1206,26 +1199,34 @@ void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size
     }
     FftStages st;
     if (const size_t M = blue_len(G)) {
-        // Transforms per workgroup: as many as the stages' registers and 64 KB of LDS hold, at least one.
-        factorize_pow2(static_cast<int>(M), st);
-        size_t fit = 16;
-        for (int i = 0; i < st.count; ++i)
-            fit = std::min<size_t>(fit, kMaxB * kInplaceThreads / (M / static_cast<size_t>(st.radix[i])));
-        const size_t one = padded_len(M) * sizeof(float2), base = M * sizeof(float2);
-        const size_t room = 64 * 1024 > base ? (64 * 1024 - base) / one : 0;
-        const int batch = static_cast<int>(std::max<size_t>(1, std::min(fit, room)));
-        const size_t lds = base + static_cast<size_t>(batch) * one;
-        const int g = static_cast<int>(G), nc = static_cast<int>(cols);
+        const int g = static_cast<int>(G), nc = static_cast<int>(cols), total_rows = static_cast<int>(P * G);
         const BlueTables tb = {tw, tw + G, tw + G + M};
-        allow_dynamic_lds(reinterpret_cast<const void*>(&k_blue_rows), lds);
-        allow_dynamic_lds(reinterpret_cast<const void*>(&k_blue_cols), lds);
-        k_blue_rows<<<dim3(static_cast<unsigned>((g + batch - 1) / batch), static_cast<unsigned>(P)), kInplaceThreads, lds,
-                      ctx->stream>>>(planes, row_out, st, tb, g, batch, static_cast<int>(col_lo), nc);
-        SVDI_LAUNCH_CHECK();
-        const int strips = (nc + batch - 1) / batch;
-        k_blue_cols<<<static_cast<unsigned>(strips * P), kInplaceThreads, lds, ctx->stream>>>(
-            row_out, out, st, tb, g, batch, nc, static_cast<int>(row_lo), static_cast<int>(rows), strips);
-        SVDI_LAUNCH_CHECK();
+        auto run = [&](auto exponent) {
+            constexpr int E = decltype(exponent)::value;
+            using L = BlueRadices<E>;
+            constexpr int kRowThreads = blue_threads<E>(true), kColThreads = blue_threads<E>(false);
+            const int batch = std::min(16, kRowThreads / L::per_transform), width = std::min(16, kColThreads / L::per_transform);
+            auto lds = [&](int n) { return (M + static_cast<size_t>(n) * padded_len(M)) * sizeof(float2); };
+            allow_dynamic_lds(reinterpret_cast<const void*>(&k_blue_rows<E>), lds(batch));
+            k_blue_rows<E><<<static_cast<unsigned>((total_rows + batch - 1) / batch), kRowThreads, lds(batch), ctx->stream>>>(
+                planes, row_out, tb, g, total_rows, batch, static_cast<int>(col_lo), nc);
+            SVDI_LAUNCH_CHECK();
+            const int strips = (nc + width - 1) / width;
+            allow_dynamic_lds(reinterpret_cast<const void*>(&k_blue_cols<E>), lds(width));
+            k_blue_cols<E><<<static_cast<unsigned>(strips * P), kColThreads, lds(width), ctx->stream>>>(
+                row_out, out, tb, g, width, nc, static_cast<int>(row_lo), static_cast<int>(rows), strips);
+            SVDI_LAUNCH_CHECK();
+        };
+        switch (__builtin_ctzll(M)) {
+            case 7: run(std::integral_constant<int, 7>()); break;
+            case 8: run(std::integral_constant<int, 8>()); break;
+            case 9: run(std::integral_constant<int, 9>()); break;
+            case 10: run(std::integral_constant<int, 10>()); break;
+            case 11: run(std::integral_constant<int, 11>()); break;
+            case 12: run(std::integral_constant<int, 12>()); break;
+            case 13: run(std::integral_constant<int, 13>()); break;
+            default: throw std::logic_error("convolution length out of range");
+        }
         return;
     }
     if (!factorize(static_cast<int>(G), st)) {
