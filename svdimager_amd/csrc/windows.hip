@@ -46,7 +46,7 @@ namespace {
 constexpr int kWin = 16;                 // window side in cells
 constexpr int kMaxClasses = 6;           // classes per window: 24 / class height (4 or 8)
 constexpr int kBinThreads = 1024;        // binning blocks
-constexpr int kBinRowsMost = 512;        // rows of a block, snapshot input: 64 .. 512
+constexpr int kBinRowsLeast = 64, kBinRowsMost = 512;   // rows of a block, snapshot input
 constexpr int kBinPerThreadMost = 16;    // samples per thread, preprocessed input: 1 .. 16
 constexpr int kLdsBins = 36864;          // largest block-local histogram (144 KB of LDS)
 constexpr size_t kMaxBlockHistBytes = size_t(1) << 31;   // per-block histograms of all bands
@@ -167,13 +167,18 @@ __device__ __forceinline__ void for_sample_bins(const SampleInput& in, const Gri
     };
     if constexpr (kSnap) {
         if (in.quad_rows) {
-            // Four consecutive rows of one channel per thread (one 16-byte load per FP32 array,
-            // 4 bytes per flag array), 128 row quads x 8 channel groups in blocks of 512 rows (16 x
-            // 64 in blocks of 64); the next channel's loads are issued before this one is binned.
-            const uint32_t quads_log2 = 31 - __builtin_clz(static_cast<uint32_t>(wg.block_size) / 4);
-            const uint32_t quad_groups = kBinThreads >> quads_log2;
-            const size_t row0 = blk * wg.block_size + 4 * (threadIdx.x & ((1u << quads_log2) - 1));
-            if (row0 >= in.num_rows) return;          // (num_rows % 4 == 0: quads are whole)
+            // Four consecutive rows of one channel per thread (one 16-byte load per FP32 array, which needs no
+            // more than 4-byte alignment, and one of 4 bytes per flag array), block_size / 4 row quads x
+            // as many channel groups as the threads are enough for; the next channel's loads are issued before
+            // this one is binned.  The last quad of a row count that is not a multiple of 4 starts earlier and
+            // leaves out the rows of the quad before it.  (5.2 M samples in 81,103 rows: scatter + count 128 us
+            // one row per thread, 119 so.)
+            const uint32_t quads = static_cast<uint32_t>(wg.block_size) / 4, quad_groups = kBinThreads / quads;
+            const uint32_t group = threadIdx.x / quads;
+            const size_t quad0 = blk * wg.block_size + 4 * (threadIdx.x - group * quads);
+            if (group >= quad_groups || quad0 >= in.num_rows) return;
+            const size_t row0 = min(quad0, in.num_rows - 4);
+            const int first = static_cast<int>(quad0 - row0);
             struct QuadLoad {
                 double nu;
                 float4 v0r, v0i, v3r, v3i, w0, w3;
@@ -187,19 +192,19 @@ __device__ __forceinline__ void for_sample_bins(const SampleInput& in, const Gri
                 q.v0r = q.v0i = q.v3r = q.v3i = zero4;
                 q.w0 = q.w3 = one4;
                 if constexpr (kVis) {
-                    q.v0r = *reinterpret_cast<const float4*>(in.v0r + idx);
-                    q.v0i = *reinterpret_cast<const float4*>(in.v0i + idx);
-                    q.v3r = *reinterpret_cast<const float4*>(in.v3r + idx);
-                    q.v3i = *reinterpret_cast<const float4*>(in.v3i + idx);
-                    if (in.w0) q.w0 = *reinterpret_cast<const float4*>(in.w0 + idx);
-                    if (in.w3) q.w3 = *reinterpret_cast<const float4*>(in.w3 + idx);
+                    __builtin_memcpy(&q.v0r, in.v0r + idx, 16);
+                    __builtin_memcpy(&q.v0i, in.v0i + idx, 16);
+                    __builtin_memcpy(&q.v3r, in.v3r + idx, 16);
+                    __builtin_memcpy(&q.v3i, in.v3i + idx, 16);
+                    if (in.w0) __builtin_memcpy(&q.w0, in.w0 + idx, 16);
+                    if (in.w3) __builtin_memcpy(&q.w3, in.w3 + idx, 16);
                 }
-                q.f0 = *reinterpret_cast<const uint32_t*>(in.f0 + idx);
-                q.f3 = *reinterpret_cast<const uint32_t*>(in.f3 + idx);
+                __builtin_memcpy(&q.f0, in.f0 + idx, 4);
+                __builtin_memcpy(&q.f3, in.f3 + idx, 4);
                 return q;
             };
             auto lane4 = [](const float4& v, int r) { return r == 0 ? v.x : r == 1 ? v.y : r == 2 ? v.z : v.w; };
-            size_t chan = threadIdx.x >> quads_log2;
+            size_t chan = group;
             if (chan >= in.num_channels) return;
             QuadLoad cur = load(chan);
             double geo[4][3];
@@ -212,6 +217,7 @@ __device__ __forceinline__ void for_sample_bins(const SampleInput& in, const Gri
                 if (chan + quad_groups < in.num_channels) nxt = load(chan + quad_groups);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
+                    if (r < first) continue;
                     SnapLoad s;
                     s.nu = cur.nu;
                     s.v0r = lane4(cur.v0r, r);
@@ -1992,9 +1998,8 @@ bool grid_windows_supported(const SampleInput& in, const GridParams& gp) {
 // and, for its histogram, with the bins (about 3.7 ns a sample in the scatter and count passes together
 // with 3 ns for ten bins), one block per CU at a time; every block also costs 14 bytes per bin of counts
 // and offsets in memory.  So a snapshot that does not fill the chip with the largest blocks takes smaller
-// ones (scatter + count of 1.4 M samples in 29,377 rows at 1000^2: 58 blocks 114 us, 230 blocks 56; of 5.2 M
-// in 81,103 rows at 512^2: 159 blocks 171, 254 blocks 127), as long as its histograms do not cost more.  Rows read four
-// at a time take powers of two (their threads are dealt by shifts).
+// ones (scatter + count of 1.4 M samples in 29,377 rows at 1000^2: 58 blocks 114 us, 230 blocks 56), as long
+// as its histograms do not cost more.
 static unsigned choose_bin_blocks(const svdi_context* ctx, const SampleInput& in, WinGeom& wg) {
     // (Channels below sixteen would leave most of sixteen groups of threads idle.)
     wg.set_rows = in.num_channels > 8 ? 64 : 256;
@@ -2002,7 +2007,7 @@ static unsigned choose_bin_blocks(const svdi_context* ctx, const SampleInput& in
     // Samples of a unit, a block's idle groups of threads included.
     auto unit_samples = [&](int size) {
         if (!in.from_snapshot) return static_cast<size_t>(kBinThreads);
-        const size_t groups = kBinThreads / (in.quad_rows ? size / 4 : wg.set_rows);
+        const size_t groups = kBinThreads / static_cast<size_t>(in.quad_rows ? size / 4 : wg.set_rows);
         return (in.num_channels + groups - 1) / groups * groups;
     };
     const int most = in.from_snapshot ? kBinRowsMost : kBinPerThreadMost;
@@ -2011,8 +2016,8 @@ static unsigned choose_bin_blocks(const svdi_context* ctx, const SampleInput& in
     // (The fixed scratch range keeps the largest blocks: fewer histograms.)
     if (ctx->ws.arena_left() == SIZE_MAX) {
         double best = 0.0;
-        const int step = in.from_snapshot ? (in.quad_rows ? 64 : wg.set_rows) : 1;
-        for (int size = most; size >= step; size = in.from_snapshot && in.quad_rows ? size / 2 : size - step) {
+        const int step = in.from_snapshot ? (in.quad_rows ? kBinRowsLeast : wg.set_rows) : 1;
+        for (int size = most; size >= step; size -= in.quad_rows && in.from_snapshot ? 16 : step) {
             const size_t blocks = blocks_of(size);
             const size_t rounds = (blocks + ctx->cu_count - 1) / ctx->cu_count;
             const double bins = static_cast<double>(wg.lbins);

@@ -1,7 +1,7 @@
 """The window binning's block sizes (rows per block by the snapshot's rows and channels, samples per
 thread of preprocessed input) against the tile gridder, whose binning is separate code: row counts
 around a block of 64 rows and above, channel counts around the groups of threads that share a row,
-rows read four at a time (a multiple of 4) and one at a time.
+and from 16384 rows on rows read four at a time, a multiple of 4 and with one to three left over.
 
 Tolerance: both gridders sum n <= 70000 samples of the same sign in FP32, errors of at most about
 sqrt(n) 2^-24 of a cell's sum (1.6e-5, averaged away in the image's central half); a sample lost or
@@ -17,8 +17,8 @@ import svdimager_amd as S
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows", [5, 63, 64, 260, 1021, 1024])
-@pytest.mark.parametrize("channels", [1, 8, 9, 17, 64, 67])
+@pytest.mark.parametrize("rows,channels", [(r, c) for r in (3, 5, 63, 64, 260, 1021, 1024) for c in (1, 8, 9, 17, 64, 67)] +
+                         [(16384, 4), (16385, 1), (16386, 3), (16387, 4), (20000, 2), (33001, 2)])
 def test_block_sizes_match_the_tile_gridder(rows, channels):
     announce(f"block sizes rows={rows} channels={channels}")
     N, cell = 96, 1e-4
