@@ -172,7 +172,9 @@ k_term_errors(DevPlan* __restrict__ plan) {
     __shared__ double jn[kMaxTerms];
     __shared__ double red[kKept][kTermThreads / 64];
     const float amax = plan->slab_alpha_max;
-    const float alpha_f = amax * static_cast<float>(blockIdx.x) / static_cast<float>(na - 1);
+    // (Alpha 0 is left to the zeros that the maxima start from: its sum is exact.  512 and 256 blocks are whole
+    // rounds over the CUs: archive 35 us, with a block more 45; two blocks a CU at 128 registers, with spills, 34.)
+    const float alpha_f = amax * static_cast<float>(blockIdx.x + 1) / static_cast<float>(na - 1);
     const double alpha = static_cast<double>(alpha_f);
     double sv[kPer], er[kPer], ei[kPer];
 #pragma unroll
@@ -271,8 +273,8 @@ void launch_plan(svdi_context* ctx, const SampleInput& in, Semantics sem, size_t
     k_plan_finalize<<<1, kThreads, 0, ctx->stream>>>(r3p, r3_blocks, t3max, t3valid, t3_blocks,
                                                     archive, target_alpha, vin, plan);
     SVDI_LAUNCH_CHECK();
-    if (archive) k_term_errors<true><<<513, kTermThreads, 0, ctx->stream>>>(plan);
-    else k_term_errors<false><<<257, kTermThreads, 0, ctx->stream>>>(plan);
+    if (archive) k_term_errors<true><<<512, kTermThreads, 0, ctx->stream>>>(plan);
+    else k_term_errors<false><<<256, kTermThreads, 0, ctx->stream>>>(plan);
     SVDI_LAUNCH_CHECK();
 }
 
