@@ -36,6 +36,7 @@
 #include "scan.hpp"
 #include "es_poly.hpp"
 #include "records.hpp"
+#include "work_shape.hpp"
 
 #include <cstring>
 #include <type_traits>
@@ -666,16 +667,6 @@ __device__ __forceinline__ int item_class(uint32_t count, uint32_t cap) {
     return c;
 }
 
-// A dense window's pieces: equal runs of `per` records (a multiple of 32), the last one shorter.
-struct Pieces {
-    uint32_t count, per;
-};
-__device__ __forceinline__ Pieces dense_pieces(const WinGeom& wg, uint32_t records) {
-    const uint32_t n = (records + wg.coop_cap - 1) / wg.coop_cap;
-    const uint32_t per = ((records + n - 1) / n + 31u) & ~31u;
-    return {(records + per - 1) / per, per};
-}
-
 // Home records of half `half` of window (wa, wb) of slab ls (0 outside the grid of windows).
 __device__ __forceinline__ uint32_t half_records(const uint32_t* __restrict__ boff, const WinGeom& wg, int ls, int wa, int wb,
                                                  int half) {
@@ -744,7 +735,7 @@ k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __res
         int pcls = -1;
         Pieces p = {0u, 0u};
         if (s.dense[j]) {
-            p = dense_pieces(wg, s.h[j + 1] - s.h[j]);
+            p = dense_pieces(s.h[j + 1] - s.h[j], wg.coop_cap);
             pcls = piece_class(wg, p);
         }
         for (int k = 0; k <= kItemClasses; ++k)
@@ -789,7 +780,7 @@ k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__
     Pieces pieces[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        pieces[j] = dense_pieces(wg, records[j]);
+        pieces[j] = dense_pieces(records[j], wg.coop_cap);
         queue[j] = ioff[records[j] != 0 ? (kItemClasses + 2 * piece_class(wg, pieces[j]) + j) * nwt + w : n];
     }
     const int wcls = wave_item_class(wg, s);
@@ -801,7 +792,7 @@ k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__
         r.add = s.s_count > 0 ? 1 : 0;
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
-            r.count[k] = records[k] != 0 ? dense_pieces(wg, records[k]).count : 0u;
+            r.count[k] = records[k] != 0 ? dense_pieces(records[k], wg.coop_cap).count : 0u;
             r.first[k] = records[k] != 0 ? slots[k] - slot0 : 0u;
         }
         red[red_at - red0] = r;
