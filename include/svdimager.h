@@ -261,8 +261,10 @@ int svdi_image_snapshots_planned(svdi_context* ctx, const svdi_snapshot* snapsho
  * of at most coop_cap records each taken by a whole workgroup.  Records are binned by row classes
  * of 2^class_log2 rows.  Zero fields select the library's defaults (coop_min 256 .. 1024 and
  * coop_cap 2048 .. 16384 by the number of samples, class_log2 2 when its histogram fits in LDS,
- * else 3).  The shape changes how the FP32 sums are ordered, not what is summed: images agree to
- * rounding. */
+ * else 3).  Every piece's partial sums take memory; should a snapshot's pieces pass what is set
+ * aside for them (several times what the snapshots of the usual arrays make), that call's pieces
+ * and then its coop_min grow until they fit.  The shape changes how the FP32 sums are ordered, not
+ * what is summed: images agree to rounding. */
 typedef struct svdi_tuning {
     uint32_t coop_min;          /* 0, or 32 .. 65536 */
     uint32_t coop_cap;          /* 0, or 4096 .. 16777216 */

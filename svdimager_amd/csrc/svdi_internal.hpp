@@ -277,7 +277,7 @@ struct WindowJob {
     const void* reduce = nullptr;          // the windows that reduce_windows completes
     uint32_t max_slots = 0;
     int K = 0, G = 0, prec = 0;
-    int geom[16] = {};                     // the window geometry (windows.hip)
+    int geom[20] = {};                     // the window geometry (windows.hip)
 };
 WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp, float2* planes);
 void contract_windows(svdi_context* ctx, const WindowJob* jobs, int count);

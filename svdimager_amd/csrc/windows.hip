@@ -116,8 +116,8 @@ struct WinGeom {
     int band_bins;   // bins per LDS band (<= kLdsBins); band y covers [y band_bins, ...) of lbins
     int block_size;  // binning blocks: rows (snapshot input), samples per thread (preprocessed)
     int set_rows;    // rows of a block read at a time (64 or 256; snapshot rows read one by one)
-    uint32_t coop_min;   // records up to which a window is one wavefront item
-    uint32_t coop_cap;   // records per workgroup piece
+    WorkShape shape;     // records above which a half is dense, and per workgroup piece (asked for; fit_shape)
+    uint32_t slots;      // partial slots (kAllSlotsFit: enough for any sizes of the halves)
 };
 
 // A work item of window `win`.  slot < 0: a wavefront item, the `count` records from `start` on
@@ -379,12 +379,46 @@ k_bin_seg_sums(const CountT* __restrict__ blockhist, int nblocks, int nbins, uin
     if (sum != 0) atomicAdd(&counts[bin], sum);
 }
 
-// cnt and offs may be the same words (32-bit counts): each is read before it is written.
+// The dense halves counted by size for fit_shape, half t by thread t of workgroups of 256; words: kShapeWords, zero
+// before.
+inline unsigned half_size_blocks(const WinGeom& wg) { return (2u * static_cast<unsigned>(wg.nwin_total) + 255) / 256; }
+__device__ __forceinline__ void count_half_sizes(const uint32_t* __restrict__ boff, const WinGeom& wg, uint32_t* __restrict__ words) {
+    __shared__ uint32_t s_words[kShapeWords];
+    for (int i = threadIdx.x; i < kShapeWords; i += 256) s_words[i] = 0u;
+    __syncthreads();
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < 2 * wg.nwin_total) {
+        const int per = 8 >> wg.cls_log2, col = t / (2 * wg.nw), h = (t - col * 2 * wg.nw) * per;
+        const uint32_t* b = boff + static_cast<size_t>(col) * wg.nh;
+        const uint32_t n = b[min(h + per, wg.nh)] - b[min(h, wg.nh)];
+        if (n > wg.shape.coop_min) {
+            const int k = 2 + 2 * shape_bucket(wg.shape.coop_min, n);
+            atomicAdd(&s_words[0], 1u);
+            atomicAdd(&s_words[1], n);
+            atomicAdd(&s_words[k], 1u);
+            atomicAdd(&s_words[k + 1], n);
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kShapeWords; i += 256)
+        if (s_words[i] != 0) atomicAdd(&words[i], s_words[i]);
+}
+__global__ void __launch_bounds__(256)
+k_win_half_sizes(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __restrict__ words) {
+    count_half_sizes(boff, wg, words);
+}
+
+// cnt and offs may be the same words (32-bit counts): each is read before it is written.  The first size_blocks
+// workgroups count the halves' sizes instead (boff holds the bins' offsets then).
 template <typename CountT>
 __global__ void __launch_bounds__(256)
 k_bin_block_offsets(const CountT* cnt, uint32_t* offs, int nblocks, int nbins, const uint32_t* __restrict__ segsum,
-                    const uint32_t* __restrict__ boff) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
+                    const uint32_t* __restrict__ boff, unsigned size_blocks, WinGeom wg, uint32_t* __restrict__ words) {
+    if (blockIdx.x < size_blocks) {
+        count_half_sizes(boff, wg, words);
+        return;
+    }
+    const int t = (blockIdx.x - size_blocks) * 256 + threadIdx.x;
     if (t >= kBinSegs * nbins) return;
     const int seg = t / nbins, bin = t - seg * nbins;
     int b0, b1;
@@ -654,11 +688,10 @@ __device__ __forceinline__ WinRange window_range(const uint32_t* __restrict__ bo
 // and workgroups finish together.
 // icount: [kItemClasses][nwin_total] wavefront items, [kItemClasses][2 nwin_total] pieces of the
 // halves, [2 nwin_total] partial slots, [nwin_total] windows that k_win_reduce completes; one exclusive
-// scan gives the queue positions, slot numbers and places in k_win_reduce's list.  totals[0] = records, [1] = wavefront items, [2] = (unused), [3] = pieces,
-// [4] = max |v| bits, [5] = piece queue head, [6] = windows that k_win_reduce completes.
+// scan gives the queue positions, slot numbers and places in k_win_reduce's list.  totals[0] = records, [1] = wavefront items, [2] = coop_min,
+// [3] = pieces, [4] = max |v| bits, [5] = piece queue head, [6] = windows that k_win_reduce completes, [7] = coop_cap (the shape
+// that fit_shape left).
 constexpr int kItemClasses = 8;
-constexpr uint32_t kCoopMinDefault = 1024;
-constexpr uint32_t kCoopCapDefault = 16384;
 
 __device__ __forceinline__ int item_class(uint32_t count, uint32_t cap) {
     if (count == 0) return kItemClasses - 1;
@@ -692,13 +725,13 @@ __device__ __forceinline__ WinSplit window_split(const uint32_t* __restrict__ bo
                                                  const WinRange& x, uint32_t end) {
     const int ls = w / wg.nwin, r = w - ls * wg.nwin;
     const int wa = r / wg.nw, wb = r - wa * wg.nw;
-    auto if_dense = [&](uint32_t n) { return n > wg.coop_min ? n : 0u; };
+    auto if_dense = [&](uint32_t n) { return n > wg.shape.coop_min ? n : 0u; };
     WinSplit s;
     s.h[0] = wg.cls_log2 == 2 ? x.bnd[2] : x.bnd[1];
     s.h[1] = wg.cls_log2 == 2 ? x.bnd[4] : x.bnd[2];
     s.h[2] = end;
-    s.dense[0] = s.h[1] - s.h[0] > wg.coop_min;
-    s.dense[1] = s.h[2] - s.h[1] > wg.coop_min;
+    s.dense[0] = s.h[1] - s.h[0] > wg.shape.coop_min;
+    s.dense[1] = s.h[2] - s.h[1] > wg.shape.coop_min;
     // (The classes below the home ones are the upper half of the window above; none at the top.)
     s.up = if_dense(s.h[0] - x.start());
     s.left[0] = if_dense(half_records(boff, wg, ls, wa, wb - 1, 0));
@@ -715,18 +748,25 @@ __device__ __forceinline__ WinSplit window_split(const uint32_t* __restrict__ bo
 
 // The queue classes of a window's wavefront item (-1: it has none) and of a dense half's pieces.
 __device__ __forceinline__ int wave_item_class(const WinGeom& wg, const WinSplit& s) {
-    return s.s_count > 0 || !s.reduced() ? item_class(s.s_count, 3 * wg.coop_min) : -1;
+    const uint32_t cap = 3u * min(wg.shape.coop_min, 0xffffffffu / 3u);
+    return s.s_count > 0 || !s.reduced() ? item_class(s.s_count, cap) : -1;
 }
-__device__ __forceinline__ int piece_class(const WinGeom& wg, const Pieces& p) { return item_class(p.per, wg.coop_cap); }
+__device__ __forceinline__ int piece_class(const WinGeom& wg, const Pieces& p) { return item_class(p.per, wg.shape.coop_cap); }
 
 __global__ void __launch_bounds__(256)
-k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __restrict__ icount, uint32_t* __restrict__ totals) {
+k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __restrict__ icount, uint32_t* __restrict__ totals,
+                  const uint32_t* __restrict__ words) {
     const int w = blockIdx.x * 256 + threadIdx.x;
     const int nwt = wg.nwin_total;
-    if (w == 0) totals[0] = boff[wg.nbins];
     if (w >= nwt) return;
     uint32_t end;
     const WinRange x = window_range(boff, wg, w, end);
+    fit_shape(words, wg.slots, wg.shape);
+    if (w == 0) {
+        totals[0] = boff[wg.nbins];
+        totals[2] = wg.shape.coop_min;
+        totals[7] = wg.shape.coop_cap;
+    }
     const WinSplit s = window_split(boff, wg, w, x, end);
     const int wcls = wave_item_class(wg, s);
     for (int k = 0; k < kItemClasses; ++k) icount[k * nwt + w] = k == wcls ? 1u : 0u;
@@ -735,7 +775,7 @@ k_win_item_counts(const uint32_t* __restrict__ boff, WinGeom wg, uint32_t* __res
         int pcls = -1;
         Pieces p = {0u, 0u};
         if (s.dense[j]) {
-            p = dense_pieces(s.h[j + 1] - s.h[j], wg.coop_cap);
+            p = dense_pieces(s.h[j + 1] - s.h[j], wg.shape.coop_cap);
             pcls = piece_class(wg, p);
         }
         for (int k = 0; k <= kItemClasses; ++k)
@@ -761,6 +801,7 @@ constexpr int kItemLanes = 2;
 __global__ void __launch_bounds__(256)
 k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__ ioff, WinGeom wg, WItem* __restrict__ items,
                  uint32_t max_items, WReduce* __restrict__ red, uint32_t* __restrict__ totals) {
+    wg.shape = {totals[2], totals[7]};
     const int t = blockIdx.x * 256 + threadIdx.x;
     const int w = t / kItemLanes, sub = t % kItemLanes;
     const int nwt = wg.nwin_total;
@@ -780,7 +821,7 @@ k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__
     Pieces pieces[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        pieces[j] = dense_pieces(records[j], wg.coop_cap);
+        pieces[j] = dense_pieces(records[j], wg.shape.coop_cap);
         queue[j] = ioff[records[j] != 0 ? (kItemClasses + 2 * piece_class(wg, pieces[j]) + j) * nwt + w : n];
     }
     const int wcls = wave_item_class(wg, s);
@@ -792,7 +833,7 @@ k_win_item_write(const uint32_t* __restrict__ boff, const uint32_t* __restrict__
         r.add = s.s_count > 0 ? 1 : 0;
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
-            r.count[k] = records[k] != 0 ? dense_pieces(records[k], wg.coop_cap).count : 0u;
+            r.count[k] = records[k] != 0 ? dense_pieces(records[k], wg.shape.coop_cap).count : 0u;
             r.first[k] = records[k] != 0 ? slots[k] - slot0 : 0u;
         }
         red[red_at - red0] = r;
@@ -2064,11 +2105,12 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     const dim3 bin_grid(blocks, bands);
 
     // counts[0, lbins) | counts[lbins + 2, +8) = totals, [+8, +10) = the coarse bins' pieces | the coarse bins' class counts and the slots
-    // handed out, kSup lbins each.
+    // handed out, kSup lbins each | the halves' sizes (fit_shape).
     const size_t nsub = coarse ? kSup * lbins : 0;
-    const size_t ncleared = lbins + 12 + 2 * nsub;
+    const size_t ncleared = lbins + 12 + 2 * nsub + kShapeWords;
     uint32_t* counts = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinCounts, ncleared * sizeof(uint32_t)));
     uint32_t* sub_counts = counts + lbins + 12;
+    uint32_t* half_sizes = sub_counts + 2 * nsub;
     // Per-block record offsets (the counts themselves when 32-bit), the (block, band) record
     // totals, then the 16-bit per-block counts when a block has fewer than 65536 samples (a
     // bin's count per block is at most its sample count).
@@ -2094,31 +2136,17 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     WRecords rec;
     rec.r = static_cast<uint4*>(ctx->ws.get(Workspace::kRecPos, max_records * sizeof(uint4)));
 
-    // Work shape: a half is dense above coop_min records, in pieces of at most coop_cap.  Fewer samples
-    // take smaller pieces, so that they still spread over the chip (a workgroup contracts a piece of
-    // 16384 records in about 100 us), and a lower threshold, so that no wavefront's item is a long
-    // chain.  Measured per call (coop_min / coop_cap): 8.4 M samples at 1024^2 869 us with
-    // 1024 / 16384, 882 with 1024 / 8192, 986 with 512 / 4096; 5.2 M at 512^2 700 with 1024 / 8192,
-    // 745 with 512 / 4096; 2.1 M at 1024^2 642 with 512 / 4096, 677 with 1024 / 8192; 1.4 M at 1000^2 635 with
-    // 512 / 4096, 661 with 256 / 2048, 672 with 1024 / 8192; 32 k at 128^2 210 with 256 / 2048, 232 with
-    // 1024 / 8192.
-    auto clamped = [](size_t v, size_t lo, size_t hi) { return static_cast<uint32_t>(std::min(std::max(v, lo), hi)); };
-    wg.coop_min = gp.coop_min != 0 ? gp.coop_min : clamped(S / 4096, 256, kCoopMinDefault);
-    wg.coop_cap = gp.coop_cap != 0 ? gp.coop_cap : clamped(S / 512, 2048, kCoopCapDefault);
-    // Wavefront items: one per window at most.  Pieces (and partial slots): at most one per dense
-    // half, of which there are at most records / (coop_min + 1), plus records / coop_cap.  The slots
-    // of the worst case are bounded to kMaxPartialBytes (in the fixed scratch range to what is left but
-    // for the items and the FFT's tables) by a coarser shape.
+    // Wavefront items: one per window at most.  Pieces, and partial slots: as many as any sizes of the halves could
+    // need, but for a bound in bytes (kMaxPartialBytes, in the fixed scratch range what is left but for the items and the FFT's
+    // tables), past which fit_shape sees to it that the slots suffice.
+    wg.shape = work_shape(S, gp.coop_min, gp.coop_cap);
     const size_t slot_bytes = static_cast<size_t>(gp.K) * kDenseCells * sizeof(float2) + sizeof(WItem);
     const size_t reserve = nwt * (sizeof(WItem) + sizeof(WReduce)) + fft_table_bytes(static_cast<size_t>(gp.G)) + (32u << 10);
     const size_t left = ctx->ws.arena_left();
     const size_t partial_bytes = std::min(kMaxPartialBytes, left > reserve ? left - reserve : 0);
-    auto slots = [&]() { return max_records / wg.coop_cap + std::min(2 * nwt, max_records / (wg.coop_min + 1)) + 1; };
-    while (slots() * slot_bytes > partial_bytes && (wg.coop_cap < max_records || wg.coop_min < max_records)) {
-        if (max_records / wg.coop_cap >= slots() / 2) wg.coop_cap *= 2;
-        else wg.coop_min *= 2;
-    }
-    const size_t max_slots = slots();
+    const size_t most = most_pieces(wg.shape, max_records, 2 * nwt), room = partial_bytes / slot_bytes;
+    const size_t max_slots = std::min(most, room);
+    wg.slots = most <= room ? kAllSlotsFit : static_cast<uint32_t>(room);
     const size_t max_items = nwt + max_slots;
     WItem* items = static_cast<WItem*>(ctx->ws.get(Workspace::kItems, max_items * sizeof(WItem) + nwt * sizeof(WReduce)));
     WReduce* red = reinterpret_cast<WReduce*>(items + max_items);
@@ -2159,13 +2187,16 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
         SVDI_LAUNCH_CHECK();
     }
     launch_exclusive_scan(ctx, counts, coff, wg.use_lds ? nullptr : cursor, sums, lbins);
+    // The halves' sizes, where they are needed, are counted on the way if the bins' offsets are there by now.
+    const bool sizes = wg.slots != kAllSlotsFit;
+    const unsigned size_blocks = sizes && wg.use_lds && !coarse ? half_size_blocks(wg) : 0u;
     if (wg.use_lds) {
         if (count16)
-            k_bin_block_offsets<uint16_t><<<seg_grid, 256, 0, ctx->stream>>>(
-                blockcount16, blockhist, static_cast<int>(blocks), wg.lbins, segsum, coff);
+            k_bin_block_offsets<uint16_t><<<seg_grid + size_blocks, 256, 0, ctx->stream>>>(
+                blockcount16, blockhist, static_cast<int>(blocks), wg.lbins, segsum, coff, size_blocks, wg, half_sizes);
         else
-            k_bin_block_offsets<uint32_t><<<seg_grid, 256, 0, ctx->stream>>>(
-                blockhist, blockhist, static_cast<int>(blocks), wg.lbins, segsum, coff);
+            k_bin_block_offsets<uint32_t><<<seg_grid + size_blocks, 256, 0, ctx->stream>>>(
+                blockhist, blockhist, static_cast<int>(blocks), wg.lbins, segsum, coff, size_blocks, wg, half_sizes);
         SVDI_LAUNCH_CHECK();
     }
     const uint32_t limit = static_cast<uint32_t>(max_records);
@@ -2194,7 +2225,11 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
                                                                         sub_counts, sub_counts + nsub, boff, rec, limit);
         SVDI_LAUNCH_CHECK();
     }
-    k_win_item_counts<<<static_cast<unsigned>((nwt + 255) / 256), 256, 0, ctx->stream>>>(boff, wg, icount, totals);
+    if (sizes && size_blocks == 0) {
+        k_win_half_sizes<<<half_size_blocks(wg), 256, 0, ctx->stream>>>(boff, wg, half_sizes);
+        SVDI_LAUNCH_CHECK();
+    }
+    k_win_item_counts<<<static_cast<unsigned>((nwt + 255) / 256), 256, 0, ctx->stream>>>(boff, wg, icount, totals, half_sizes);
     SVDI_LAUNCH_CHECK();
     launch_exclusive_scan(ctx, icount, ioff, nullptr, sums, ncounts);
     k_win_item_write<<<static_cast<unsigned>((kItemLanes * nwt + 255) / 256), 256, 0, ctx->stream>>>(
