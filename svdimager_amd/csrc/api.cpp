@@ -277,7 +277,8 @@ struct Enqueued {
     GridParams gp;
     ImageParams ip;
     float2* planes = nullptr;
-    float2* rowfft = nullptr;
+    float2* rowfft = nullptr;              // the transformed rows; before them the window gridder's scratch
+    size_t rowfft_bytes = 0;
     float2* colfft = nullptr;
     float* conv = nullptr;
     const float* vin_dev = nullptr;
@@ -307,7 +308,6 @@ Enqueued image_prepare(svdi_context* ctx, const SampleInput& in, const svdi_opti
     }
     const size_t P = hp.batch_slabs * static_cast<size_t>(K);
     e.planes = static_cast<float2*>(ctx->ws.get(Workspace::kPlanes, P * G * G * sizeof(float2)));
-    e.rowfft = static_cast<float2*>(ctx->ws.get(Workspace::kRowFft, P * fft_row_elems(G, hp.cols) * sizeof(float2)));
     e.colfft = static_cast<float2*>(ctx->ws.get(Workspace::kColFft, P * hp.rows * hp.cols * sizeof(float2)));
     float* conv = static_cast<float*>(ctx->ws.get(Workspace::kConv, (N / 2 + 1) * sizeof(float)));
     e.conv = conv;
@@ -374,6 +374,14 @@ Enqueued image_prepare(svdi_context* ctx, const SampleInput& in, const svdi_opti
                         : grid_windows_supported(in, probe) ? SVDI_GRIDDER_MFMA : SVDI_GRIDDER_TILED;
     cs.gridder = gridder;
     e.gridder = gridder;
+
+    e.rowfft_bytes = P * fft_row_elems(G, hp.cols) * sizeof(float2);
+    if (gridder == SVDI_GRIDDER_MFMA && grid_windows_supported(in, probe)) {
+        const WindowScratch w = window_scratch(ctx, in, probe, e.rowfft_bytes);
+        e.rowfft_bytes = w.wanted;
+        if (ctx->ws.frozen()) e.rowfft_bytes = std::max(w.least, std::min(w.wanted, ctx->ws.held(Workspace::kRowFft)));
+    }
+    e.rowfft = static_cast<float2*>(ctx->ws.get(Workspace::kRowFft, e.rowfft_bytes));
     return e;
 }
 
@@ -383,7 +391,7 @@ void image_grid(svdi_context* ctx, const SampleInput& in, CallState& cs, Enqueue
     e.gp.nslabs = static_cast<int>(nb);
     const size_t tok = stage_begin(ctx, 2);
     if (e.gridder == SVDI_GRIDDER_MFMA) {
-        cs.tile_totals = launch_grid_windows(ctx, in, e.gp, e.planes);
+        cs.tile_totals = launch_grid_windows(ctx, in, e.gp, e.planes, e.rowfft, e.rowfft_bytes);
     } else if (e.gridder == SVDI_GRIDDER_TILED) {
         cs.tile_totals = launch_grid_tiled(ctx, in, e.gp, e.planes);
     } else {
@@ -1010,7 +1018,7 @@ int image_batch_planned(svdi_context* ctx, const svdi_snapshot* snaps, size_t co
                     if (e[k].gridder == SVDI_GRIDDER_MFMA) {
                         e[k].gp.slab_start = 0;
                         e[k].gp.nslabs = static_cast<int>(e[k].total_slabs);
-                        jobs.push_back(bin_windows(lane, in[k], e[k].gp, e[k].planes));
+                        jobs.push_back(bin_windows(lane, in[k], e[k].gp, e[k].planes, e[k].rowfft, e[k].rowfft_bytes));
                         SVDI_HIP(hipEventRecord(lane->ev_plan, lane->stream));
                         binned.push_back(k);
                     } else {

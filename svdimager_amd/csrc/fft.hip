@@ -1120,8 +1120,6 @@ static size_t blue_len(size_t G) {
 }
 static size_t twiddle_elems(size_t G) { return G + (fft_split(G) != 0 ? kTabAll : 2 * blue_len(G)); }
 
-size_t fft_table_bytes(size_t G) { return twiddle_elems(G) * sizeof(float2); }
-
 // The twiddle table of G in the context's workspace, computed on the stream (no host copy, no
 // synchronisation) when G or the table's address changed since the last call.
 void fft_prepare(svdi_context* ctx, size_t G) {

@@ -136,17 +136,18 @@ class Workspace {
     enum Slot {
         kPartials, kPlan, kGeometry, kRot, kConv, kPlanes, kRowFft, kColFft, kTwiddles,
         kBinCounts, kBinOffsets, kBinCursor, kRecPos, kRecVim, kItems, kMisc, kImage,
-        kInBin, kInVre, kInVim, kInVin, kInSnap, kR3Partials, kScanSums, kRunPos, kRunOff, kItemCounts, kItemOffsets, kWinPartial, kSlots
+        kInBin, kInVre, kInVim, kInVin, kInSnap, kR3Partials, kScanSums, kRunPos, kRunOff, kItemCounts, kItemOffsets, kSlots
     };
     void* get(Slot s, size_t bytes);
     void release();
     size_t bytes_held() const;
     void begin_arena(void* base, size_t capacity);
     void end_arena();
-    // Bytes of the arena not carved yet (SIZE_MAX outside arena mode).
-    size_t arena_left() const { return arena_ != nullptr ? arena_cap_ - arena_used_ : SIZE_MAX; }
+    size_t held(Slot s) const { return size_[s]; }
     // Frozen: a slot that would have to grow throws ArgError instead of allocating.
     void set_frozen(bool on) { frozen_ = on; }
+    bool frozen() const { return frozen_; }
+    bool in_arena() const { return arena_ != nullptr; }
     ~Workspace() { release(); }
 
   private:
@@ -259,8 +260,15 @@ void launch_grid_atomic(svdi_context* ctx, const SampleInput& in, const GridPara
 // {records, items} of the launch.
 const uint32_t* launch_grid_tiled(svdi_context* ctx, const SampleInput& in, const GridParams& gp,
                                   float2* planes);
+// windows.hip's scratch (WindowScratch) is free for other use as soon as the planes are written.
 const uint32_t* launch_grid_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp,
-                                    float2* planes);
+                                    float2* planes, void* scratch, size_t scratch_bytes);
+// Scratch of a call whose slab batches have gp.nslabs slabs each and the last one the rest, in a buffer that also holds
+// row_bytes of something else: the size to allocate, and the least that does.
+struct WindowScratch {
+    size_t least, wanted;
+};
+WindowScratch window_scratch(const svdi_context* ctx, const SampleInput& in, const GridParams& gp, size_t row_bytes);
 // The window gridder in three steps, so that one contraction launch (on the calling context's
 // stream) can take several slab batches, of several snapshots, binned on other streams:
 // bin_windows enqueues the binning of one slab batch, contract_windows the contraction of up to
@@ -279,7 +287,8 @@ struct WindowJob {
     int K = 0, G = 0, prec = 0;
     int geom[20] = {};                     // the window geometry (windows.hip)
 };
-WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp, float2* planes);
+WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp, float2* planes, void* scratch,
+                      size_t scratch_bytes);
 void contract_windows(svdi_context* ctx, const WindowJob* jobs, int count);
 void reduce_windows(svdi_context* ctx, const WindowJob& job);
 // api.cpp: the batched call (status), and svdi_last_error's message for failures reported
@@ -294,7 +303,6 @@ bool grid_windows_supported(const SampleInput& in, const GridParams& gp);
 
 // fft.hip
 void fft_prepare(svdi_context* ctx, size_t G);
-size_t fft_table_bytes(size_t G);
 // float2 elements of a plane's row-transformed columns (launch_fft2_inverse's row_out).
 size_t fft_row_elems(size_t G, size_t cols);
 // Layout of a transformed plane's window: row-major (split = 0), or, for G = 1536 s (split = s), the

@@ -51,7 +51,6 @@ constexpr int kBinRowsLeast = 64, kBinRowsMost = 512;   // rows of a block, snap
 constexpr int kBinPerThreadMost = 16;    // samples per thread, preprocessed input: 1 .. 16
 constexpr int kLdsBins = 36864;          // largest block-local histogram (144 KB of LDS)
 constexpr size_t kMaxBlockHistBytes = size_t(1) << 31;   // per-block histograms of all bands
-constexpr size_t kMaxPartialBytes = size_t(1) << 29;     // partial slots of the dense halves
 constexpr int kSupLog2 = 3;              // row classes binned together when the bins pass kLdsBins
 constexpr int kSup = 1 << kSupLog2;
 constexpr int kChunk = 32;               // samples per MFMA reduction step
@@ -2019,23 +2018,81 @@ static int effective_class_log2(const GridParams& gp, int nw) {
     return gp.class_log2 == 2 || gp.class_log2 == 3 ? gp.class_log2 : window_class_log2(gp, nw);
 }
 
+// Records at most: one row class and two window columns per sample.
+static size_t max_window_records(const SampleInput& in) { return 2 * in.num_samples; }
+// Pieces of the coarse bins at most (k_sub_list).
+static size_t sub_piece_cap(const WinGeom& wg, size_t max_records) {
+    return static_cast<size_t>(wg.nwin_total / wg.nw) * ((wg.nh + kSup - 1) / kSup) + max_records / kSubPiece;
+}
+
 bool grid_windows_supported(const SampleInput& in, const GridParams& gp) {
     if (gp.G > 8192 || gp.G < 1) return false;
     const int nw = (gp.G + kWin - 1) / kWin;
     if (window_bins(gp, nw, effective_class_log2(gp, nw)) >= (1ull << 30)) return false;
-    return 2 * in.num_samples < (1ull << 31);             // records: at most two per sample
+    return max_window_records(in) < (1ull << 31);
 }
 
-// The binning's block size (WinGeom) and the number of blocks.  A block's time goes with its samples
+// The window geometry of a slab batch, but for what depends on the binning's blocks.
+static WinGeom window_geometry(const SampleInput& in, const GridParams& gp) {
+    WinGeom wg = {};
+    wg.nw = (gp.G + kWin - 1) / kWin;
+    wg.cls_log2 = effective_class_log2(gp, wg.nw);
+    wg.ncls = 24 >> wg.cls_log2;
+    wg.nh = (gp.G + (1 << wg.cls_log2) - 1) >> wg.cls_log2;
+    wg.nwin = wg.nw * wg.nw;
+    wg.nwin_total = wg.nwin * gp.nslabs;
+    wg.nbins = static_cast<int>(window_bins(gp, wg.nw, wg.cls_log2));
+    wg.shape = work_shape(in.num_samples, gp.coop_min, gp.coop_cap);
+    // Bins that pass the LDS histogram are counted and scattered as coarse bins of eight row classes,
+    // whose records k_sub_bins then sorts by class: one pass over the samples where there were up to
+    // eight, for one more over the records.  16.7 M samples at 4096^2 (294,912 bins): count, scatter and
+    // offsets 1.77 ms, now 0.70; 3.8 M at 2048^2 in three slabs 396 us, now 310.  The records wait in the planes, which
+    // nothing has written yet; if these are too small, in LDS bands of the bins themselves.
+    const size_t planes_bytes = static_cast<size_t>(gp.nslabs) * gp.K * gp.G * gp.G * sizeof(float2);
+    const size_t max_records = max_window_records(in);
+    const bool coarse = wg.nbins > kLdsBins &&
+                        max_records * sizeof(uint4) + sub_piece_cap(wg, max_records) * sizeof(SubPiece) <= planes_bytes;
+    wg.sup_log2 = coarse ? kSupLog2 : 0;
+    wg.sup_rows = (wg.nh + (1 << wg.sup_log2) - 1) >> wg.sup_log2;
+    wg.lbins = gp.nslabs * wg.nw * wg.sup_rows;
+    // (Channels below sixteen would leave most of sixteen groups of threads idle.)
+    wg.set_rows = in.num_channels > 8 ? 64 : 256;
+    return wg;
+}
+
+// The binning's blocks of a size, and what they keep in memory: per-block record offsets (the counts
+// themselves when 32-bit), the (block, band) record totals, then the 16-bit per-block counts when a block has fewer
+// than 65536 samples (a bin's count per block is at most its sample count).  LDS bands of at most kLdsBins bins, unless
+// the per-block histograms would pass kMaxBlockHistBytes (then one global atomic per record).
+struct BinBlocks {
+    int size = 0;                                          // rows (snapshot input), samples per thread (preprocessed)
+    size_t blocks = 0, bands = 1, nhist = 1, bytes = 0;
+    bool use_lds = false, count16 = false;
+};
+static BinBlocks bin_blocks(const SampleInput& in, const WinGeom& wg, int size) {
+    BinBlocks b;
+    b.size = size;
+    const size_t units = in.from_snapshot ? in.num_rows : (in.num_samples + kBinThreads - 1) / kBinThreads;
+    const size_t lbins = static_cast<size_t>(wg.lbins);
+    b.blocks = (units + size - 1) / static_cast<size_t>(size);
+    b.use_lds = b.blocks * lbins * sizeof(uint32_t) <= kMaxBlockHistBytes;
+    if (b.use_lds) {
+        b.bands = (lbins + kLdsBins - 1) / kLdsBins;
+        b.nhist = b.blocks * lbins;
+        b.count16 = static_cast<size_t>(size) * (in.from_snapshot ? in.num_channels : kBinThreads) < 65536;
+    }
+    b.bytes = (b.nhist + b.blocks * b.bands) * sizeof(uint32_t) + (b.count16 ? b.nhist * sizeof(uint16_t) : 0);
+    return b;
+}
+
+// The blocks that a call takes, of those whose memory is at most `room` (the largest size's is given).  A block's time
+// goes with its samples
 // and, for its histogram, with the bins (about 3.7 ns a sample in the scatter and count passes together
 // with 3 ns for ten bins), one block per CU at a time; every block also costs 14 bytes per bin of counts
 // and offsets in memory.  So a snapshot that does not fill the chip with the largest blocks takes smaller
 // ones (scatter + count of 1.4 M samples in 29,377 rows at 1000^2: 58 blocks 114 us, 230 blocks 56), as long
 // as its histograms do not cost more.
-static unsigned choose_bin_blocks(const svdi_context* ctx, const SampleInput& in, WinGeom& wg) {
-    // (Channels below sixteen would leave most of sixteen groups of threads idle.)
-    wg.set_rows = in.num_channels > 8 ? 64 : 256;
-    const size_t units = in.from_snapshot ? in.num_rows : (in.num_samples + kBinThreads - 1) / kBinThreads;
+static BinBlocks choose_bin_blocks(const svdi_context* ctx, const SampleInput& in, const WinGeom& wg, size_t room) {
     // Samples of a unit, a block's idle groups of threads included.
     auto unit_samples = [&](int size) {
         if (!in.from_snapshot) return static_cast<size_t>(kBinThreads);
@@ -2043,66 +2100,74 @@ static unsigned choose_bin_blocks(const svdi_context* ctx, const SampleInput& in
         return (in.num_channels + groups - 1) / groups * groups;
     };
     const int most = in.from_snapshot ? kBinRowsMost : kBinPerThreadMost;
-    auto blocks_of = [&](int size) { return (units + size - 1) / static_cast<size_t>(size); };
-    wg.block_size = most;
-    // (The fixed scratch range keeps the largest blocks: fewer histograms.)
-    if (ctx->ws.arena_left() == SIZE_MAX) {
-        double best = 0.0;
-        const int step = in.from_snapshot ? (in.quad_rows ? kBinRowsLeast : wg.set_rows) : 1;
-        for (int size = most; size >= step; size -= in.quad_rows && in.from_snapshot ? 16 : step) {
-            const size_t blocks = blocks_of(size);
-            const size_t rounds = (blocks + ctx->cu_count - 1) / ctx->cu_count;
-            const double bins = static_cast<double>(wg.lbins);
-            const double ns = rounds * (3.7 * static_cast<double>(size * unit_samples(size)) + 0.3 * std::min(bins, 1.0 * kLdsBins)) +
-                              blocks * bins * 0.0035;
-            if (size != most && (ns >= best || blocks * bins * sizeof(uint32_t) > kMaxBlockHistBytes / 8)) continue;
-            best = ns;
-            wg.block_size = size;
-        }
+    const int least = !in.from_snapshot ? 1 : in.quad_rows ? kBinRowsLeast : wg.set_rows;
+    const int step = in.from_snapshot && in.quad_rows ? 16 : least;
+    BinBlocks pick;
+    double best = 0.0;
+    for (int size = most; size >= least; size -= step) {
+        const BinBlocks b = bin_blocks(in, wg, size);
+        const size_t rounds = (b.blocks + ctx->cu_count - 1) / ctx->cu_count;
+        const double bins = static_cast<double>(wg.lbins);
+        const double ns = rounds * (3.7 * static_cast<double>(size * unit_samples(size)) + 0.3 * std::min(bins, 1.0 * kLdsBins)) +
+                          b.blocks * bins * 0.0035;
+        if (size != most && (ns >= best || b.bytes > room)) continue;
+        best = ns;
+        pick = b;
     }
-    return static_cast<unsigned>(blocks_of(wg.block_size));
+    return pick;
 }
 
-WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp, float2* planes) {
+// Bytes of the window gridder's scratch: the binning's blocks first, then work items, partial sums and the scratch line.
+constexpr size_t kTrash = 64;                              // float2
+static size_t item_bytes(const WinGeom& wg) {
+    return static_cast<size_t>(wg.nwin_total) * (sizeof(WItem) + sizeof(WReduce)) + kTrash * sizeof(float2);
+}
+static size_t slot_bytes(const GridParams& gp) { return static_cast<size_t>(gp.K) * kDenseCells * sizeof(float2) + sizeof(WItem); }
+
+// The scratch is the buffer of the transformed rows (row_bytes), which is idle until the planes are
+// done.  It holds a slot for every 576 grid cells, and snapshots of the usual arrays make a piece for every 1,300 to
+// 17,000.  Small grids of many samples make more (1,219 at 512^2, one for every 484), so the buffer is larger
+// by a slot for every 4,608 samples where the worst case asks for it.  (With slots for the worst case, items and
+// histograms in buffers of their own the context held 1,029 MB after the SKA-Low snapshot and 591 after one of 1.4 M samples at 1000^2; so 609 and 345.)
+WindowScratch window_scratch(const svdi_context* ctx, const SampleInput& in, const GridParams& gp, size_t row_bytes) {
+    WindowScratch s = {row_bytes, row_bytes};
+    GridParams batch = gp;
+    for (int nslabs : {gp.nslabs, gp.total_slabs % gp.nslabs}) {           // whole slab batches and the last one
+        if (nslabs == 0) continue;
+        batch.nslabs = nslabs;
+        const WinGeom wg = window_geometry(in, batch);
+        const size_t most = most_pieces(wg.shape, max_window_records(in), 2 * static_cast<size_t>(wg.nwin_total));
+        const size_t bound = row_bytes + (in.num_samples / 4608 + 16) * slot_bytes(gp);
+        const int largest = in.from_snapshot ? kBinRowsMost : kBinPerThreadMost;
+        s.least = std::max({s.least, item_bytes(wg), bin_blocks(in, wg, largest).bytes});
+        s.wanted = std::max(s.wanted, std::min(item_bytes(wg) + most * slot_bytes(gp), bound));
+        // (The fixed scratch range leaves the smaller blocks' histograms no more room than there is.)
+        if (!ctx->ws.in_arena()) s.wanted = std::max(s.wanted, choose_bin_blocks(ctx, in, wg, kMaxBlockHistBytes / 8).bytes);
+    }
+    s.wanted = std::max(s.wanted, s.least);
+    return s;
+}
+
+WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp, float2* planes, void* scratch,
+                      size_t scratch_bytes) {
     if (gp.K < 1 || gp.K > kMaxTerms) throw std::logic_error("term count out of range");
     if (!grid_windows_supported(in, gp)) throw UnsupportedError("grid or sample count too large for the window gridder");
-    WinGeom wg;
-    wg.nw = (gp.G + kWin - 1) / kWin;
-    wg.cls_log2 = effective_class_log2(gp, wg.nw);
-    wg.ncls = 24 >> wg.cls_log2;
-    wg.nh = (gp.G + (1 << wg.cls_log2) - 1) >> wg.cls_log2;
-    wg.nwin = wg.nw * wg.nw;
-    wg.nwin_total = wg.nwin * gp.nslabs;
-    const size_t nbins_sz = window_bins(gp, wg.nw, wg.cls_log2);
-    wg.nbins = static_cast<int>(nbins_sz);
-    const size_t S = in.num_samples;
-    const size_t max_records = 2 * S;                      // one row class, at most two window columns
-    const size_t nbins = nbins_sz;
+    WinGeom wg = window_geometry(in, gp);
+    const size_t max_records = max_window_records(in);
+    const size_t nbins = static_cast<size_t>(wg.nbins), lbins = static_cast<size_t>(wg.lbins);
     const size_t nwt = static_cast<size_t>(wg.nwin_total);
-    // Bins that pass the LDS histogram are counted and scattered as coarse bins of eight row classes,
-    // whose records k_sub_bins then sorts by class: one pass over the samples where there were up to
-    // eight, for one more over the records.  16.7 M samples at 4096^2 (294,912 bins): count, scatter and
-    // offsets 1.77 ms, now 0.70; 3.8 M at 2048^2 in three slabs 396 us, now 310.  The records wait in the planes, which nothing has written yet; if
-    // these are too small, in LDS bands of the bins themselves.
-    const size_t sub_bins = static_cast<size_t>(gp.nslabs) * wg.nw * ((wg.nh + kSup - 1) / kSup);
-    const uint32_t sub_cap = static_cast<uint32_t>(sub_bins + max_records / kSubPiece);
-    const size_t sub_bytes = sub_cap * sizeof(SubPiece);
-    const size_t planes_bytes = static_cast<size_t>(gp.nslabs) * gp.K * gp.G * gp.G * sizeof(float2);
-    const bool coarse = nbins > static_cast<size_t>(kLdsBins) && max_records * sizeof(uint4) + sub_bytes <= planes_bytes;
-    wg.sup_log2 = coarse ? kSupLog2 : 0;
-    wg.sup_rows = (wg.nh + (1 << wg.sup_log2) - 1) >> wg.sup_log2;
-    const size_t lbins = static_cast<size_t>(gp.nslabs) * wg.nw * wg.sup_rows;
-    wg.lbins = static_cast<int>(lbins);
-    const unsigned blocks = choose_bin_blocks(ctx, in, wg);
-    // LDS bands of at most kLdsBins bins, unless the per-block histograms would pass
-    // kMaxBlockHistBytes (then one global atomic per record).
+    const bool coarse = wg.sup_log2 != 0;
+    const uint32_t sub_cap = static_cast<uint32_t>(sub_piece_cap(wg, max_records));
+    const BinBlocks bb = choose_bin_blocks(ctx, in, wg, std::min(scratch_bytes, kMaxBlockHistBytes / 8));
+    if (std::max(bb.bytes, item_bytes(wg)) > scratch_bytes) throw std::logic_error("the window gridder's scratch is too small");
+    const unsigned blocks = static_cast<unsigned>(bb.blocks);
+    wg.block_size = bb.size;
+    wg.use_lds = bb.use_lds ? 1 : 0;
+    const bool count16 = bb.count16;
     const size_t nbands = (lbins + kLdsBins - 1) / kLdsBins;
-    wg.use_lds = static_cast<size_t>(blocks) * lbins * sizeof(uint32_t) <= kMaxBlockHistBytes ? 1 : 0;
     wg.band_bins = static_cast<int>((lbins + nbands - 1) / nbands);
-    const unsigned bands = wg.use_lds ? static_cast<unsigned>(nbands) : 1u;
-    const size_t nhist = wg.use_lds ? static_cast<size_t>(blocks) * lbins : 1;
     const size_t bin_lds = wg.use_lds ? static_cast<size_t>(wg.band_bins) * sizeof(uint32_t) : 0;
-    const dim3 bin_grid(blocks, bands);
+    const dim3 bin_grid(blocks, static_cast<unsigned>(bb.bands));
 
     // counts[0, lbins) | counts[lbins + 2, +8) = totals, [+8, +10) = the coarse bins' pieces | the coarse bins' class counts and the slots
     // handed out, kSup lbins each | the halves' sizes (fit_shape).
@@ -2111,16 +2176,9 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     uint32_t* counts = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinCounts, ncleared * sizeof(uint32_t)));
     uint32_t* sub_counts = counts + lbins + 12;
     uint32_t* half_sizes = sub_counts + 2 * nsub;
-    // Per-block record offsets (the counts themselves when 32-bit), the (block, band) record
-    // totals, then the 16-bit per-block counts when a block has fewer than 65536 samples (a
-    // bin's count per block is at most its sample count).
-    const size_t block_samples = static_cast<size_t>(wg.block_size) * (in.from_snapshot ? in.num_channels : kBinThreads);
-    const bool count16 = wg.use_lds && block_samples < 65536;
-    const size_t ntot = static_cast<size_t>(blocks) * bands;
-    uint32_t* blockhist = static_cast<uint32_t*>(ctx->ws.get(
-        Workspace::kRunOff, (nhist + ntot) * sizeof(uint32_t) + (count16 ? nhist * sizeof(uint16_t) : 0)));
-    uint32_t* blocktot = blockhist + nhist;
-    uint16_t* blockcount16 = count16 ? reinterpret_cast<uint16_t*>(blocktot + ntot) : nullptr;
+    uint32_t* blockhist = static_cast<uint32_t*>(scratch);
+    uint32_t* blocktot = blockhist + bb.nhist;
+    uint16_t* blockcount16 = count16 ? reinterpret_cast<uint16_t*>(blocktot + bb.blocks * bb.bands) : nullptr;
     uint32_t* boff = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinOffsets, (nbins + 8) * sizeof(uint32_t)));
     // Cursors (without LDS histograms); segment sums [kBinSegs][lbins]; the coarse bins' offsets.
     uint32_t* cursor = static_cast<uint32_t*>(ctx->ws.get(
@@ -2137,23 +2195,16 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     rec.r = static_cast<uint4*>(ctx->ws.get(Workspace::kRecPos, max_records * sizeof(uint4)));
 
     // Wavefront items: one per window at most.  Pieces, and partial slots: as many as any sizes of the halves could
-    // need, but for a bound in bytes (kMaxPartialBytes, in the fixed scratch range what is left but for the items and the FFT's
-    // tables), past which fit_shape sees to it that the slots suffice.
-    wg.shape = work_shape(S, gp.coop_min, gp.coop_cap);
-    const size_t slot_bytes = static_cast<size_t>(gp.K) * kDenseCells * sizeof(float2) + sizeof(WItem);
-    const size_t reserve = nwt * (sizeof(WItem) + sizeof(WReduce)) + fft_table_bytes(static_cast<size_t>(gp.G)) + (32u << 10);
-    const size_t left = ctx->ws.arena_left();
-    const size_t partial_bytes = std::min(kMaxPartialBytes, left > reserve ? left - reserve : 0);
-    const size_t most = most_pieces(wg.shape, max_records, 2 * nwt), room = partial_bytes / slot_bytes;
+    // need, or as many as the scratch holds: then fit_shape sees to it that they suffice.
+    const size_t most = most_pieces(wg.shape, max_records, 2 * nwt);
+    const size_t room = std::min((scratch_bytes - item_bytes(wg)) / slot_bytes(gp), static_cast<size_t>(kAllSlotsFit - 1));
     const size_t max_slots = std::min(most, room);
     wg.slots = most <= room ? kAllSlotsFit : static_cast<uint32_t>(room);
     const size_t max_items = nwt + max_slots;
-    WItem* items = static_cast<WItem*>(ctx->ws.get(Workspace::kItems, max_items * sizeof(WItem) + nwt * sizeof(WReduce)));
-    WReduce* red = reinterpret_cast<WReduce*>(items + max_items);
-    const size_t piece_floats2 = static_cast<size_t>(gp.K) * kDenseCells;
-    float2* partial = static_cast<float2*>(
-        ctx->ws.get(Workspace::kWinPartial, (max_slots * piece_floats2 + 64) * sizeof(float2)));
-    float2* trash = partial + max_slots * piece_floats2;
+    float2* partial = static_cast<float2*>(scratch);
+    float2* trash = partial + max_slots * static_cast<size_t>(gp.K) * kDenseCells;
+    WReduce* red = reinterpret_cast<WReduce*>(trash + kTrash);
+    WItem* items = reinterpret_cast<WItem*>(red + nwt);
 
     launch_fill(ctx, reinterpret_cast<float*>(counts), ncleared, 0.0f);
     // 16-bit LDS histograms (two bins per word) when there are also more blocks than CUs, so that
@@ -2308,8 +2359,8 @@ void reduce_windows(svdi_context* ctx, const WindowJob& job) {
 }
 
 const uint32_t* launch_grid_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp,
-                                    float2* planes) {
-    const WindowJob job = bin_windows(ctx, in, gp, planes);
+                                    float2* planes, void* scratch, size_t scratch_bytes) {
+    const WindowJob job = bin_windows(ctx, in, gp, planes, scratch, scratch_bytes);
     contract_windows(ctx, &job, 1);
     reduce_windows(ctx, job);
     return job.totals;
