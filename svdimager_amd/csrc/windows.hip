@@ -2173,7 +2173,11 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     // handed out, kSup lbins each | the halves' sizes (fit_shape).
     const size_t nsub = coarse ? kSup * lbins : 0;
     const size_t ncleared = lbins + 12 + 2 * nsub + kShapeWords;
-    uint32_t* counts = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinCounts, ncleared * sizeof(uint32_t)));
+    // (Both forms' sizes where there are two: records that did not fit the planes and then do find room under capture.)
+    const size_t sub_rows = (static_cast<size_t>(wg.nh) + kSup - 1) / kSup, sub_lbins = nwt / wg.nw * sub_rows;
+    const size_t ncounts_held = nbins > static_cast<size_t>(kLdsBins) ? std::max(nbins, (1 + 2 * kSup) * sub_lbins) : lbins;
+    uint32_t* counts = static_cast<uint32_t*>(
+        ctx->ws.get(Workspace::kBinCounts, (ncounts_held + 12 + kShapeWords) * sizeof(uint32_t)));
     uint32_t* sub_counts = counts + lbins + 12;
     uint32_t* half_sizes = sub_counts + 2 * nsub;
     uint32_t* blockhist = static_cast<uint32_t*>(scratch);
