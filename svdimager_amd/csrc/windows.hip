@@ -1365,8 +1365,11 @@ constexpr int kDStride = 32;                                    // halves or flo
 template <int P, int MB>
 struct DenseTraits {
     using T = WinTraits<P>;
-    static constexpr int kWaves = MB == 1 ? 12 : 8;
-    static constexpr int kBatch = MB == 1 ? 8192 : 4096;        // records sorted at a time
+    // The modes of single-f16 ES products stage less and keep within 128 registers (168 with sixteen terms of one f16 each):
+    // more wavefronts, and with one f16 per term value a whole default piece sorted at once.  (SKA-Low snapshot, call:
+    // single 759 us with twelve wavefronts and 8192 records, 748 so, splitc 772 and 768; single at 16 terms 1130 and 1120.)
+    static constexpr int kWaves = MB == 1 ? T::kWaves : P == kPrecSingle ? 12 : 8;
+    static constexpr int kBatch = MB > 1 ? 4096 : P == kPrecSingle ? 16384 : 8192;             // records sorted at a time
     static constexpr int kPer = (kBatch + kWaves * 64 - 1) / (kWaves * 64);
     static constexpr int kRows = kDenseURows + kDenseVRows;
     // Per wavefront: the ES rows (ku hi [lo], kv hi [lo] in f16, or ku, kv in FP32), then c[16].
