@@ -688,8 +688,9 @@ __device__ __forceinline__ WinRange window_range(const uint32_t* __restrict__ bo
 // icount: [kItemClasses][nwin_total] wavefront items, [kItemClasses][2 nwin_total] pieces of the
 // halves, [2 nwin_total] partial slots, [nwin_total] windows that k_win_reduce completes; one exclusive
 // scan gives the queue positions, slot numbers and places in k_win_reduce's list.  totals[0] = records, [1] = wavefront items, [2] = coop_min,
-// [3] = pieces, [4] = max |v| bits, [5] = piece queue head, [6] = windows that k_win_reduce completes, [7] = coop_cap (the shape
-// that fit_shape left).
+// [3] = pieces, [4] = max |v| bits, [6] = windows that k_win_reduce completes, [7] = coop_cap (the shape that fit_shape
+// left), [8], [9] = the coarse bins' pieces, [kPieceHead ..] = the piece queue's heads.
+constexpr int kPieceHead = 10;           // two words: blocks of eight terms, of sixteen
 constexpr int kItemClasses = 8;
 
 __device__ __forceinline__ int item_class(uint32_t count, uint32_t cap) {
@@ -1297,6 +1298,7 @@ struct WinJob {
     float2* trash;
     WinGeom wg;
     int K, G;
+    int k_lo, k_hi;          // the terms of a dense launch
 };
 struct WinJobs {
     WinJob job[kMaxJobs];
@@ -1646,7 +1648,7 @@ k_win_dense(WinJobs jobs) {
     uint32_t* const s_gid = s_gend + 64;                   // and group; [128] their number
     const int njobs = jobs.count;
 
-    // The jobs' pieces as offsets of one queue, whose head is job 0's totals[5].  The claimed index
+    // The jobs' pieces as offsets of one queue, whose head is a word of job 0's totals.  The claimed index
     // is read back into a scalar register, so the loop exit is wave-uniform by construction and
     // every wavefront runs the same barriers.
     if (threadIdx.x == 0) {
@@ -1657,7 +1659,7 @@ k_win_dense(WinJobs jobs) {
             c += static_cast<int>(jobs.job[j].totals[3]);
         }
         s_off[njobs] = c;
-        s_item = static_cast<int>(atomicAdd(&jobs.job[0].totals[5], 1u));
+        s_item = static_cast<int>(atomicAdd(&jobs.job[0].totals[kPieceHead + MB - 1], 1u));
     }
     // A piece's job and record range, requested while the piece before it is contracted.
     struct Piece {
@@ -1685,21 +1687,21 @@ k_win_dense(WinJobs jobs) {
         lds_barrier();                                   // s_item read; the tile is free
         // The next piece is claimed now and published with this one's sorted indices.
         uint32_t gnext = 0;
-        if (threadIdx.x == 0) gnext = atomicAdd(&jobs.job[0].totals[5], 1u);
+        if (threadIdx.x == 0) gnext = atomicAdd(&jobs.job[0].totals[kPieceHead + MB - 1], 1u);
         int gi_next = nitems;
         Piece itn;
         const WinJob& J = jobs.job[it.job];
         const JobScale scale = job_scale(J);
-        const int K = J.K;
+        const int K = J.K, k_lo = J.k_lo, k_hi = J.k_hi;
         // (The upper half's records store their row relative to the window below.)
         const int row_adj = (it.half_skip & 1) ? kDenseHalf : 0;
         const bool skip = (it.half_skip & 2) != 0;
-        for (int kg = 0; kg < K; kg += 8 * MB) {
+        for (int kg = k_lo; kg < k_hi; kg += 8 * MB) {
             for (int i = threadIdx.x; i < D::kTileFloats / 4; i += kThreads)
                 reinterpret_cast<float4*>(dense_lds)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             for (int b0 = 0; b0 < it.count; b0 += D::kBatch) {
                 const uint4* rec = it.rec + b0;
-                if (kg == 0 || it.count > D::kBatch) {
+                if (kg == k_lo || it.count > D::kBatch) {
                     // Sort the batch's records by key = (column, first row): counts with each record's
                     // rank, the counts' prefix, then the sorted indices.
                     const int nb = min(D::kBatch, it.count - b0);
@@ -1758,10 +1760,10 @@ k_win_dense(WinJobs jobs) {
                 }
                 if (threadIdx.x == 0) {
                     s_chunk = 0;
-                    if (b0 == 0 && kg == 0) s_item = static_cast<int>(gnext);
+                    if (b0 == 0 && kg == k_lo) s_item = static_cast<int>(gnext);
                 }
                 lds_barrier();
-                if (b0 == 0 && kg == 0) {
+                if (b0 == 0 && kg == k_lo) {
                     gi_next = __builtin_amdgcn_readfirstlane(s_item);
                     if (gi_next < nitems) fetch(gi_next, itn);
                 }
@@ -1854,14 +1856,14 @@ k_win_dense(WinJobs jobs) {
             }
             // The piece's share: [term][row][column] with the checkerboard sign.
             float2* out = J.partial + (static_cast<size_t>(it.slot) * K + kg) * kDenseCells;
-            const int nk = min(8 * MB, K - kg);
+            const int nk = min(8 * MB, k_hi - kg);
             for (int v = threadIdx.x; v < nk * kDenseCells; v += kThreads) {
                 const int k = v / kDenseCells, cell = v - k * kDenseCells;
                 const float sg = ((cell / kDenseCols + cell) & 1) ? -scale.inv : scale.inv;     // (kDenseCols even)
                 out[v] = make_float2(static_cast<float>(tile[2 * k * kDenseTileStride + cell]) * sg,
                                      static_cast<float>(tile[(2 * k + 1) * kDenseTileStride + cell]) * sg);
             }
-            if (kg + 8 * MB < K) lds_barrier();
+            if (kg + 8 * MB < k_hi) lds_barrier();
         }
         if (gi_next >= nitems) break;
         it = itn;
@@ -2172,16 +2174,16 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     const size_t bin_lds = wg.use_lds ? static_cast<size_t>(wg.band_bins) * sizeof(uint32_t) : 0;
     const dim3 bin_grid(blocks, static_cast<unsigned>(bb.bands));
 
-    // counts[0, lbins) | counts[lbins + 2, +8) = totals, [+8, +10) = the coarse bins' pieces | the coarse bins' class counts and the slots
-    // handed out, kSup lbins each | the halves' sizes (fit_shape).
+    // counts[0, lbins) | counts[lbins + 2, +12) = totals | the coarse bins' class counts and the slots handed out, kSup lbins
+    // each | the halves' sizes (fit_shape).
     const size_t nsub = coarse ? kSup * lbins : 0;
-    const size_t ncleared = lbins + 12 + 2 * nsub + kShapeWords;
+    const size_t ncleared = lbins + 14 + 2 * nsub + kShapeWords;
     // (Both forms' sizes where there are two: records that did not fit the planes and then do find room under capture.)
     const size_t sub_rows = (static_cast<size_t>(wg.nh) + kSup - 1) / kSup, sub_lbins = nwt / wg.nw * sub_rows;
     const size_t ncounts_held = nbins > static_cast<size_t>(kLdsBins) ? std::max(nbins, (1 + 2 * kSup) * sub_lbins) : lbins;
     uint32_t* counts = static_cast<uint32_t*>(
-        ctx->ws.get(Workspace::kBinCounts, (ncounts_held + 12 + kShapeWords) * sizeof(uint32_t)));
-    uint32_t* sub_counts = counts + lbins + 12;
+        ctx->ws.get(Workspace::kBinCounts, (ncounts_held + 14 + kShapeWords) * sizeof(uint32_t)));
+    uint32_t* sub_counts = counts + lbins + 14;
     uint32_t* half_sizes = sub_counts + 2 * nsub;
     uint32_t* blockhist = static_cast<uint32_t*>(scratch);
     uint32_t* blocktot = blockhist + bb.nhist;
@@ -2313,9 +2315,10 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
 
 void contract_windows(svdi_context* ctx, const WindowJob* jobs, int count) {
     if (count < 1 || count > kMaxJobs) throw std::logic_error("window job count out of range");
-    // The dense halves of up to eight terms and of more go in launches of their own: blocks of 16 terms have eight wavefronts and
-    // half the batch, and multiply zeros for the upper eight of a job that has no more (eight SKA-Low snapshots, one of
-    // them of 16 terms, as one planned batch: all in one launch 6.9 to 7.2 ms, 6.0 to 6.1 so).
+    // The dense halves' blocks of sixteen terms and of eight go in launches of their own.  Sixteen have eight wavefronts and half
+    // the batch, and multiply zeros for terms that a job does not have, so a job's last terms go with the eights where they are
+    // no more (eight SKA-Low snapshots, one of them of 16 terms, as one planned batch: all in one launch of sixteens 6.9 to
+    // 7.2 ms, 6.0 to 6.1 so; one of 24 terms: contraction by sixteens alone 1207 us, 1068 so).
     WinJobs wj = {}, by_terms[2] = {};
     wj.count = count;
     for (int j = 0; j < count; ++j) {
@@ -2330,8 +2333,15 @@ void contract_windows(svdi_context* ctx, const WindowJob* jobs, int count) {
         std::memcpy(&d.wg, jobs[j].geom, sizeof d.wg);
         d.K = jobs[j].K;
         d.G = jobs[j].G;
-        WinJobs& t = by_terms[d.K <= 8 ? 0 : 1];
-        t.job[t.count++] = d;
+        auto add = [&](WinJobs& t, int k_lo, int k_hi) {
+            if (k_lo >= k_hi) return;
+            WinJob& part = t.job[t.count++] = d;
+            part.k_lo = k_lo;
+            part.k_hi = k_hi;
+        };
+        const int sixteens = d.K % 16 <= 8 ? d.K - d.K % 16 : d.K;
+        add(by_terms[0], sixteens, d.K);
+        add(by_terms[1], 0, sixteens);
     }
     const size_t tok = stage_begin(ctx, 5);
     const unsigned grid = static_cast<unsigned>(std::max(1, ctx->cu_count - ctx->grid_reserve));
