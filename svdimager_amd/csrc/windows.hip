@@ -2130,9 +2130,9 @@ static size_t item_bytes(const WinGeom& wg) {
 static size_t slot_bytes(const GridParams& gp) { return static_cast<size_t>(gp.K) * kDenseCells * sizeof(float2) + sizeof(WItem); }
 
 // The scratch is the buffer of the transformed rows (row_bytes), which is idle until the planes are
-// done.  It holds a slot for every 576 grid cells, and snapshots of the usual arrays make a piece for every 1,300 to
+// done.  It holds a slot for every 576 grid cells, and most snapshots make a piece for every 1,300 to
 // 17,000.  Small grids of many samples make more (1,219 at 512^2, one for every 484), so the buffer is larger
-// by a slot for every 4,608 samples where the worst case asks for it.  (With slots for the worst case, items and
+// by a slot for every 4,608 samples, or as large as usual_pieces says, where the worst case asks for it.  (With slots for the worst case, items and
 // histograms in buffers of their own the context held 1,029 MB after the SKA-Low snapshot and 591 after one of 1.4 M samples at 1000^2; so 609 and 345.)
 WindowScratch window_scratch(const svdi_context* ctx, const SampleInput& in, const GridParams& gp, size_t row_bytes) {
     WindowScratch s = {row_bytes, row_bytes};
@@ -2142,11 +2142,14 @@ WindowScratch window_scratch(const svdi_context* ctx, const SampleInput& in, con
         batch.nslabs = nslabs;
         const WinGeom wg = window_geometry(in, batch);
         const size_t most = most_pieces(wg.shape, max_window_records(in), 2 * static_cast<size_t>(wg.nwin_total));
-        const size_t bound = row_bytes + (in.num_samples / 4608 + 16) * slot_bytes(gp);
+        size_t bound = row_bytes + (in.num_samples / 4608 + 16) * slot_bytes(gp);
+        // (The fixed scratch range leaves no more room than that, neither for the slots nor for the smaller blocks' histograms.)
+        if (!ctx->ws.in_arena())
+            bound = std::max(bound, item_bytes(wg) + slot_bytes(gp) * usual_pieces(wg.shape, in.num_samples,
+                                                                                  2 * static_cast<size_t>(wg.nwin_total)));
         const int largest = in.from_snapshot ? kBinRowsMost : kBinPerThreadMost;
         s.least = std::max({s.least, item_bytes(wg), bin_blocks(in, wg, largest).bytes});
         s.wanted = std::max(s.wanted, std::min(item_bytes(wg) + most * slot_bytes(gp), bound));
-        // (The fixed scratch range leaves the smaller blocks' histograms no more room than there is.)
         if (!ctx->ws.in_arena()) s.wanted = std::max(s.wanted, choose_bin_blocks(ctx, in, wg, kMaxBlockHistBytes / 8).bytes);
     }
     s.wanted = std::max(s.wanted, s.least);

@@ -48,10 +48,19 @@ inline size_t most_pieces(const WorkShape& s, size_t records, size_t halves) {
     return records / s.coop_cap + std::min(halves, records / (static_cast<size_t>(s.coop_min) + 1));
 }
 
+// Slots that snapshots of the usual arrays do with, from few samples on large grids to many on small ones: they make 1.4
+// records a sample, and dense halves of several times coop_min on average (pieces made, and this: 29 and 46 for 32 k samples
+// at 128^2, 951 and 1,536 for 1.4 M at 1000^2, 1,492 and 2,301 for 8.4 M at 1024^2, 915 and 1,056 for 2.1 M at 128^2, which with
+// 518 slots took 388 us, so 353).
+inline size_t usual_pieces(const WorkShape& s, size_t samples, size_t halves) {
+    return samples * 3 / 2 / s.coop_cap + std::min(halves, samples * 3 / 16 / s.coop_min);
+}
+
 // Every piece takes a partial slot.  Where the slots are fewer than most_pieces (the worst case is several times what
 // any snapshot makes: 17,361 for the SKA-Low one, which makes 1,492), the dense halves are counted by size first, and
-// if their pieces do not fit, the shape is made coarser on the device: the pieces longer, until all dense records' take half
-// the slots, then the threshold higher by quarters of an octave, so that the smallest halves are left to wavefront items.
+// if their pieces do not fit, the shape is made coarser on the device: the pieces longer, until all dense records' take what the
+// halves leave, at least half the slots, then the threshold higher by quarters of an octave, so that the smallest halves
+// are left to wavefront items.
 // words: [0] dense halves, [1] their records, [2 + 2 b], [3 + 2 b] those of size bucket b, which holds the halves of
 // more than shape_threshold(coop_min, b) and at most shape_threshold(coop_min, b + 1) records.
 constexpr int kShapeBuckets = 112;                 // 28 octaves: 32 records to 2^31
@@ -70,7 +79,9 @@ SVDI_HD int shape_bucket(uint32_t coop_min, uint32_t records) {     // records >
 }
 SVDI_HD void fit_shape(const uint32_t* words, uint32_t slots, WorkShape& s) {
     if (slots == kAllSlotsFit || words[0] + words[1] / s.coop_cap <= slots) return;
-    while (words[1] / s.coop_cap > slots / 2) s.coop_cap *= 2;          // (at most twice the records, below 2^32)
+    const uint32_t cuts = words[0] < slots / 2 ? slots - words[0] : slots / 2;
+    const uint32_t cap = cuts != 0 ? words[1] / cuts + 1 : 0xffffffffu;
+    if (cap > s.coop_cap) s.coop_cap = cap;
     uint32_t halves = 0, records = 0;
     int b = kShapeBuckets;
     for (; b > 0; --b) {

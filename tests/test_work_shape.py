@@ -130,8 +130,8 @@ def test_the_shape_asked_for_is_the_shape_that_runs(lib):
 @pytest.mark.parametrize("slots", [0, 1, 7, 40, 400, 4000])
 @pytest.mark.parametrize("spread", [2.0, 5.0, 9.0])
 def test_pieces_fit_the_slots(lib, slots, spread):
-    """Where they do not, the least coarser shape of the steps that does: pieces of half the slots, then a higher
-    threshold by quarters of an octave, under which only smaller halves are left out."""
+    """Where they do not, the least coarser shape that does: pieces that take what the halves leave, at least half the
+    slots, then a threshold higher by quarters of an octave, under which only smaller halves are left out."""
     rng = np.random.default_rng([slots, int(spread)])
     for cmin, cap in ((32, 4096), (256, 2048), (1024, 16384)):
         sizes = np.minimum(np.exp(rng.normal(np.log(4.0 * cmin), spread / 2, 3000)), 6e5).astype(np.int64)
@@ -140,8 +140,11 @@ def test_pieces_fit_the_slots(lib, slots, spread):
         if len(dense) + dense.sum() // cap <= slots:
             assert (m, c) == (cmin, cap)
         assert _made(sizes, (m, c)) <= slots
-        assert c >= cap and c % cap == 0 and (c // cap) & (c // cap - 1) == 0
-        assert c == cap or dense.sum() // (c // 2) > slots // 2
+        cuts = max(slots - len(dense), slots // 2)
+        assert c >= cap and (cuts == 0 or dense.sum() // c <= cuts)
+        assert c == cap or cuts == 0 or dense.sum() // (c - 1) >= cuts
+        if len(dense) < slots // 2:
+            assert m == cmin
         if m > cmin:                                       # a quarter of an octave lower would not have fitted
             lower = max(cmin, int(m / 1.26) - 1) if m < 0xffffffff else int(sizes.max()) - 1
             left = sizes[sizes > lower]
