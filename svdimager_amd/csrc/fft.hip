@@ -1242,7 +1242,7 @@ void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size
     // Transforms per workgroup: about kPassElems elements, so that two workgroups and more share a CU and one's
     // loads run beside the other's stages; columns at least four (32-byte row segments) unless the LDS does
     // not hold them; fewer where the workgroups would not fill the chip twice.  The threads: up to 512 with a
-    // butterfly or so each, more only where 512 could not hold a stage.
+    // butterfly or so each, more where 512 could not hold a stage or a CU holds one workgroup.
     const int n = static_cast<int>(G);
     int held[2] = {kHoldLess, kHoldMore};          // elements per thread, the least of the stages
     for (int i = 0; i < st.count; ++i) {
@@ -1272,6 +1272,9 @@ void launch_fft2_inverse(svdi_context* ctx, const float2* planes, size_t P, size
             s.threads *= 2;
             if (s.threads == kPassThreads && elems > s.threads * held[0]) s.more = true;
         }
+        // (With one workgroup to a CU nothing else hides its waits: 8 planes of 5000^2 rows + columns 2.43 ms with 512 threads,
+        // 2.25 so; of 7200^2 2.36 and 2.07.)
+        if (s.threads < kPassThreads && 2 * lds_of(ntrans) > kPassLds) s = {kPassThreads, elems > kPassThreads * held[0]};
         return s;
     };
     auto grid_of = [&](int tiles, int ntrans, int threads) {
