@@ -378,8 +378,14 @@ Enqueued image_prepare(svdi_context* ctx, const SampleInput& in, const svdi_opti
     e.rowfft_bytes = P * fft_row_elems(G, hp.cols) * sizeof(float2);
     if (gridder == SVDI_GRIDDER_MFMA && grid_windows_supported(in, probe)) {
         const WindowScratch w = window_scratch(ctx, in, probe, e.rowfft_bytes);
-        e.rowfft_bytes = w.wanted;
-        if (ctx->ws.frozen()) e.rowfft_bytes = std::max(w.least, std::min(w.wanted, ctx->ws.held(Workspace::kRowFft)));
+        // Where it cannot be had, what there is: the held buffer under capture, the rest of the fixed scratch range.
+        size_t room = w.wanted;
+        if (ctx->ws.frozen()) room = ctx->ws.held(Workspace::kRowFft);
+        if (ctx->ws.in_arena()) {
+            fft_prepare(ctx, G);
+            room = ctx->ws.arena_left();
+        }
+        e.rowfft_bytes = std::max(w.least, std::min(w.wanted, room));
     }
     e.rowfft = static_cast<float2*>(ctx->ws.get(Workspace::kRowFft, e.rowfft_bytes));
     return e;

@@ -148,6 +148,7 @@ class Workspace {
     void set_frozen(bool on) { frozen_ = on; }
     bool frozen() const { return frozen_; }
     bool in_arena() const { return arena_ != nullptr; }
+    size_t arena_left() const { return arena_cap_ - arena_used_; }
     ~Workspace() { release(); }
 
   private:
@@ -264,11 +265,12 @@ const uint32_t* launch_grid_tiled(svdi_context* ctx, const SampleInput& in, cons
 const uint32_t* launch_grid_windows(svdi_context* ctx, const SampleInput& in, const GridParams& gp,
                                     float2* planes, void* scratch, size_t scratch_bytes);
 // Scratch of a call whose slab batches have gp.nslabs slabs each and the last one the rest, in a buffer that also holds
-// row_bytes of something else: the size to allocate, and the least that does.
+// row_bytes of something else: the size to allocate, and the least that does.  (In arena mode the gridder's other buffers
+// are carved here, so that what is left is known.)
 struct WindowScratch {
     size_t least, wanted;
 };
-WindowScratch window_scratch(const svdi_context* ctx, const SampleInput& in, const GridParams& gp, size_t row_bytes);
+WindowScratch window_scratch(svdi_context* ctx, const SampleInput& in, const GridParams& gp, size_t row_bytes);
 // The window gridder in three steps, so that one contraction launch (on the calling context's
 // stream) can take several slab batches, of several snapshots, binned on other streams:
 // bin_windows enqueues the binning of one slab batch, contract_windows the contraction of up to

@@ -2065,6 +2065,30 @@ static WinGeom window_geometry(const SampleInput& in, const GridParams& gp) {
     return wg;
 }
 
+// A slab batch's buffers in the context's workspace, but for the scratch.
+struct WindowBuffers {
+    uint32_t *counts, *boff, *cursor, *sums, *icount, *ioff;
+    uint4* records;
+};
+static size_t item_counts(const WinGeom& wg) { return (3 * kItemClasses + 3) * static_cast<size_t>(wg.nwin_total); }
+static WindowBuffers window_buffers(svdi_context* ctx, const SampleInput& in, const WinGeom& wg, bool use_lds) {
+    const size_t nbins = static_cast<size_t>(wg.nbins), lbins = static_cast<size_t>(wg.lbins), ncounts = item_counts(wg);
+    auto words = [&](Workspace::Slot slot, size_t n) { return static_cast<uint32_t*>(ctx->ws.get(slot, n * sizeof(uint32_t))); };
+    // (Both forms' sizes where there are two: records that did not fit the planes and then do find room under capture.)
+    const size_t sub_lbins = static_cast<size_t>(wg.nwin_total / wg.nw) * ((wg.nh + kSup - 1) / kSup);
+    const size_t held = wg.nbins > kLdsBins ? std::max(nbins, (1 + 2 * kSup) * sub_lbins) : lbins;
+    WindowBuffers b;
+    b.counts = words(Workspace::kBinCounts, held + 14 + kShapeWords);
+    b.boff = words(Workspace::kBinOffsets, nbins + 8);
+    // Cursors (without LDS histograms); segment sums [kBinSegs][lbins]; the coarse bins' offsets.
+    b.cursor = words(Workspace::kBinCursor, lbins + 8 + (use_lds ? kBinSegs * lbins : 0) + (wg.sup_log2 != 0 ? lbins + 8 : 0));
+    b.sums = words(Workspace::kScanSums, scan_blocks(std::max(lbins, ncounts)));
+    b.icount = words(Workspace::kItemCounts, ncounts + 8);
+    b.ioff = words(Workspace::kItemOffsets, ncounts + 8);
+    b.records = static_cast<uint4*>(ctx->ws.get(Workspace::kRecPos, max_window_records(in) * sizeof(uint4)));
+    return b;
+}
+
 // The binning's blocks of a size, and what they keep in memory: per-block record offsets (the counts
 // themselves when 32-bit), the (block, band) record totals, then the 16-bit per-block counts when a block has fewer
 // than 65536 samples (a bin's count per block is at most its sample count).  LDS bands of at most kLdsBins bins, unless
@@ -2115,7 +2139,7 @@ static BinBlocks choose_bin_blocks(const svdi_context* ctx, const SampleInput& i
         const double bins = static_cast<double>(wg.lbins);
         const double ns = rounds * (3.7 * static_cast<double>(size * unit_samples(size)) + 0.3 * std::min(bins, 1.0 * kLdsBins)) +
                           b.blocks * bins * 0.0035;
-        if (size != most && (ns >= best || b.bytes > room)) continue;
+        if (size != most && (ns >= best || !b.use_lds || b.bytes > room)) continue;
         best = ns;
         pick = b;
     }
@@ -2132,25 +2156,25 @@ static size_t slot_bytes(const GridParams& gp) { return static_cast<size_t>(gp.K
 // The scratch is the buffer of the transformed rows (row_bytes), which is idle until the planes are
 // done.  It holds a slot for every 576 grid cells, and most snapshots make a piece for every 1,300 to
 // 17,000.  Small grids of many samples make more (1,219 at 512^2, one for every 484), so the buffer is larger
-// by a slot for every 4,608 samples, or as large as usual_pieces says, where the worst case asks for it.  (With slots for the worst case, items and
-// histograms in buffers of their own the context held 1,029 MB after the SKA-Low snapshot and 591 after one of 1.4 M samples at 1000^2; so 609 and 345.)
-WindowScratch window_scratch(const svdi_context* ctx, const SampleInput& in, const GridParams& gp, size_t row_bytes) {
+// by a slot for every 4,608 samples, or as large as usual_pieces says, where the worst case asks for it.  (With slots for
+// the worst case, items and histograms in buffers of their own the context held 1,029 MB after the SKA-Low snapshot and
+// 591 after one of 1.4 M samples at 1000^2; so 609 and 345.)
+WindowScratch window_scratch(svdi_context* ctx, const SampleInput& in, const GridParams& gp, size_t row_bytes) {
     WindowScratch s = {row_bytes, row_bytes};
     GridParams batch = gp;
     for (int nslabs : {gp.nslabs, gp.total_slabs % gp.nslabs}) {           // whole slab batches and the last one
         if (nslabs == 0) continue;
         batch.nslabs = nslabs;
         const WinGeom wg = window_geometry(in, batch);
-        const size_t most = most_pieces(wg.shape, max_window_records(in), 2 * static_cast<size_t>(wg.nwin_total));
-        size_t bound = row_bytes + (in.num_samples / 4608 + 16) * slot_bytes(gp);
-        // (The fixed scratch range leaves no more room than that, neither for the slots nor for the smaller blocks' histograms.)
-        if (!ctx->ws.in_arena())
-            bound = std::max(bound, item_bytes(wg) + slot_bytes(gp) * usual_pieces(wg.shape, in.num_samples,
-                                                                                  2 * static_cast<size_t>(wg.nwin_total)));
-        const int largest = in.from_snapshot ? kBinRowsMost : kBinPerThreadMost;
-        s.least = std::max({s.least, item_bytes(wg), bin_blocks(in, wg, largest).bytes});
-        s.wanted = std::max(s.wanted, std::min(item_bytes(wg) + most * slot_bytes(gp), bound));
-        if (!ctx->ws.in_arena()) s.wanted = std::max(s.wanted, choose_bin_blocks(ctx, in, wg, kMaxBlockHistBytes / 8).bytes);
+        const size_t halves = 2 * static_cast<size_t>(wg.nwin_total), allowance = in.num_samples / 4608 + 16;
+        const size_t slots = std::min(most_pieces(wg.shape, max_window_records(in), halves),
+                                      std::max((row_bytes - std::min(row_bytes, item_bytes(wg))) / slot_bytes(gp) + allowance,
+                                               usual_pieces(wg.shape, in.num_samples, halves)));
+        const BinBlocks largest = bin_blocks(in, wg, in.from_snapshot ? kBinRowsMost : kBinPerThreadMost);
+        s.least = std::max({s.least, item_bytes(wg), largest.bytes});
+        s.wanted = std::max({s.wanted, item_bytes(wg) + slots * slot_bytes(gp),
+                             choose_bin_blocks(ctx, in, wg, kMaxBlockHistBytes / 8).bytes});
+        if (ctx->ws.in_arena()) (void)window_buffers(ctx, in, wg, largest.use_lds);
     }
     s.wanted = std::max(s.wanted, s.least);
     return s;
@@ -2181,30 +2205,19 @@ WindowJob bin_windows(svdi_context* ctx, const SampleInput& in, const GridParams
     // each | the halves' sizes (fit_shape).
     const size_t nsub = coarse ? kSup * lbins : 0;
     const size_t ncleared = lbins + 14 + 2 * nsub + kShapeWords;
-    // (Both forms' sizes where there are two: records that did not fit the planes and then do find room under capture.)
-    const size_t sub_rows = (static_cast<size_t>(wg.nh) + kSup - 1) / kSup, sub_lbins = nwt / wg.nw * sub_rows;
-    const size_t ncounts_held = nbins > static_cast<size_t>(kLdsBins) ? std::max(nbins, (1 + 2 * kSup) * sub_lbins) : lbins;
-    uint32_t* counts = static_cast<uint32_t*>(
-        ctx->ws.get(Workspace::kBinCounts, (ncounts_held + 14 + kShapeWords) * sizeof(uint32_t)));
+    const WindowBuffers buf = window_buffers(ctx, in, wg, bb.use_lds);
+    uint32_t *const counts = buf.counts, *const boff = buf.boff, *const cursor = buf.cursor, *const sums = buf.sums;
+    uint32_t *const icount = buf.icount, *const ioff = buf.ioff;
     uint32_t* sub_counts = counts + lbins + 14;
     uint32_t* half_sizes = sub_counts + 2 * nsub;
     uint32_t* blockhist = static_cast<uint32_t*>(scratch);
     uint32_t* blocktot = blockhist + bb.nhist;
     uint16_t* blockcount16 = count16 ? reinterpret_cast<uint16_t*>(blocktot + bb.blocks * bb.bands) : nullptr;
-    uint32_t* boff = static_cast<uint32_t*>(ctx->ws.get(Workspace::kBinOffsets, (nbins + 8) * sizeof(uint32_t)));
-    // Cursors (without LDS histograms); segment sums [kBinSegs][lbins]; the coarse bins' offsets.
-    uint32_t* cursor = static_cast<uint32_t*>(ctx->ws.get(
-        Workspace::kBinCursor, (lbins + 8 + (wg.use_lds ? kBinSegs * lbins : 0) + (coarse ? lbins + 8 : 0)) * sizeof(uint32_t)));
     uint32_t* segsum = cursor + lbins + 8;
     uint32_t* coff = coarse ? segsum + (wg.use_lds ? kBinSegs * lbins : 0) : boff;
-    const size_t ncounts = (3 * kItemClasses + 3) * nwt;
-    uint32_t* sums = static_cast<uint32_t*>(
-        ctx->ws.get(Workspace::kScanSums, scan_blocks(std::max(lbins, ncounts)) * sizeof(uint32_t)));
-    uint32_t* icount = static_cast<uint32_t*>(ctx->ws.get(Workspace::kItemCounts, (ncounts + 8) * sizeof(uint32_t)));
-    uint32_t* ioff = static_cast<uint32_t*>(ctx->ws.get(Workspace::kItemOffsets, (ncounts + 8) * sizeof(uint32_t)));
+    const size_t ncounts = item_counts(wg);
     uint32_t* totals = counts + lbins + 2;
-    WRecords rec;
-    rec.r = static_cast<uint4*>(ctx->ws.get(Workspace::kRecPos, max_records * sizeof(uint4)));
+    const WRecords rec = {buf.records};
 
     // Wavefront items: one per window at most.  Pieces, and partial slots: as many as any sizes of the halves could
     // need, or as many as the scratch holds: then fit_shape sees to it that they suffice.
