@@ -2098,6 +2098,10 @@ struct BinBlocks {
     size_t blocks = 0, bands = 1, nhist = 1, bytes = 0;
     bool use_lds = false, count16 = false;
 };
+static int most_block_size(const SampleInput& in) { return in.from_snapshot ? kBinRowsMost : kBinPerThreadMost; }
+static int least_block_size(const SampleInput& in, const WinGeom& wg) {
+    return !in.from_snapshot ? 1 : in.quad_rows ? kBinRowsLeast : wg.set_rows;
+}
 static BinBlocks bin_blocks(const SampleInput& in, const WinGeom& wg, int size) {
     BinBlocks b;
     b.size = size;
@@ -2128,8 +2132,7 @@ static BinBlocks choose_bin_blocks(const svdi_context* ctx, const SampleInput& i
         const size_t groups = kBinThreads / static_cast<size_t>(in.quad_rows ? size / 4 : wg.set_rows);
         return (in.num_channels + groups - 1) / groups * groups;
     };
-    const int most = in.from_snapshot ? kBinRowsMost : kBinPerThreadMost;
-    const int least = !in.from_snapshot ? 1 : in.quad_rows ? kBinRowsLeast : wg.set_rows;
+    const int most = most_block_size(in), least = least_block_size(in, wg);
     const int step = in.from_snapshot && in.quad_rows ? 16 : least;
     BinBlocks pick;
     double best = 0.0;
@@ -2170,13 +2173,14 @@ WindowScratch window_scratch(svdi_context* ctx, const SampleInput& in, const Gri
         const size_t slots = std::min(most_pieces(wg.shape, max_window_records(in), halves),
                                       std::max((row_bytes - std::min(row_bytes, item_bytes(wg))) / slot_bytes(gp) + allowance,
                                                usual_pieces(wg.shape, in.num_samples, halves)));
-        const BinBlocks largest = bin_blocks(in, wg, in.from_snapshot ? kBinRowsMost : kBinPerThreadMost);
+        const BinBlocks largest = bin_blocks(in, wg, most_block_size(in));
         s.least = std::max({s.least, item_bytes(wg), largest.bytes});
-        s.wanted = std::max({s.wanted, item_bytes(wg) + slots * slot_bytes(gp),
-                             choose_bin_blocks(ctx, in, wg, kMaxBlockHistBytes / 8).bytes});
+        s.wanted = std::max({s.wanted, s.least, item_bytes(wg) + slots * slot_bytes(gp)});
+        // (The choice is made only where it can matter: it is host time of every call.)
+        if (bin_blocks(in, wg, least_block_size(in, wg)).bytes > s.wanted)
+            s.wanted = std::max(s.wanted, choose_bin_blocks(ctx, in, wg, kMaxBlockHistBytes / 8).bytes);
         if (ctx->ws.in_arena()) (void)window_buffers(ctx, in, wg, largest.use_lds);
     }
-    s.wanted = std::max(s.wanted, s.least);
     return s;
 }
 
