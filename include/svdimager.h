@@ -187,7 +187,7 @@ int svdi_image_snapshot(svdi_context* ctx, const svdi_snapshot* snapshot, float*
  * forbid hipMalloc).  The call's scratch (rotation, plan, binning records, planes, FFT buffers)
  * is carved from a fixed device array of SVDI_NOALLOC_SCRATCH_BYTES that the library holds on
  * every GPU it runs on until the process ends; a snapshot or image that needs more returns
- * SVDI_ERR_INVALID_ARGUMENT with the sizes in svdi_last_error() (about 2 M samples at 512^2
+ * SVDI_ERR_INVALID_ARGUMENT with the sizes in svdi_last_error() (about 5 M samples at 512^2
  * fit).  Slabs are imaged one at a time unless opts->max_batch_slabs says otherwise.  Every
  * context on a GPU shares that GPU's array: calls that overlap in time on one GPU (from two
  * contexts or threads) race and must be serialised by the caller.  The call returns when the

@@ -1344,9 +1344,9 @@ __device__ __forceinline__ int job_of(const int* off, int count, int g) {
 // because its LDS atomics are: ds_add_f32 handles one lane in three cycles on this chip (193 cycles
 // per wavefront, measured), ds_add_f64 a wavefront in 9.
 //
-// Measured (SKA-Low snapshot, 8.4 M samples at 1024^2, 62% of the records in dense halves): 250 us, and
-// 143 us for the wavefront items that remain, against 476 us for window contraction of everything;
-// eight such snapshots in a batch 5.43 against 6.11 ms.  It issues a quarter of the MFMAs and 0.4 of
+// Measured (SKA-Low snapshot, 8.4 M samples at 1024^2, 62% of the records in dense halves): 240 us, and
+// 139 us for the wavefront items that remain, against 476 us for window contraction of everything;
+// eight such snapshots in a batch 5.35 against 6.11 ms.  It issues a quarter of the MFMAs and 0.4 of
 // the VALU instructions of the window form (3.5 M and 71 M).  About 110 us of it are the sort, the
 // tile's clearing and write-out and the barriers around them, the rest the chunks, which wait for
 // their LDS operands as long as they compute (a chunk's chain is about 5000 cycles with three
